@@ -23,10 +23,12 @@ SOURCES = [
     "rkx_host.cpp",
     "rkx_batch.cpp",
     "rkx_methods.cpp",
+    "rkx_kernels_step.hip",
     "rkx_kernels_d.hip",
     "rkx_kernels_gather.hip",
     "rkx_kernels_lvpairs.hip",
     "rkx_kernels_sweep.hip",
+    "rkx_kernels_sweep_verner65.hip",
     "rkx_kernels_sweep_dopri87.hip",
     "rkx_kernels_lv.hip",
     "rkx_kernels_chain.hip",

@@ -23,7 +23,7 @@ namespace rkx {
 namespace {
 
 constexpr int kBatchCap = 1024;       // instances per batch
-constexpr int kPollSteps = 16;        // batched steps between state polls
+constexpr int kPollSteps = 16;        // batched steps between state polls (a multiple of kRing)
 
 struct batch_inst {
   bool used = false;
@@ -36,6 +36,7 @@ struct batch_inst {
   rkx_method m{};
   dev_ode dp{};
   dev_method dm{};
+  step_refs ref{};                      // fused kernels: state, ring and table of its slot
   sweep_cfg base{1, 1};                 // tile shape chosen at admission
   sweep_cfg cfg{1, 1};                  // current shape (bands shortened as the batch drains)
   double *y[2] = {nullptr, nullptr};
@@ -61,6 +62,7 @@ struct rkx_batch {
   hipStream_t stream = nullptr;
   rkx_batch_opts opts{};
   state *st_dev = nullptr;
+  step_ring *rg_dev = nullptr;
   dev_coef *cf_dev = nullptr;
   dev_method *dm_dev = nullptr;
   sweep_inst *si_dev = nullptr;
@@ -135,7 +137,7 @@ int adapt_bands(rkx_batch *b)
       if (!I.used || I.done || I.storage != RKX_STORAGE_LOW || I.K <= 0)
         continue;
       const sweep_cfg c{I.base.waves, rows_at(I, div)};
-      const sweep_inst si = make_sweep_inst(I.dp, I.m, c, nullptr, nullptr, nullptr);
+      const sweep_inst si = make_sweep_inst(I.dp, I.m, c, {}, nullptr, nullptr);
       const int band = sweep_band_rows(I.pattern, I.m.s, std::min(si.R, I.dp.N));
       const double iters = band + 2.0 * (I.m.s - 1);
       auto &e = g[{I.pattern, I.K}];
@@ -167,7 +169,7 @@ int adapt_bands(rkx_batch *b)
     if (c.rows == I.cfg.rows)
       continue;
     I.cfg = c;
-    const sweep_inst si = make_sweep_inst(I.dp, I.m, c, b->st_dev + i, I.y[0], I.y[1]);
+    const sweep_inst si = make_sweep_inst(I.dp, I.m, c, I.ref, I.y[0], I.y[1]);
     RKX_HIP(hipMemcpyAsync(b->si_dev + i, &si, sizeof(si), hipMemcpyHostToDevice, b->stream));
   }
   return RKX_OK;
@@ -177,7 +179,7 @@ int adapt_bands(rkx_batch *b)
 // last band, plus the 2(s-1) halo rows).
 int tile_iters(const batch_inst &I, int t)
 {
-  const sweep_inst si = make_sweep_inst(I.dp, I.m, I.cfg, nullptr, nullptr, nullptr);
+  const sweep_inst si = make_sweep_inst(I.dp, I.m, I.cfg, {}, nullptr, nullptr);
   return sweep_tile_iters(I.pattern, I.m.s, si, t);
 }
 
@@ -218,9 +220,9 @@ int rebuild_tables(rkx_batch *b)
     g.K = I.K;
     int nt = 0;
     if (I.K == 0) {
-      nt = make_chain_inst(I.dp, I.m, nullptr, nullptr, nullptr).nwg;
+      nt = make_chain_inst(I.dp, I.m, {}, nullptr, nullptr).nwg;
     } else {
-      const sweep_inst si = make_sweep_inst(I.dp, I.m, I.cfg, nullptr, nullptr, nullptr);
+      const sweep_inst si = make_sweep_inst(I.dp, I.m, I.cfg, {}, nullptr, nullptr);
       nt = si.ntiles;
       if (!sweep_inst_single_reflect(I.pattern, I.m.s, si))
         g.gen = true;
@@ -252,26 +254,26 @@ int rebuild_tables(rkx_batch *b)
   return RKX_OK;
 }
 
-int enqueue_batched_step(rkx_batch *b)
+// One attempted step of every active instance; r: the ring slot the fused
+// kernels read.
+int enqueue_batched_step(rkx_batch *b, int r)
 {
   for (auto &kv : b->groups) {
     const tile_group &g = kv.second;
-    if (g.tiles.empty())
+    const int nt = static_cast<int>(g.tiles.size());
+    if (nt == 0)
       continue;
     if (g.K == 0)
-      RKX_HIP(launch_chain(g.pattern, b->ci_dev, g.dev, static_cast<int>(g.tiles.size()),
-                           b->stream));
+      RKX_HIP(launch_chain(g.pattern, {{}, b->ci_dev, g.dev, nt, r}, b->stream));
     else
-      RKX_HIP(launch_sweep(g.pattern, g.K, g.gen, b->si_dev, g.dev,
-                           static_cast<int>(g.tiles.size()), b->stream));
+      RKX_HIP(launch_sweep(g.pattern, g.K, g.gen, {{}, b->si_dev, g.dev, nt, r}, b->stream));
   }
   for (int i = 0; i < b->hi_slot; ++i) {
     batch_inst &I = b->inst[static_cast<size_t>(i)];
     if (!I.used || I.done)
       continue;
     if (I.storage == RKX_STORAGE_LOW && I.K < 0)
-      RKX_HIP(launch_lv_step(I.dp, b->cf_dev + i, I.m.s, b->st_dev + i, I.y[0], I.y[1],
-                             b->stream));
+      RKX_HIP(launch_lv_step(I.dp, I.m.s, I.ref, I.y[0], I.y[1], r, b->stream));
     else if (I.storage == RKX_STORAGE_FULL)
       RKX_HIP(launch_d_step(I.dp, b->cf_dev + i, I.m.s, b->st_dev + i, I.y[0], I.y[1], I.w,
                             I.dy, I.err, b->stream));
@@ -298,7 +300,7 @@ int capture_chunk(rkx_batch *b)
   RKX_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
   int rc = RKX_OK;
   for (int j = 0; j < kPollSteps && rc == RKX_OK; ++j)
-    rc = enqueue_batched_step(b);
+    rc = enqueue_batched_step(b, j & (kRing - 1));
   hipGraph_t g = nullptr;
   const hipError_t e = hipStreamEndCapture(b->stream, &g);
   if (rc != RKX_OK) {
@@ -314,8 +316,10 @@ int capture_chunk(rkx_batch *b)
 }
 
 // Enqueue k batched steps and a snapshot of every instance's state into
-// snapshot buffer `slot`; full chunks replay the captured graph.
-int launch_chunk(rkx_batch *b, int slot, int k)
+// snapshot buffer `slot`; full chunks replay the captured graph.  last: the
+// run's last chunk, after which the attempts just made get their control, so
+// the snapshot counts them and the next run starts at ring slot 0 again.
+int launch_chunk(rkx_batch *b, int slot, int k, bool last)
 {
   if (b->dirty) {
     if (int rc = rebuild_tables(b))
@@ -329,9 +333,11 @@ int launch_chunk(rkx_batch *b, int slot, int k)
     RKX_HIP(hipGraphLaunch(b->graph_exec, b->stream));
   } else {
     for (int j = 0; j < k; ++j)
-      if (int rc = enqueue_batched_step(b))
+      if (int rc = enqueue_batched_step(b, j & (kRing - 1)))
         return rc;
   }
+  if (last)
+    RKX_HIP(launch_step_flush(b->st_dev, b->hi_slot, k & (kRing - 1), b->stream));
   RKX_HIP(hipMemcpyAsync(b->st_pinned + static_cast<size_t>(slot) * kBatchCap, b->st_dev,
                          sizeof(state) * b->hi_slot, hipMemcpyDeviceToHost, b->stream));
   RKX_HIP(hipEventRecord(b->ev[slot], b->stream));
@@ -350,7 +356,7 @@ int read_snapshot(rkx_batch *b, int slot, int *newly_done)
       continue;
     const state &s = snap[i];
     I.snap = s;
-    if (s.done && !I.done) {
+    if (s.v.done && !I.done) {
       I.done = true;
       ++*newly_done;
     }
@@ -396,6 +402,7 @@ int rkx_batch_create(rkx_batch **out, const rkx_batch_opts *o)
     }
   };
   dalloc(reinterpret_cast<void **>(&b->st_dev), sizeof(state) * kBatchCap);
+  dalloc(reinterpret_cast<void **>(&b->rg_dev), sizeof(step_ring) * kBatchCap);
   dalloc(reinterpret_cast<void **>(&b->cf_dev), sizeof(dev_coef) * kBatchCap);
   dalloc(reinterpret_cast<void **>(&b->dm_dev), sizeof(dev_method) * kBatchCap);
   dalloc(reinterpret_cast<void **>(&b->si_dev), sizeof(sweep_inst) * kBatchCap);
@@ -413,6 +420,12 @@ int rkx_batch_create(rkx_batch **out, const rkx_batch_opts *o)
   if (rc) {
     rkx_batch_destroy(b);
     return rc;
+  }
+  // slots without a fused instance have no ring (launch_step_flush skips them)
+  if (hipMemset(b->st_dev, 0, sizeof(state) * kBatchCap) != hipSuccess) {
+    (void) hipGetLastError();
+    rkx_batch_destroy(b);
+    return fail(RKX_EDEVICE, "rkx_batch_create: clearing the states failed");
   }
   b->inst.resize(kBatchCap);
   int dev = 0, cus = 0;
@@ -438,8 +451,8 @@ int rkx_batch_destroy(rkx_batch *b)
   for (auto &kv : b->groups)
     if (kv.second.dev)
       (void) hipFree(kv.second.dev);
-  for (void *p : {static_cast<void *>(b->st_dev), static_cast<void *>(b->cf_dev),
-                  static_cast<void *>(b->dm_dev), static_cast<void *>(b->si_dev),
+  for (void *p : {static_cast<void *>(b->st_dev), static_cast<void *>(b->rg_dev),
+                  static_cast<void *>(b->cf_dev), static_cast<void *>(b->dm_dev), static_cast<void *>(b->si_dev),
                   static_cast<void *>(b->ci_dev)})
     if (p)
       (void) hipFree(p);
@@ -531,21 +544,27 @@ int rkx_batch_add(rkx_batch *b, const rkx_ode *p, const rkx_method *m, double t0
   I.bytes = need;
 
   state hs{};
-  hs.t = t0;
-  hs.te = te;
-  hs.tol = tol;
-  hs.h = initial_h(te - t0, tol, step_limit, h0);
-  hs.step_limit = step_limit;
-  hs.ord = m->ord;
+  hs.v.t = t0;
+  hs.v.te = te;
+  hs.v.tol = tol;
+  hs.v.h = initial_h(te - t0, tol, step_limit, h0);
+  hs.v.step_limit = step_limit;
+  hs.v.ord = m->ord;
+  hs.v.done = !(t0 < te);
   hs.ctrl = b->opts.ctrl;
   hs.s = m->s;
   hs.meth = b->dm_dev + slot;
   hs.coef = b->cf_dev + slot;
-  hs.done = !(t0 < te);
+  step_ring hr{};
+  if (storage == RKX_STORAGE_LOW) {
+    hs.ring = b->rg_dev + slot;
+    hr = make_ring(hs.v);
+    I.ref = step_refs{b->st_dev + slot, hs.ring, hs.meth};
+  }
   dev_coef hc{};
-  premult(I.dm, m->s, hs.h, hc);
+  premult(I.dm, m->s, hs.v.h, hc);
   I.snap = hs;
-  I.done = hs.done;
+  I.done = hs.v.done;
   if (storage == RKX_STORAGE_LOW && pairs) {
     I.pattern = 0;
     I.K = -1;
@@ -553,7 +572,7 @@ int rkx_batch_add(rkx_batch *b, const rkx_ode *p, const rkx_method *m, double t0
     I.pattern = sweep_pattern(*m);
     I.K = 0;
     const chain_inst ci =
-        make_chain_inst(dp, *m, b->st_dev + slot, I.y[0], I.y[1]);
+        make_chain_inst(dp, *m, I.ref, I.y[0], I.y[1]);
     RKX_HIP(hipMemcpyAsync(b->ci_dev + slot, &ci, sizeof(ci), hipMemcpyHostToDevice, b->stream));
   } else if (storage == RKX_STORAGE_LOW) {
     I.pattern = sweep_pattern(*m);
@@ -561,12 +580,13 @@ int rkx_batch_add(rkx_batch *b, const rkx_ode *p, const rkx_method *m, double t0
     I.base = I.cfg;
     I.K = I.cfg.waves;
     const sweep_inst si =
-        make_sweep_inst(dp, *m, I.cfg, b->st_dev + slot, I.y[0], I.y[1]);
+        make_sweep_inst(dp, *m, I.cfg, I.ref, I.y[0], I.y[1]);
     RKX_HIP(hipMemcpyAsync(b->si_dev + slot, &si, sizeof(si), hipMemcpyHostToDevice, b->stream));
   }
   RKX_HIP(hipMemcpyAsync(b->dm_dev + slot, &I.dm, sizeof(I.dm), hipMemcpyHostToDevice, b->stream));
   RKX_HIP(hipMemcpyAsync(b->cf_dev + slot, &hc, sizeof(hc), hipMemcpyHostToDevice, b->stream));
   RKX_HIP(hipMemcpyAsync(b->st_dev + slot, &hs, sizeof(hs), hipMemcpyHostToDevice, b->stream));
+  RKX_HIP(hipMemcpyAsync(b->rg_dev + slot, &hr, sizeof(hr), hipMemcpyHostToDevice, b->stream));
   RKX_HIP(hipMemcpyAsync(I.y[0], y0, vec, hipMemcpyHostToDevice, b->stream));
   RKX_HIP(hipStreamSynchronize(b->stream));
   b->bytes += need;
@@ -596,7 +616,7 @@ int rkx_batch_run(rkx_batch *b, int max_steps, int *active)
   int cur = 0;
   if (max_steps > 0 && count_active() > 0) {
     const int k = std::min(kPollSteps, max_steps);
-    if (int rc = launch_chunk(b, cur, k))
+    if (int rc = launch_chunk(b, cur, k, k >= max_steps))
       return rc;
     enqueued += k;
     pending[cur] = true;
@@ -605,7 +625,7 @@ int rkx_batch_run(rkx_batch *b, int max_steps, int *active)
     const int nxt = cur ^ 1;
     if (enqueued < max_steps && count_active() > 0) {
       const int k = std::min(kPollSteps, max_steps - enqueued);
-      if (int rc = launch_chunk(b, nxt, k))
+      if (int rc = launch_chunk(b, nxt, k, enqueued + k >= max_steps))
         return rc;
       enqueued += k;
       pending[nxt] = true;
@@ -631,10 +651,10 @@ int rkx_batch_status(rkx_batch *b, int id, rkx_stats *st, int *done)
   const batch_inst &I = b->inst[static_cast<size_t>(id)];
   if (st) {
     std::memset(st, 0, sizeof(*st));
-    st->steps_acc = I.snap.acc;
-    st->steps_rej = I.snap.rej;
-    st->t = I.snap.t;
-    st->h = I.snap.h;
+    st->steps_acc = I.snap.v.acc;
+    st->steps_rej = I.snap.v.rej;
+    st->t = I.snap.v.t;
+    st->h = I.snap.v.h;
     st->resident_bytes = I.bytes;
   }
   if (done)
@@ -650,7 +670,7 @@ int rkx_batch_result(rkx_batch *b, int id, double *y)
   RKX_HIP(hipStreamSynchronize(b->stream));
   state s;
   RKX_HIP(hipMemcpy(&s, b->st_dev + id, sizeof(state), hipMemcpyDeviceToHost));
-  RKX_HIP(hipMemcpy(y, I.y[s.cur], static_cast<size_t>(I.ode.n) * sizeof(double),
+  RKX_HIP(hipMemcpy(y, I.y[s.v.cur], static_cast<size_t>(I.ode.n) * sizeof(double),
                     hipMemcpyDeviceToHost));
   return RKX_OK;
 }
@@ -678,7 +698,7 @@ int rkx_batch_tile(rkx_batch *b, int id, int *waves, int *rows)
   *rows = 0;
   if (I.storage == RKX_STORAGE_LOW && I.K > 0) {
     *waves = I.cfg.waves;
-    *rows = make_sweep_inst(I.dp, I.m, I.cfg, nullptr, nullptr, nullptr).R;
+    *rows = make_sweep_inst(I.dp, I.m, I.cfg, {}, nullptr, nullptr).R;
   }
   return RKX_OK;
 }

@@ -27,26 +27,6 @@ using gmut = __attribute__((address_space(1))) double;
 __device__ __forceinline__ gconst *as_global(const double *p) { return (gconst *) p; }
 __device__ __forceinline__ gmut *as_global(double *p) { return (gmut *) p; }
 
-// What a step kernel reads of its state at its start.  Read through the
-// global address space, before any store of the kernel, the loads are
-// scalar (through the generic pointer they were vector loads), cur and done
-// in one.  No workgroup of a state reads it after that state's control has
-// run: the control runs in the last of the state's workgroups to finish,
-// after all of them have started.
-struct step_view {
-  int done, cur;
-  double h;
-  const dev_method *meth;
-};
-__device__ __forceinline__ step_view read_step(const state *st)
-{
-  static_assert(offsetof(state, done) == offsetof(state, cur) + 4, "cur, done adjacent");
-  using gstate = const __attribute__((address_space(1))) state;
-  using gu64 = const __attribute__((address_space(1))) unsigned long long;
-  gstate *g = (gstate *) st;
-  const unsigned long long cd = *(gu64 *) &g->cur;     // cur, done in one load
-  return step_view{static_cast<int>(cd >> 32), static_cast<int>(cd & 0xffffffffu), g->h, g->meth};
-}
 using gmethod = const __attribute__((address_space(1))) dev_method;
 __device__ __forceinline__ gmethod *as_global(const dev_method *m) { return (gmethod *) m; }
 
@@ -188,10 +168,6 @@ __device__ __forceinline__ void err_term(double e, double yn, double yo, double 
 
 // ---- step control (include/tools.h:217-278, 191-198) ------------------------
 
-// Runs in exactly one thread after every workgroup has folded its maximum into
-// st->err_bits / st->zero_div.  Resets the accumulators for the next step.
-// The new h uses libm_pow, the C library's pow restated bitwise, so the
-// device reproduces the reference's step sizes without a host round trip.
 // Every workgroup thread t of nt computes its share of the premultiplied
 // coefficients of the next step from the raw table: the same products h*A,
 // h*b, h*(b - b_hat) as premult, each written to both places it is read from.
@@ -221,9 +197,20 @@ __device__ inline void premult_block(const dev_method &m, int s, double h, dev_c
   }
 }
 
-// Runs in exactly one thread after every workgroup has folded its maximum into
-// st->err_bits / st->zero_div.  Resets the accumulators for the next step.
-// The new h uses libm_pow, the C library's pow restated bitwise, so the
+// The trace of an attempt made from v (one thread).
+__device__ inline void trace_attempt(state *st, const step_vars &v, double err)
+{
+  const int attempt = v.acc + v.rej;
+  if (st->trace && attempt < st->trace_cap) {
+    st->trace[3 * attempt + 0] = v.t;
+    st->trace[3 * attempt + 1] = v.h;
+    st->trace[3 * attempt + 2] = err;
+  }
+}
+
+// Full-storage forms: runs in exactly one thread after every workgroup has
+// folded its maximum into st->err_bits / st->zero_div.  Resets the
+// accumulators for the next step.  The new h uses libm_pow, the C library's pow restated bitwise, so the
 // device reproduces the reference's step sizes without a host round trip.
 // Returns whether the next step's coefficients need premultiplying (device
 // control), which the caller's workgroup does with premult_block.
@@ -238,44 +225,230 @@ __device__ inline bool dev_control(state *st)
   st->err = zero ? fmax(1.7E308, q) : q;
   if (st->ctrl == RKX_CTRL_HOST)
     return false;
-  const int attempt = st->acc + st->rej;
-  if (st->trace && attempt < st->trace_cap) {
-    st->trace[3 * attempt + 0] = st->t;
-    st->trace[3 * attempt + 1] = st->h;
-    st->trace[3 * attempt + 2] = st->err;
-  }
-  const bool need = ctrl_decide(*st);
-  const double p = need ? libm_pow(st->pow_x, st->pow_y, dev_pow_tables) : 0.0;
-  ctrl_finish(*st, need, p);
+  trace_attempt(st, st->v, st->err);
+  double px = 0.0, py = 0.0;
+  const bool need = ctrl_decide(st->v, st->err, px, py);
+  ctrl_finish(st->v, need, need ? libm_pow(px, py, dev_pow_tables) : 0.0);
   return true;
 }
 
 // ---- reductions -----------------------------------------------------------------
-__device__ __forceinline__ double wave_max(double v)
+// A lane's double moved by a DPP control (lanes without a source keep v).
+template <int CTRL>
+__device__ __forceinline__ double dpp_keep(double v)
 {
-  for (int off = 32; off > 0; off >>= 1)
-    v = fmax(v, __shfl_xor(v, off, 64));
+  const long long b = __double_as_longlong(v);
+  const int lo = static_cast<int>(b), hi = static_cast<int>(b >> 32);
+  const int ml = __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, false);
+  const int mh = __builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, false);
+  return __longlong_as_double((static_cast<long long>(mh) << 32) | static_cast<unsigned int>(ml));
+}
+// Maximum over the wavefront, valid in lane 63: shifts within rows of 16
+// lanes, then each row's last lane broadcast to the next row(s).  All in
+// registers; six exchanges through LDS (shuffles) took 0.3 us at the end of
+// every step.
+__device__ __forceinline__ double wave_max63(double v)
+{
+  v = fmax(v, dpp_keep<0x111>(v));   // row_shr:1
+  v = fmax(v, dpp_keep<0x112>(v));   // row_shr:2
+  v = fmax(v, dpp_keep<0x114>(v));   // row_shr:4
+  v = fmax(v, dpp_keep<0x118>(v));   // row_shr:8
+  v = fmax(v, dpp_keep<0x142>(v));   // row_bcast:15
+  v = fmax(v, dpp_keep<0x143>(v));   // row_bcast:31
   return v;
 }
 
-// Folds each thread's (qmax, zero) into the step accumulators and runs the
-// control in the last of the `nblocks` workgroups that work on this state to
-// finish (nblocks = 0: the whole grid).  Must be called by all threads of the
-// block.  red must hold blockDim.x/64 doubles of LDS.  coef = false: the
-// kernels of this state form h * dev_method::col themselves, so the control
-// writes no premultiplied coefficients.
-__device__ inline void block_finish(state *st, double qmax, unsigned int zero, double *red,
-                                    unsigned int *zred, unsigned int nblocks = 0u,
-                                    bool coef = true)
+// ---- step control of the fused kernels --------------------------------------
+// The tables of libm_pow spread over a wavefront: lane l holds entries l and
+// l + 64, loaded once at the start of a kernel beside its other first loads,
+// so the two lookups are lane reads instead of two dependent trips to memory.
+// For arguments that are the same in every lane.
+struct lane_pow_tables {
+  double lg[2][3];
+  unsigned long long ex[2][2];
+  __device__ void load()
+  {
+    const int lane = threadIdx.x & 63;
+    for (int q = 0; q < 2; ++q) {
+      for (int c = 0; c < 3; ++c)
+        lg[q][c] = dev_pow_tables.logt[lane + 64 * q][c];
+      for (int c = 0; c < 2; ++c)
+        ex[q][c] = dev_pow_tables.expt[2 * (lane + 64 * q) + c];
+    }
+  }
+  static __device__ unsigned long long lane_of(unsigned long long b, int src)
+  {
+    const unsigned int lo = __builtin_amdgcn_readlane(static_cast<unsigned int>(b), src);
+    const unsigned int hi = __builtin_amdgcn_readlane(static_cast<unsigned int>(b >> 32), src);
+    return (static_cast<unsigned long long>(hi) << 32) | lo;
+  }
+  __device__ double log_at(int i, int c) const
+  {
+    const int u = __builtin_amdgcn_readfirstlane(i);
+    const unsigned long long b =
+        __builtin_bit_cast(unsigned long long, u >= 64 ? lg[1][c] : lg[0][c]);
+    return __builtin_bit_cast(double, lane_of(b, u & 63));
+  }
+  __device__ unsigned long long exp_at(int k, int c) const
+  {
+    const int u = __builtin_amdgcn_readfirstlane(k);
+    return lane_of(u >= 64 ? ex[1][c] : ex[0][c], u & 63);
+  }
+};
+
+// The (instance, tile within it) a workgroup works on: entry `tile` of the
+// launch's table, or tile `tile` of its one instance.
+template <class INST>
+__device__ __forceinline__ int2 launch_tile(const fused_launch<INST> &a, int tile)
 {
-  if (nblocks == 0u)
-    nblocks = gridDim.x * gridDim.y * gridDim.z;
+  if (!a.tiles)
+    return make_int2(0, tile);
+  const int2 t = a.tiles[tile];
+  return make_int2(__builtin_amdgcn_readfirstlane(t.x), __builtin_amdgcn_readfirstlane(t.y));
+}
+// That instance, in scalar registers (said explicitly: merged from two
+// sources, its fields would otherwise occupy vector registers throughout the
+// kernel, 40 of them in the row sweep).
+template <class INST>
+__device__ __forceinline__ INST launch_inst(const fused_launch<INST> &a, int i)
+{
+  if (!a.tiles)
+    return a.one;
+  static_assert(sizeof(INST) % 4 == 0, "whole words");
+  using gword = const __attribute__((address_space(1))) int;
+  gword *src = (gword *) (a.insts + i);
+  int w[sizeof(INST) / 4];
+  for (unsigned k = 0; k < sizeof(INST) / 4; ++k)
+    w[k] = __builtin_amdgcn_readfirstlane(src[k]);
+  INST r;
+  __builtin_memcpy(&r, w, sizeof(INST));
+  return r;
+}
+
+using gslot = const __attribute__((address_space(1))) step_slot;
+
+// The loop variables of a slot, through the global address space (scalar loads).
+__device__ __forceinline__ step_vars slot_vars(gslot *s)
+{
+  step_vars v;
+  v.t = s->v.t;
+  v.h = s->v.h;
+  v.te = s->v.te;
+  v.tol = s->v.tol;
+  v.acc = s->v.acc;
+  v.rej = s->v.rej;
+  v.cur = s->v.cur;
+  v.done = s->v.done;
+  v.step_limit = s->v.step_limit;
+  v.ord = s->v.ord;
+  return v;
+}
+
+// The loop variables as the host sees them (one thread).
+__device__ inline void publish(state *st, const step_vars &v, double err)
+{
+  st->v.t = v.t;
+  st->v.h = v.h;
+  st->v.acc = v.acc;
+  st->v.rej = v.rej;
+  st->v.cur = v.cur;
+  st->v.done = v.done;
+  st->err = err;
+}
+
+struct step_now {
+  double h;
+  int cur, done;
+};
+struct step_lds {
+  double h;
+  int cur, done;
+  unsigned long long *err;   // this step's error accumulator, for step_fold: kept
+                             // here, it occupies no scalar registers meanwhile
+};
+
+// The start of a fused step, called by every thread of every workgroup: the
+// pending control of the attempt before, in the first wavefront, handed to
+// the others through LDS (one barrier).  leader: the one workgroup of the instance that writes the
+// next slot and clears the accumulator of the launch after next.
+__device__ inline step_now step_begin(const step_refs &R, int r, bool leader, step_lds &x)
+{
+  if (threadIdx.x < 64) {
+    gslot *s = (gslot *) &R.ring->slot[r];
+    using gu64 = const __attribute__((address_space(1))) unsigned long long;
+    const unsigned long long bits = *(gu64 *) &R.ring->err[r].bits;
+    step_vars v = slot_vars(s);
+    const int pending = s->pending;
+    lane_pow_tables T;
+    T.load();
+    if (pending) {
+      const double err = __longlong_as_double(static_cast<long long>(bits));
+      if (leader && threadIdx.x == 0)
+        trace_attempt(R.st, v, err);
+      double px = 0.0, py = 0.0;
+      const bool need = ctrl_decide(v, err, px, py);
+      ctrl_finish(v, need, need ? libm_pow(px, py, T) : 0.0);
+      if (leader && threadIdx.x == 0)
+        publish(R.st, v, err);
+    }
+    if (threadIdx.x == 0) {
+      x.h = v.h;
+      x.cur = v.cur;
+      x.done = v.done;
+      x.err = &R.ring->err[(r + 1) & (kRing - 1)].bits;
+      if (leader) {
+        step_slot &o = R.ring->slot[(r + 1) & (kRing - 1)];
+        o.v = v;
+        o.pending = !v.done;
+        __hip_atomic_store(&R.ring->err[(r + 2) & (kRing - 1)].bits, 0ull, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+  }
+  __syncthreads();
+  step_now n;
+  n.h = wave_uniform(x.h);
+  n.cur = __builtin_amdgcn_readfirstlane(x.cur);
+  n.done = __builtin_amdgcn_readfirstlane(x.done);
+  return n;
+}
+
+// The end of a fused step, called by every thread: folds the error maximum
+// (zero: some divisor was 0, the 1.7e308 sentinel) into the accumulator the
+// next launch reads.  red must hold blockDim.x/64 doubles of LDS.
+__device__ inline void step_fold(const step_lds &x, double qmax, unsigned int zero, double *red)
+{
+  const int wid = threadIdx.x >> 6;
+  const int nw = (blockDim.x + 63) >> 6;
+  if (zero)
+    qmax = fmax(qmax, 1.7E308);
+  qmax = wave_max63(qmax);
+  if ((threadIdx.x & 63) == 63)
+    red[wid] = qmax;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double m = red[0];
+    for (int w = 1; w < nw; ++w)
+      m = fmax(m, red[w]);
+    __hip_atomic_fetch_max(x.err, static_cast<unsigned long long>(__double_as_longlong(m)),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// ---- end of a full-storage step ----------------------------------------------
+// Folds each thread's (qmax, zero) into the step accumulators and runs the
+// control in the last workgroup of the grid to finish.  Must be called by all
+// threads of the block.  red must hold blockDim.x/64 doubles of LDS.
+__device__ inline void block_finish(state *st, double qmax, unsigned int zero, double *red,
+                                    unsigned int *zred)
+{
+  const unsigned int nblocks = gridDim.x * gridDim.y * gridDim.z;
   const int lane = threadIdx.x & 63;
   const int wid = threadIdx.x >> 6;
   const int nw = (blockDim.x + 63) >> 6;
-  qmax = wave_max(qmax);
+  qmax = wave_max63(qmax);
   const unsigned long long zb = __ballot(zero != 0u);
-  if (lane == 0) {
+  if (lane == 63) {
     red[wid] = qmax;
     zred[wid] = zb ? 1u : 0u;
   }
@@ -302,10 +475,10 @@ __device__ inline void block_finish(state *st, double qmax, unsigned int zero, d
     if (threadIdx.x == 0) {
       __threadfence();
       pm = dev_control(st) ? 1 : 0;
-      hn = st->h;
+      hn = st->v.h;
     }
     __syncthreads();
-    if (pm && coef)
+    if (pm)
       premult_block(*st->meth, st->s, hn, *st->coef, static_cast<int>(threadIdx.x),
                     static_cast<int>(blockDim.x));
   }

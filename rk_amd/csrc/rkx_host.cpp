@@ -2,8 +2,8 @@
 //
 // The step loop of the reference's solver() (src/impl/seq/D.c:58-78) runs on
 // the device: every step's kernels read t, h and the current-buffer index from
-// a device-resident state and the last workgroup of the step's final kernel
-// decides accept/reject and the next h.  The host only enqueues chunks of
+// a device-resident state, and the step control (accept/reject and the next
+// h) runs on the device as well.  The host only enqueues chunks of
 // steps, captured once as a hipGraph, and polls the state between chunks;
 // kernels of a chunk that run past the end of the integration return at once.
 #include "rkx_internal.hpp"
@@ -169,15 +169,29 @@ struct graph_holder {
 
 }  // namespace
 
-// The step control on the host: ctrl_decide/ctrl_finish with the C library's
-// pow, then the premultiplied coefficients of the next step.
-void host_finish(state &st, const dev_method &dm, dev_coef &hc)
+// The step control on the host: ctrl_decide/ctrl_finish with the C library's pow.
+void host_finish(step_vars &v, double err)
 {
-  const bool need = ctrl_decide(st);
-  const double p = need ? std::pow(st.pow_x, st.pow_y) : 0.0;
-  ctrl_finish(st, need, p);
-  premult(dm, st.s, st.h, hc);
+  double px = 0.0, py = 0.0;
+  const bool need = ctrl_decide(v, err, px, py);
+  ctrl_finish(v, need, need ? std::pow(px, py) : 0.0);
 }
+
+step_ring make_ring(const step_vars &v)
+{
+  step_ring g{};
+  g.slot[0].v = v;
+  return g;
+}
+
+// The control block of a solve: everything small that its kernels read, in
+// one allocation and one copy.
+struct solve_ctl {
+  state st;
+  step_ring ring;
+  dev_method meth;
+  dev_coef coef;
+};
 
 // DUMP output (include/tools.h:239-256): one line per attempted step, t and
 // h then every component of the step's new y, "%.20e" separated by tabs.  The
@@ -527,15 +541,12 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
   double *ybuf[2] = {nullptr, nullptr};
   double *w = nullptr, *dy = nullptr, *err = nullptr, *trace_dev = nullptr;
   double *v = nullptr, *w1 = nullptr;   // gather forms: v_0..v_{s-1}; F's second w
-  state *st_dev = nullptr;
-  dev_method *dm_dev = nullptr;
-  dev_coef *cf_dev = nullptr;
-  if (int rc = mem.alloc(reinterpret_cast<void **>(&st_dev), sizeof(state)))
+  solve_ctl *ctl_dev = nullptr;
+  if (int rc = mem.alloc(reinterpret_cast<void **>(&ctl_dev), sizeof(solve_ctl)))
     return rc;
-  if (int rc = mem.alloc(reinterpret_cast<void **>(&dm_dev), sizeof(dev_method)))
-    return rc;
-  if (int rc = mem.alloc(reinterpret_cast<void **>(&cf_dev), sizeof(dev_coef)))
-    return rc;
+  state *st_dev = &ctl_dev->st;
+  dev_coef *cf_dev = &ctl_dev->coef;
+  const step_refs ref{st_dev, &ctl_dev->ring, &ctl_dev->meth};
   for (int b = 0; b < 2; ++b)
     if (int rc = mem.alloc(reinterpret_cast<void **>(&ybuf[b]), vec))
       return rc;
@@ -561,28 +572,28 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
                            sizeof(double) * 3 * static_cast<size_t>(o.trace_cap)))
       return rc;
 
-  dev_method dm;
-  fill_dev_method(*m, dm);
-  state hs{};
-  hs.t = t0;
-  hs.te = te;
-  hs.tol = tol;
-  hs.h = initial_h(te - t0, tol, o.step_limit, o.h0);
-  hs.step_limit = o.step_limit;
-  hs.ord = m->ord;
+  solve_ctl hc{};
+  fill_dev_method(*m, hc.meth);
+  state &hs = hc.st;
+  hs.v.t = t0;
+  hs.v.te = te;
+  hs.v.tol = tol;
+  hs.v.h = initial_h(te - t0, tol, o.step_limit, o.h0);
+  hs.v.step_limit = o.step_limit;
+  hs.v.ord = m->ord;
+  hs.v.done = !(t0 < te);
   hs.ctrl = o.ctrl;
   hs.trace = trace_dev;
   hs.trace_cap = o.trace_cap;
   hs.s = s;
-  hs.meth = dm_dev;
+  hs.meth = &ctl_dev->meth;
   hs.coef = cf_dev;
-  dev_coef hc{};
-  premult(dm, s, hs.h, hc);
-  hs.cur = 0;
-  hs.done = !(t0 < te);
-  RKX_HIP(hipMemcpyAsync(dm_dev, &dm, sizeof(dm), hipMemcpyHostToDevice, stream));
-  RKX_HIP(hipMemcpyAsync(cf_dev, &hc, sizeof(hc), hipMemcpyHostToDevice, stream));
-  RKX_HIP(hipMemcpyAsync(st_dev, &hs, sizeof(hs), hipMemcpyHostToDevice, stream));
+  if (fused) {
+    hs.ring = ref.ring;
+    hc.ring = make_ring(hs.v);
+  }
+  premult(hc.meth, s, hs.v.h, hc.coef);
+  RKX_HIP(hipMemcpyAsync(ctl_dev, &hc, sizeof(hc), hipMemcpyHostToDevice, stream));
   RKX_HIP(hipMemcpyAsync(ybuf[0], y0_dev, vec, hipMemcpyDeviceToDevice, stream));
 
   sweep_cfg cfg{1, 1};
@@ -595,42 +606,37 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
   if (cfg.waves < 1 || cfg.waves > 4 || cfg.rows < 1 || 64 * cfg.waves <= 2 * s)
     return fail(RKX_EINVAL, "rkx_solve: tile_waves must be 1..4 (and wider than 2s), "
                             "tile_rows >= 1");
-  sweep_inst *inst_dev = nullptr;
-  chain_inst *chain_dev = nullptr;
-  int ntiles = 0;
+  fused_launch<sweep_inst> sl{};
+  fused_launch<chain_inst> cl{};
   bool gen_rows = false;   // the general ghost-row form (sweep_inst_single_reflect)
   const int pattern = sweep_pattern(*m);
   if (sweep && sweep_resident_blocks(pattern, cfg.waves) < 1)
     return fail(RKX_EINVAL, "rkx_solve: tile_waves wider than this table's fused kernel "
                             "(DOPRI87: at most 2)");
   if (chain) {
-    if (int rc = mem.alloc(reinterpret_cast<void **>(&chain_dev), sizeof(chain_inst)))
-      return rc;
-    const chain_inst hi = make_chain_inst(dp, *m, st_dev, ybuf[0], ybuf[1]);
-    ntiles = hi.nwg;
-    RKX_HIP(hipMemcpyAsync(chain_dev, &hi, sizeof(hi), hipMemcpyHostToDevice, stream));
-    RKX_HIP(hipStreamSynchronize(stream));
+    cl.one = make_chain_inst(dp, *m, ref, ybuf[0], ybuf[1]);
+    cl.ntiles = cl.one.nwg;
   } else if (sweep) {
-    if (int rc = mem.alloc(reinterpret_cast<void **>(&inst_dev), sizeof(sweep_inst)))
-      return rc;
-    const sweep_inst hi = make_sweep_inst(dp, *m, cfg, st_dev, ybuf[0], ybuf[1]);
-    ntiles = hi.ntiles;
-    gen_rows = !sweep_inst_single_reflect(pattern, s, hi);
-    RKX_HIP(hipMemcpyAsync(inst_dev, &hi, sizeof(hi), hipMemcpyHostToDevice, stream));
-    RKX_HIP(hipStreamSynchronize(stream));
+    sl.one = make_sweep_inst(dp, *m, cfg, ref, ybuf[0], ybuf[1]);
+    sl.ntiles = sl.one.ntiles;
+    gen_rows = !sweep_inst_single_reflect(pattern, s, sl.one);
   }
 
-  auto enqueue_step = [&]() -> hipError_t {
+  // one attempted step; r: the ring slot a fused kernel reads
+  auto enqueue_step = [&](int r) -> hipError_t {
     if (impl == RKX_IMPL_D)
       return launch_d_step(dp, cf_dev, s, st_dev, ybuf[0], ybuf[1], w, dy, err, stream);
     if (gather)
       return launch_gather_step(impl, dp, cf_dev, s, nz, st_dev, ybuf[0], ybuf[1], v, w, w1,
                                 stream);
     if (pairs)
-      return launch_lv_step(dp, cf_dev, s, st_dev, ybuf[0], ybuf[1], stream);
-    if (chain)
-      return launch_chain(pattern, chain_dev, nullptr, ntiles, stream);
-    return launch_sweep(pattern, cfg.waves, gen_rows, inst_dev, nullptr, ntiles, stream);
+      return launch_lv_step(dp, s, ref, ybuf[0], ybuf[1], r, stream);
+    if (chain) {
+      cl.r = r;
+      return launch_chain(pattern, cl, stream);
+    }
+    sl.r = r;
+    return launch_sweep(pattern, cfg.waves, gen_rows, sl, stream);
   };
 
   state *hs_pinned = nullptr;   // [0], [1]: snapshots of two chunks in flight
@@ -644,19 +650,28 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
   RKX_HIP(hipStreamSynchronize(stream));
   const auto t_start = std::chrono::steady_clock::now();
 
-  if (hs.done) {
+  if (hs.v.done) {
     hs_pinned[0] = hs;
   } else if (o.ctrl == RKX_CTRL_HOST) {
     // One host round trip per step: the device computes the error norm, the
     // host runs the reference's step control with the C library's pow.
-    state cur = hs;
+    step_vars cur = hs.v;
     dump_file dump;
     std::vector<double> ydump;
-    while (!cur.done) {
-      RKX_HIP(enqueue_step());
-      RKX_HIP(hipMemcpyAsync(hs_pinned, st_dev, sizeof(state), hipMemcpyDeviceToHost, stream));
-      RKX_HIP(hipStreamSynchronize(stream));
-      cur = hs_pinned[0];
+    for (int r = 0; !cur.done;) {
+      RKX_HIP(enqueue_step(r));
+      r = (r + 1) & (kRing - 1);
+      double step_err;
+      if (fused) {
+        RKX_HIP(hipMemcpyAsync(&hs_pinned->err, &ref.ring->err[r].bits, sizeof(double),
+                               hipMemcpyDeviceToHost, stream));
+        RKX_HIP(hipStreamSynchronize(stream));
+        step_err = hs_pinned->err;
+      } else {
+        RKX_HIP(hipMemcpyAsync(hs_pinned, st_dev, sizeof(state), hipMemcpyDeviceToHost, stream));
+        RKX_HIP(hipStreamSynchronize(stream));
+        step_err = hs_pinned->err;
+      }
       const int attempt = cur.acc + cur.rej;
       if (o.dump_path) {
         // the step's new y is in the other buffer until the decision flips cur
@@ -668,15 +683,22 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
       if (o.trace && attempt < o.trace_cap) {
         o.trace[3 * attempt + 0] = cur.t;
         o.trace[3 * attempt + 1] = cur.h;
-        o.trace[3 * attempt + 2] = cur.err;
+        o.trace[3 * attempt + 2] = step_err;
       }
-      host_finish(cur, dm, hc);
-      RKX_HIP(hipMemcpyAsync(cf_dev, &hc, sizeof(hc), hipMemcpyHostToDevice, stream));
-      hs_pinned[0] = cur;
-      RKX_HIP(hipMemcpyAsync(st_dev, hs_pinned, sizeof(state), hipMemcpyHostToDevice, stream));
+      host_finish(cur, step_err);
+      if (fused) {
+        const step_slot next{cur, 0};
+        RKX_HIP(hipMemcpyAsync(&ref.ring->slot[r], &next, sizeof(next), hipMemcpyHostToDevice,
+                               stream));
+      } else {
+        premult(hc.meth, s, cur.h, hc.coef);
+        RKX_HIP(hipMemcpyAsync(cf_dev, &hc.coef, sizeof(hc.coef), hipMemcpyHostToDevice, stream));
+        hs_pinned->v = cur;
+        RKX_HIP(hipMemcpyAsync(st_dev, hs_pinned, sizeof(state), hipMemcpyHostToDevice, stream));
+      }
+      RKX_HIP(hipStreamSynchronize(stream));
     }
-    RKX_HIP(hipStreamSynchronize(stream));
-    hs_pinned[0] = cur;
+    hs_pinned[0].v = cur;
   } else {
     // Chunks of steps captured once as a graph.  The host keeps two chunks in
     // flight: it enqueues chunk k+1 (and a snapshot copy of the state) before
@@ -686,12 +708,12 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
     // per snapshot (a short solve keeps short chunks: after the last step
     // every launch in flight returns at once, but still costs its launch).
     constexpr int kChunkGrowAfter = 8, kChunkReps = 4;
-    const int chunk = fused ? 32 : 16;
+    const int chunk = fused ? 32 : 16;   // a multiple of kRing: every chunk starts at slot 0
     graph_holder gh;
     RKX_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
     hipError_t cap_err = hipSuccess;
     for (int k = 0; k < chunk && cap_err == hipSuccess; ++k)
-      cap_err = enqueue_step();
+      cap_err = enqueue_step(k & (kRing - 1));
     hipError_t end_err = hipStreamEndCapture(stream, &gh.g);
     if (cap_err != hipSuccess)
       return fail(RKX_EDEVICE, std::string("kernel launch during capture failed: ") +
@@ -727,11 +749,11 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
       if (int rc = launch_chunk(b))
         return rc;
       RKX_HIP(hipEventSynchronize(ev[a]));
-      if (hs_pinned[a].done)
+      if (hs_pinned[a].v.done)
         break;
       // every chunk must advance the attempt counter; a chunk that does not
       // means the device-side step control is not running -- stop, do not spin
-      const int att = hs_pinned[a].acc + hs_pinned[a].rej;
+      const int att = hs_pinned[a].v.acc + hs_pinned[a].v.rej;
       stalled = (att == last_attempts) ? stalled + 1 : 0;
       last_attempts = att;
       if (stalled >= 3) {
@@ -743,7 +765,7 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
     RKX_HIP(hipMemcpy(&hs_pinned[0], st_dev, sizeof(state), hipMemcpyDeviceToHost));
   }
   const auto t_end = std::chrono::steady_clock::now();
-  const state fin = hs_pinned[0];
+  const step_vars fin = hs_pinned[0].v;
   RKX_HIP(hipMemcpyAsync(y_dev, ybuf[fin.cur], vec, hipMemcpyDeviceToDevice, stream));
   if (o.trace_cap > 0 && o.ctrl != RKX_CTRL_HOST) {
     const int ntr = std::min(o.trace_cap, fin.acc + fin.rej);

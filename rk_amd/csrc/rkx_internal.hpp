@@ -64,26 +64,57 @@ struct dev_coef {
   double col[RKX_MAX_STAGES][RKX_MAX_STAGES + 2];
 };
 
-// Integration state of one solve, resident in device memory.  Written only by
-// the step control (the last workgroup of a step, or the host).
-struct alignas(64) state {
+// What the step control reads and updates: the loop variables of one solve.
+struct step_vars {
   double t, h, te, tol;
-  double err;                        // error norm of the last attempt
-  unsigned long long err_bits;       // atomicMax accumulator (bits of a double >= 0)
-  unsigned int zero_div;             // some divisor max(|y|,|y_old|) was 0
-  unsigned int blocks_done;          // last-workgroup detection
   int acc, rej;
   int cur;                           // which of the two y buffers holds y
   int done;                          // the step loop has ended
   int step_limit;
   int ord;
+};
+
+// The step ring of an instance with a fused kernel (one launch per attempted
+// step).  Launch number k of an instance reads slot k & 3, runs the step
+// control of the attempt before it (pending) in every workgroup from the
+// error maximum in err[k & 3], makes its own attempt, folds its error into
+// err[(k+1) & 3] and leaves the loop variables it worked with in slot
+// (k+1) & 3.  Every workgroup computes the same control from the same values,
+// so a step ends with one atomic maximum per workgroup and no workgroup waits
+// for another: counting the workgroups that finished and running the control
+// in the last of them cost two atomics in a row, a device-wide fence and the
+// control itself at the end of every step, with nothing to overlap them (one
+// pair of LV: 7.1 us per step).
+constexpr int kRing = 4;
+struct alignas(64) step_slot {
+  step_vars v;
+  int pending;                       // the attempt from v awaits its control
+};
+struct step_ring {
+  step_slot slot[kRing];
+  struct alignas(128) {
+    unsigned long long bits;         // atomic maximum: bits of a double >= 0
+  } err[kRing];
+};
+
+struct state;
+
+// Integration state of one solve, resident in device memory.  Written only by
+// the step control (the last workgroup of a full-storage step, the first
+// workgroup of a fused one, or the host).
+struct alignas(64) state {
+  step_vars v;
+  double err;                        // error norm of the last attempt
+  unsigned long long err_bits;       // atomicMax accumulator (bits of a double >= 0)
+  unsigned int zero_div;             // some divisor max(|y|,|y_old|) was 0
+  unsigned int blocks_done;          // last-workgroup detection
   int ctrl;                          // RKX_CTRL_*
   int trace_cap;
   int s;                             // stages
-  double pow_x, pow_y;               // arguments of the step's pow (ctrl_decide)
   double *trace;                     // device buffer, 3 doubles per attempt
   const dev_method *meth;            // raw coefficients for the premultiplication
   dev_coef *coef;                    // premultiplied coefficients of the next step
+  step_ring *ring;                   // fused kernels (nullptr: full storage)
 };
 
 // premult of the raw table by h (identical on host and device)
@@ -104,39 +135,39 @@ __host__ __device__ inline void premult(const dev_method &m, int s, double h, de
 }
 
 // Step control of include/tools.h:235-278, split at the one libm call.
-// ctrl_decide: accept/reject with st.err, advance t and the counters, and set
-// pow_x = tol/err, pow_y = 1/(ord+1).  Returns true when the new h needs
-// p = pow(pow_x, pow_y) (variable step size).
-__host__ __device__ inline bool ctrl_decide(state &st)
+// ctrl_decide: accept/reject with err, advance t and the counters, and give
+// pow's arguments x = tol/err, y = 1/(ord+1).  Returns true when the new h
+// needs p = pow(x, y) (variable step size).
+__host__ __device__ inline bool ctrl_decide(step_vars &v, double err, double &x, double &y)
 {
-  if (st.tol <= 0.0) {                 // fixed step size (tools.h:258-263)
-    st.t += st.h;
-    st.acc += 1;
-    st.cur ^= 1;
+  if (v.tol <= 0.0) {                  // fixed step size (tools.h:258-263)
+    v.t += v.h;
+    v.acc += 1;
+    v.cur ^= 1;
     return false;
   }
-  if (st.err <= st.tol) {              // accept (tools.h:264-270)
-    st.t += st.h;
-    st.acc += 1;
-    st.cur ^= 1;
+  if (err <= v.tol) {                  // accept (tools.h:264-270)
+    v.t += v.h;
+    v.acc += 1;
+    v.cur ^= 1;
   } else {                             // reject: y stays in the other buffer
-    st.rej += 1;
+    v.rej += 1;
   }
-  st.pow_x = st.tol / st.err;
-  st.pow_y = 1.0 / (st.ord + 1.0);
+  x = v.tol / err;
+  y = 1.0 / (v.ord + 1.0);
   return true;
 }
 
 // ctrl_finish: h_new_acc/h_new_rej with p (tools.h:221-233), then the
 // for-increment h = fmin(h, te - t) and the loop test of FOR_ALL_GRIDPOINTS
-// (tools.h:191-198).  The caller premultiplies the coefficients with the new h.
-__host__ __device__ inline void ctrl_finish(state &st, bool used_pow, double p)
+// (tools.h:191-198).
+__host__ __device__ inline void ctrl_finish(step_vars &v, bool used_pow, double p)
 {
   if (used_pow)
-    st.h = st.h * fmin(2.0, fmax(0.5, 0.9 * p));
-  st.h = fmin(st.h, st.te - st.t);
-  const int attempts = st.acc + st.rej;
-  st.done = !((st.t < st.te) && (st.step_limit <= 0 || attempts < st.step_limit));
+    v.h = v.h * fmin(2.0, fmax(0.5, 0.9 * p));
+  v.h = fmin(v.h, v.te - v.t);
+  const int attempts = v.acc + v.rej;
+  v.done = !((v.t < v.te) && (v.step_limit <= 0 || attempts < v.step_limit));
 }
 
 // ---- host runtime helpers (rkx_host.cpp) ------------------------------------
@@ -145,9 +176,17 @@ int check_method(const rkx_method *m);
 void fill_dev_method(const rkx_method &m, dev_method &d);
 double initial_h(double H, double tol, int limit, double h0);   // src/tools.c:25-36
 int default_stream(hipStream_t *out);
-// the step control on the host (ctrl_decide/ctrl_finish with the C library's
-// pow) and the next step's premultiplied coefficients
-void host_finish(state &st, const dev_method &dm, dev_coef &hc);
+// the step control on the host: ctrl_decide/ctrl_finish with the C library's pow
+void host_finish(step_vars &v, double err);
+
+// What a fused kernel is given of an instance's device-side step state.
+struct step_refs {
+  state *st;             // published loop variables, trace buffer
+  step_ring *ring;
+  const dev_method *meth;
+};
+// Rings of instances about to run their first step (nothing pending).
+step_ring make_ring(const step_vars &v);
 
 // Kernel launchers (rkx_kernels_*.hip).  All return hipError_t of the launch.
 hipError_t launch_eval_rng(const dev_ode &p, int i, int j, const double *y, double *f,
@@ -158,8 +197,13 @@ hipError_t launch_d_step(const dev_ode &p, const dev_coef *cf, int s, state *st,
 // Stage-fused step of independent LV pairs (rkx_kernels_lvpairs.hip): every
 // table with 2, 3, 4, 7, 8 or 13 stages
 bool pairs_supported(const dev_ode &p, const rkx_method &m);
-hipError_t launch_lv_step(const dev_ode &p, const dev_coef *cf, int s, state *st, double *y0,
-                          double *y1, hipStream_t stream);
+hipError_t launch_lv_step(const dev_ode &p, int s, const step_refs &R, double *y0, double *y1,
+                          int r, hipStream_t stream);
+// Runs the pending step control of n states (those without a ring are left
+// alone), publishes it, and moves each ring on to slot 0 (rkx_kernels_step.hip):
+// after launches that ended on ring slot r, before the host reads the states
+// for good or starts again at slot 0.
+hipError_t launch_step_flush(state *st, int n, int r, hipStream_t stream);
 
 // Gather forms A, E, F (src/impl/seq/A.c, E.c, F.c): non-zero patterns of the
 // raw table (zero_pattern, src/methods.c:24-39) as bit masks, bit i of rowA[l]
@@ -198,7 +242,7 @@ struct sweep_inst {
   int ntiles;            // workgroups that share this state per step
   double coef;           // (alpha*(N-1))*(N-1)
   double *y0, *y1;       // the two y buffers
-  state *st;             // step state; the kernel forms h*A etc. from st->meth
+  step_refs ref;         // the kernel forms h*A etc. from ref.meth
 };
 
 bool sweep_supported(const dev_ode &p, const rkx_method &m);
@@ -220,15 +264,30 @@ bool sweep_inst_single_reflect(int pattern, int s, const sweep_inst &I);
 // Row iterations of tile t of an instance (its band, or the shorter last
 // band, plus the 2(s-1) halo rows; paired bands run the full band height).
 int sweep_tile_iters(int pattern, int s, const sweep_inst &I, int t);
-sweep_inst make_sweep_inst(const dev_ode &p, const rkx_method &m, const sweep_cfg &c, state *st,
-                           double *y0, double *y1);
-// tiles == nullptr: a single instance (insts[0]) with ntiles tiles; gen: the
-// general reflection form (some instance fails sweep_single_reflect)
-hipError_t launch_sweep(int pattern, int K, bool gen, const sweep_inst *insts, const int2 *tiles,
-                        int ntiles, hipStream_t stream);
-// the DOPRI87 kernels (their own translation unit: 13 stages take long to build)
-hipError_t launch_sweep_dopri87(int K, bool gen, const sweep_inst *insts, const int2 *tiles,
-                                int ntiles, hipStream_t stream);
+sweep_inst make_sweep_inst(const dev_ode &p, const rkx_method &m, const sweep_cfg &c,
+                           const step_refs &ref, double *y0, double *y1);
+// A launch of a fused kernel over many instances (device tables) or, with
+// tiles == nullptr, over the one instance it is given by value (its fields
+// then come with the kernel's arguments, which saves a step of its chain of
+// dependent loads).  r: the ring slot every instance of the launch reads.
+template <class INST>
+struct fused_launch {
+  INST one;
+  const INST *insts;
+  const int2 *tiles;
+  int ntiles;
+  int r;
+};
+// gen: the general reflection form (some instance fails sweep_single_reflect)
+hipError_t launch_sweep(int pattern, int K, bool gen, const fused_launch<sweep_inst> &a,
+                        hipStream_t stream);
+// the VERNER65 and DOPRI87 kernels (translation units of their own: many stages
+// take long to build)
+hipError_t launch_sweep_verner65(int K, bool gen, const fused_launch<sweep_inst> &a,
+                                 hipStream_t stream);
+int resident_blocks_verner65(int K);
+hipError_t launch_sweep_dopri87(int K, bool gen, const fused_launch<sweep_inst> &a,
+                                hipStream_t stream);
 int resident_blocks_dopri87(int K);
 // workgroups of the fused kernel resident per CU for a pattern and strip
 // width; 0: the strip is too wide for that table's kernel
@@ -242,13 +301,12 @@ struct chain_inst {
   int nwg;               // workgroups per step (each loops over segments)
   double c0, d0, d1, c1, diff;
   double *y0, *y1;
-  state *st;             // step state; the kernel forms h*A etc. from st->meth
+  step_refs ref;         // the kernel forms h*A etc. from ref.meth
 };
 
 bool chain_supported(const dev_ode &p, const rkx_method &m);
-chain_inst make_chain_inst(const dev_ode &p, const rkx_method &m, state *st, double *y0,
-                           double *y1);
-hipError_t launch_chain(int pattern, const chain_inst *insts, const int2 *tiles, int ntiles,
-                        hipStream_t stream);
+chain_inst make_chain_inst(const dev_ode &p, const rkx_method &m, const step_refs &ref,
+                           double *y0, double *y1);
+hipError_t launch_chain(int pattern, const fused_launch<chain_inst> &a, hipStream_t stream);
 
 }  // namespace rkx

@@ -34,38 +34,34 @@ __device__ __forceinline__ int wrap(long long c, int M)
 }
 
 template <class P>
-__global__ __launch_bounds__(kCB) void k_chain(const chain_inst *__restrict__ insts,
-                                               const int2 *__restrict__ tiles, int ntiles)
+__global__ __launch_bounds__(kCB) void k_chain(fused_launch<chain_inst> a)
 {
   constexpr int s = P::s;
   constexpr int C = kCPT;
   __shared__ double2 edgeL[2][kCB], edgeR[2][kCB];
   __shared__ double red[kCB / 64];
-  __shared__ unsigned int zred[kCB / 64];
+  __shared__ step_lds head;
 
-  const int T = ntiles;
+  const int T = a.ntiles;
   const int b = blockIdx.x;
   const int x8 = b & 7, q = T >> 3, rm = T & 7;
   const int tile = x8 * q + min(x8, rm) + (b >> 3);
-  const int2 td = tiles ? tiles[tile] : make_int2(0, tile);
-  const chain_inst &I = insts[td.x];
-  double *const y0p = I.y0, *const y1p = I.y1;
+  const int2 td = launch_tile(a, tile);
+  const chain_inst I = launch_inst(a, td.x);
   const int M = I.cells;
-  state *st = I.st;
-  const step_view sv = read_step(st);
-  if (sv.done)
+  const step_now sn = step_begin(I.ref, a.r, td.y == 0, head);
+  if (sn.done)
     return;
-  const int cur = sv.cur;
-  const double2 *__restrict__ y = reinterpret_cast<const double2 *>(cur ? y1p : y0p);
-  double2 *__restrict__ yn = reinterpret_cast<double2 *>(cur ? y0p : y1p);
+  const double2 *__restrict__ y = reinterpret_cast<const double2 *>(sn.cur ? I.y1 : I.y0);
+  double2 *__restrict__ yn = reinterpret_cast<double2 *>(sn.cur ? I.y0 : I.y1);
   dev_ode p{};
   p.c0 = I.c0;
   p.d0 = I.d0;
   p.d1 = I.d1;
   p.c1 = I.c1;
   const double D = I.diff;
-  gmethod *__restrict__ mt = as_global(sv.meth);
-  const double h = sv.h;                         // this step's h (uniform)
+  gmethod *__restrict__ mt = as_global(I.ref.meth);
+  const double h = sn.h;                         // this step's h (uniform)
 
   const int t = threadIdx.x;
 
@@ -165,7 +161,7 @@ __global__ __launch_bounds__(kCB) void k_chain(const chain_inst *__restrict__ in
   });
   __syncthreads();                       // the next segment reuses the edge buffers
   }
-  block_finish(st, qmax, zero, red, zred, static_cast<unsigned int>(I.nwg), false);
+  step_fold(head, qmax, zero, red);
 }
 
 }  // namespace
@@ -176,8 +172,8 @@ bool chain_supported(const dev_ode &p, const rkx_method &m)
   return p.kind == RKX_LV_CHAIN && pat >= 1 && pat <= 6 && kT > 2 * m.s;
 }
 
-chain_inst make_chain_inst(const dev_ode &p, const rkx_method &m, state *st, double *y0,
-                           double *y1)
+chain_inst make_chain_inst(const dev_ode &p, const rkx_method &m, const step_refs &ref,
+                           double *y0, double *y1)
 {
   chain_inst I{};
   I.cells = p.cells;
@@ -191,18 +187,17 @@ chain_inst make_chain_inst(const dev_ode &p, const rkx_method &m, state *st, dou
   I.diff = p.diff;
   I.y0 = y0;
   I.y1 = y1;
-  I.st = st;
+  I.ref = ref;
   return I;
 }
 
-hipError_t launch_chain(int pattern, const chain_inst *insts, const int2 *tiles, int ntiles,
-                        hipStream_t stream)
+hipError_t launch_chain(int pattern, const fused_launch<chain_inst> &a, hipStream_t stream)
 {
-  if (ntiles <= 0)
+  if (a.ntiles <= 0)
     return hipSuccess;
   return dispatch_pattern(pattern, [&](auto pat) {
     using P = decltype(pat);
-    hipLaunchKernelGGL(k_chain<P>, dim3(ntiles), dim3(kCB), 0, stream, insts, tiles, ntiles);
+    hipLaunchKernelGGL(k_chain<P>, dim3(a.ntiles), dim3(kCB), 0, stream, a);
     return hipGetLastError();
   });
 }

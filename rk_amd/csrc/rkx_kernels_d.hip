@@ -27,7 +27,7 @@ constexpr int kLastBlocks = 256;
 
 __device__ __forceinline__ double *ycur(state *st, double *y0, double *y1)
 {
-  return st->cur ? y1 : y0;
+  return st->v.cur ? y1 : y0;
 }
 
 __global__ __launch_bounds__(kBlock) void k_d_first(dev_ode p, const dev_coef *__restrict__ m,
@@ -36,7 +36,7 @@ __global__ __launch_bounds__(kBlock) void k_d_first(dev_ode p, const dev_coef *_
                                                     double *__restrict__ dy,
                                                     double *__restrict__ err)
 {
-  if (st->done)
+  if (st->v.done)
     return;
   const int cell = blockIdx.x * kBlock + threadIdx.x;
   if (cell >= p.cells)
@@ -65,7 +65,7 @@ __global__ __launch_bounds__(kBlock) void k_d_interm(dev_ode p, const dev_coef *
                                                      double *__restrict__ dy,
                                                      double *__restrict__ err)
 {
-  if (st->done)
+  if (st->v.done)
     return;
   const int cell = blockIdx.x * kBlock + threadIdx.x;
   if (cell >= p.cells)
@@ -103,9 +103,9 @@ __global__ __launch_bounds__(kLastThreads) void k_d_last(dev_ode p,
 {
   __shared__ double red[kLastThreads / 64];
   __shared__ unsigned int zred[kLastThreads / 64];
-  if (st->done)
+  if (st->v.done)
     return;                       // uniform: every block of the grid returns
-  const int cur = st->cur;
+  const int cur = st->v.cur;
   const double *y = cur ? y1 : y0;
   double *ynew = cur ? y0 : y1;
   double qmax = 0.0;

@@ -33,7 +33,7 @@ constexpr int kGOutBlocks = 256;
 
 __device__ __forceinline__ const double *gcur(const state *st, const double *y0, const double *y1)
 {
-  return st->cur ? y1 : y0;
+  return st->v.cur ? y1 : y0;
 }
 
 // v_l = f(w) on every cell (block_rhs); stage 0 reads the current y
@@ -42,7 +42,7 @@ __global__ __launch_bounds__(kGBlock) void k_g_rhs(dev_ode p, int l, state *st,
                                                    const double *__restrict__ w,
                                                    double *__restrict__ v)
 {
-  if (st->done)
+  if (st->v.done)
     return;
   const int cell = blockIdx.x * kGBlock + threadIdx.x;
   if (cell >= p.cells)
@@ -64,7 +64,7 @@ __global__ __launch_bounds__(kGBlock) void k_g_gather(dev_ode p, const dev_coef 
                                                       const double *__restrict__ v,
                                                       double *__restrict__ w)
 {
-  if (st->done)
+  if (st->v.done)
     return;
   const int cell = blockIdx.x * kGBlock + threadIdx.x;
   if (cell >= p.cells)
@@ -93,7 +93,7 @@ __global__ __launch_bounds__(kGBlock) void k_g_rhs_gather(dev_ode p,
                                                           double *__restrict__ v,
                                                           double *__restrict__ wn)
 {
-  if (st->done)
+  if (st->v.done)
     return;
   const int cell = blockIdx.x * kGBlock + threadIdx.x;
   if (cell >= p.cells)
@@ -131,9 +131,9 @@ __global__ __launch_bounds__(kGOutThreads) void k_g_output(dev_ode p,
 {
   __shared__ double red[kGOutThreads / 64];
   __shared__ unsigned int zred[kGOutThreads / 64];
-  if (st->done)
+  if (st->v.done)
     return;
-  const int cur = st->cur;
+  const int cur = st->v.cur;
   const double *y = cur ? y1 : y0;
   double *ynew = cur ? y0 : y1;
   const size_t n = static_cast<size_t>(p.n);

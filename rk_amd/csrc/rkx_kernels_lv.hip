@@ -43,7 +43,7 @@ __global__ __launch_bounds__(kLvBlock) void k_lv_ensemble(int count, lv_method m
   p.d1 = prm[4 * k + 2];
   p.c1 = prm[4 * k + 3];
   double y[2] = {y0[2 * k], y0[2 * k + 1]};
-  state st{};
+  step_vars st{};
   st.t = t0;
   st.te = te;
   st.tol = tol;
@@ -89,14 +89,14 @@ __global__ __launch_bounds__(kLvBlock) void k_lv_ensemble(int count, lv_method m
     unsigned int zero = 0u;
     err_term(er[0], yn[0], y[0], q, zero);
     err_term(er[1], yn[1], y[1], q, zero);
-    st.err = zero ? fmax(1.7E308, q) : q;
     const int cur_before = st.cur;
-    const bool need = ctrl_decide(st);
+    double px = 0.0, py = 0.0;
+    const bool need = ctrl_decide(st, zero ? fmax(1.7E308, q) : q, px, py);
     if (st.cur != cur_before) {          // accepted: y <- y_new
       y[0] = yn[0];
       y[1] = yn[1];
     }
-    ctrl_finish(st, need, need ? libm_pow(st.pow_x, st.pow_y, dev_pow_tables) : 0.0);
+    ctrl_finish(st, need, need ? libm_pow(px, py, dev_pow_tables) : 0.0);
     ++attempts;
   }
   yout[2 * k] = y[0];

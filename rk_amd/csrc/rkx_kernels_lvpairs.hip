@@ -8,8 +8,8 @@
 // as in seq D), so the step equals D's bitwise.  It reads y once and writes
 // y_new once into the other y buffer: 16 bytes in and 16 out per pair per
 // step, the low-storage form (two vectors of n) of a problem whose stencil
-// needs no halo.  The error max-norm is folded per workgroup and the last
-// workgroup runs the step control (block_finish).
+// needs no halo.  The error max-norm is folded per workgroup; the next step's
+// kernel runs the control (step_begin).
 #include "rkx_device.hpp"
 
 #include <algorithm>
@@ -24,18 +24,41 @@ namespace {
 constexpr int kPBlock = 1024;
 constexpr int kPMaxBlocks = 256;
 
+// h times the table, in the layout the stages read it: row S-1-i.. of A below
+// the diagonal by consuming stage, then b and e.  Tables of up to 8 stages
+// move to scalar registers; 13 stages (182 coefficients) stay in LDS.
 template <int S>
-__global__ __launch_bounds__(kPBlock) void k_lv_step(dev_ode p, const dev_coef *__restrict__ m,
-                                                    state *st, double *y0, double *y1)
+__global__ __launch_bounds__(kPBlock) void k_lv_step(dev_ode p, step_refs R, int r, double *y0,
+                                                    double *y1)
 {
   __shared__ double red[kPBlock / 64];
-  __shared__ unsigned int zred[kPBlock / 64];
-  const step_view sv = read_step(st);
-  if (sv.done)
+  __shared__ step_lds head;
+  __shared__ double cl[S * (S + 2)];
+  const step_now sn = step_begin(R, r, blockIdx.x == 0, head);
+  if (sn.done)
     return;                       // uniform: every block of the grid returns
-  const int cur = sv.cur;
-  const double *y = cur ? y1 : y0;
-  double *ynew = cur ? y0 : y1;
+  for (int k = threadIdx.x; k < S * (S + 2); k += kPBlock) {
+    const int i = k / (S + 2), l = k - i * (S + 2);
+    const double *src = (l < S) ? &R.meth->A[i * RKX_MAX_STAGES + l]
+                                : (l == S ? &R.meth->b[i] : &R.meth->e[i]);
+    cl[k] = sn.h * *src;
+  }
+  __syncthreads();
+  // coefficient l of row i: l < i h A[i][l], S h b[i], S + 1 h e[i]
+  double cs[S <= 8 ? S * (S + 2) : 1];
+  if constexpr (S <= 8) {
+#pragma unroll
+    for (int k = 0; k < S * (S + 2); ++k)
+      cs[k] = wave_uniform(cl[k]);
+  }
+  auto cf = [&](int i, int l) -> double {
+    if constexpr (S <= 8)
+      return cs[i * (S + 2) + l];
+    else
+      return cl[i * (S + 2) + l];
+  };
+  const double *y = sn.cur ? y1 : y0;
+  double *ynew = sn.cur ? y0 : y1;
   double qmax = 0.0;
   unsigned int zero = 0u;
   for (int pair = blockIdx.x * kPBlock + threadIdx.x; pair < p.cells;
@@ -46,40 +69,40 @@ __global__ __launch_bounds__(kPBlock) void k_lv_step(dev_ode p, const dev_coef *
     lv_pair(p, Y.x, Y.y, fx, fy);
 #pragma unroll
     for (int l = 1; l < S; ++l) {
-      const double a = m->hA[l * RKX_MAX_STAGES + 0];
+      const double a = cf(l, 0);
       wx[l] = Y.x + a * fx;
       wy[l] = Y.y + a * fy;
     }
-    double dx = m->hb[0] * fx, dyv = m->hb[0] * fy;
-    double ex = m->he[0] * fx, ey = m->he[0] * fy;
+    double dx = cf(0, S) * fx, dyv = cf(0, S) * fy;
+    double ex = cf(0, S + 1) * fx, ey = cf(0, S + 1) * fy;
 #pragma unroll
     for (int i = 1; i < S; ++i) {
       lv_pair(p, wx[i], wy[i], fx, fy);
 #pragma unroll
       for (int l = i + 1; l < S; ++l) {
-        const double a = m->hA[l * RKX_MAX_STAGES + i];
+        const double a = cf(l, i);
         wx[l] += a * fx;
         wy[l] += a * fy;
       }
-      dx += m->hb[i] * fx;
-      dyv += m->hb[i] * fy;
-      ex += m->he[i] * fx;
-      ey += m->he[i] * fy;
+      dx += cf(i, S) * fx;
+      dyv += cf(i, S) * fy;
+      ex += cf(i, S + 1) * fx;
+      ey += cf(i, S + 1) * fy;
     }
     const double2 yn = make_double2(Y.x + dx, Y.y + dyv);
     *reinterpret_cast<double2 *>(ynew + 2 * pair) = yn;
     err_term(ex, yn.x, Y.x, qmax, zero);
     err_term(ey, yn.y, Y.y, qmax, zero);
   }
-  block_finish(st, qmax, zero, red, zred);
+  step_fold(head, qmax, zero, red);
 }
 
 template <int S>
-hipError_t launch_s(const dev_ode &p, const dev_coef *m, state *st, double *y0, double *y1,
+hipError_t launch_s(const dev_ode &p, const step_refs &R, double *y0, double *y1, int r,
                     hipStream_t stream)
 {
   const int grid = std::max(1, std::min((p.cells + kPBlock - 1) / kPBlock, kPMaxBlocks));
-  hipLaunchKernelGGL((k_lv_step<S>), dim3(grid), dim3(kPBlock), 0, stream, p, m, st, y0, y1);
+  hipLaunchKernelGGL((k_lv_step<S>), dim3(grid), dim3(kPBlock), 0, stream, p, R, r, y0, y1);
   return hipGetLastError();
 }
 
@@ -95,16 +118,16 @@ bool pairs_supported(const dev_ode &p, const rkx_method &m)
   }
 }
 
-hipError_t launch_lv_step(const dev_ode &p, const dev_coef *m, int s, state *st, double *y0,
-                          double *y1, hipStream_t stream)
+hipError_t launch_lv_step(const dev_ode &p, int s, const step_refs &R, double *y0, double *y1,
+                          int r, hipStream_t stream)
 {
   switch (s) {
-  case 2: return launch_s<2>(p, m, st, y0, y1, stream);
-  case 3: return launch_s<3>(p, m, st, y0, y1, stream);
-  case 4: return launch_s<4>(p, m, st, y0, y1, stream);
-  case 7: return launch_s<7>(p, m, st, y0, y1, stream);
-  case 8: return launch_s<8>(p, m, st, y0, y1, stream);
-  case 13: return launch_s<13>(p, m, st, y0, y1, stream);
+  case 2: return launch_s<2>(p, R, y0, y1, r, stream);
+  case 3: return launch_s<3>(p, R, y0, y1, r, stream);
+  case 4: return launch_s<4>(p, R, y0, y1, r, stream);
+  case 7: return launch_s<7>(p, R, y0, y1, r, stream);
+  case 8: return launch_s<8>(p, R, y0, y1, r, stream);
+  case 13: return launch_s<13>(p, R, y0, y1, r, stream);
   default: return hipErrorInvalidValue;
   }
 }

@@ -1,6 +1,7 @@
 // Host side of the stage-fused BRUSS2D step (rkx_sweep_kernel.hpp): tile
 // geometry and defaults, and the launches of the kernels of the tables with
-// a compiled zero pattern (DOPRI87's are built in rkx_kernels_sweep_dopri87.hip).
+// a compiled zero pattern (VERNER65's and DOPRI87's are built in
+// rkx_kernels_sweep_verner65.hip and rkx_kernels_sweep_dopri87.hip).
 #include "rkx_sweep_kernel.hpp"
 
 #include <algorithm>
@@ -13,7 +14,7 @@ int resident_blocks(int pattern, int K)
 {
   switch (pattern) {
   case 1: return blocks_per_cu_k<pat_dopri54>(K);
-  case 2: return blocks_per_cu_k<pat_verner65>(K);
+  case 2: return resident_blocks_verner65(K);
   case 3: return blocks_per_cu_k<pat_rkf23>(K);
   case 4: return blocks_per_cu_k<pat_heun2>(K);
   case 5: return blocks_per_cu_k<pat_rk4>(K);
@@ -227,8 +228,8 @@ sweep_cfg sweep_default_cfg(const dev_ode &p, const rkx_method &m)
 }
 
 // Geometry of one instance's tiles for strips of 64*K columns and bands of R rows.
-sweep_inst make_sweep_inst(const dev_ode &p, const rkx_method &m, const sweep_cfg &c, state *st,
-                           double *y0, double *y1)
+sweep_inst make_sweep_inst(const dev_ode &p, const rkx_method &m, const sweep_cfg &c,
+                           const step_refs &ref, double *y0, double *y1)
 {
   sweep_inst I{};
   const strip_geom g = strips_of(p.N, m.s, c.waves);
@@ -243,7 +244,7 @@ sweep_inst make_sweep_inst(const dev_ode &p, const rkx_method &m, const sweep_cf
   I.coef = p.coef;
   I.y0 = y0;
   I.y1 = y1;
-  I.st = st;
+  I.ref = ref;
   return I;
 }
 
@@ -251,19 +252,19 @@ int sweep_pattern(const rkx_method &m) { return pattern_of(m); }
 
 int sweep_resident_blocks(int pattern, int K) { return resident_blocks(pattern, K); }
 
-hipError_t launch_sweep(int pattern, int K, bool gen, const sweep_inst *insts, const int2 *tiles,
-                        int ntiles, hipStream_t stream)
+hipError_t launch_sweep(int pattern, int K, bool gen, const fused_launch<sweep_inst> &a,
+                        hipStream_t stream)
 {
-  if (ntiles <= 0)
+  if (a.ntiles <= 0)
     return hipSuccess;
   switch (pattern) {
-  case 1: return launch_pat<pat_dopri54>(K, gen, insts, tiles, ntiles, stream);
-  case 2: return launch_pat<pat_verner65>(K, gen, insts, tiles, ntiles, stream);
-  case 3: return launch_pat<pat_rkf23>(K, gen, insts, tiles, ntiles, stream);
-  case 4: return launch_pat<pat_heun2>(K, gen, insts, tiles, ntiles, stream);
-  case 5: return launch_pat<pat_rk4>(K, gen, insts, tiles, ntiles, stream);
-  case 6: return launch_pat<pat_ssprk3>(K, gen, insts, tiles, ntiles, stream);
-  case 7: return launch_sweep_dopri87(K, gen, insts, tiles, ntiles, stream);
+  case 1: return launch_pat<pat_dopri54>(K, gen, a, stream);
+  case 2: return launch_sweep_verner65(K, gen, a, stream);
+  case 3: return launch_pat<pat_rkf23>(K, gen, a, stream);
+  case 4: return launch_pat<pat_heun2>(K, gen, a, stream);
+  case 5: return launch_pat<pat_rk4>(K, gen, a, stream);
+  case 6: return launch_pat<pat_ssprk3>(K, gen, a, stream);
+  case 7: return launch_sweep_dopri87(K, gen, a, stream);
   default: return hipErrorInvalidValue;
   }
 }

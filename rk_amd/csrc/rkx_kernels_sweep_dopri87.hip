@@ -5,12 +5,12 @@
 
 namespace rkx {
 
-hipError_t launch_sweep_dopri87(int K, bool gen, const sweep_inst *insts, const int2 *tiles,
-                                int ntiles, hipStream_t stream)
+hipError_t launch_sweep_dopri87(int K, bool gen, const fused_launch<sweep_inst> &a,
+                                hipStream_t stream)
 {
-  if (ntiles <= 0)
+  if (a.ntiles <= 0)
     return hipSuccess;
-  return launch_pat<pat_dopri87>(K, gen, insts, tiles, ntiles, stream);
+  return launch_pat<pat_dopri87>(K, gen, a, stream);
 }
 
 int resident_blocks_dopri87(int K) { return blocks_per_cu_k<pat_dopri87>(K); }

@@ -56,8 +56,6 @@ int scratch_ptr(unsigned char **out)
   return RKX_OK;
 }
 
-size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
-
 }  // namespace
 }  // namespace rkx
 
@@ -110,50 +108,39 @@ int rkx_solve_noalloc(const rkx_ode *p, const rkx_method *m, double t0, double t
   if (int rc = scratch_ptr(&base))
     return rc;
 
-  // scratch layout: state | method | coefficients | instance | second y buffer
-  size_t off = 0;
-  state *st_dev = reinterpret_cast<state *>(base + off);
-  off = align_up(off + sizeof(state), 256);
-  dev_method *dm_dev = reinterpret_cast<dev_method *>(base + off);
-  off = align_up(off + sizeof(dev_method), 256);
-  dev_coef *cf_dev = reinterpret_cast<dev_coef *>(base + off);
-  off = align_up(off + sizeof(dev_coef), 256);
-  void *inst_dev = base + off;
-  off = align_up(off + std::max(sizeof(sweep_inst), sizeof(chain_inst)), 256);
-  static_assert(sizeof(state) + sizeof(dev_method) + sizeof(dev_coef) + sizeof(sweep_inst) +
-                        sizeof(chain_inst) + 5 * 256 <= kHeaderBytes,
-                "scratch header too small");
+  // scratch layout: state, ring and method | second y buffer
+  struct header {
+    state st;
+    step_ring ring;
+    dev_method meth;
+  };
+  static_assert(sizeof(header) <= kHeaderBytes, "scratch header too small");
+  header *hd = reinterpret_cast<header *>(base);
+  const step_refs ref{&hd->st, &hd->ring, &hd->meth};
   double *ybuf[2] = {y_dev, reinterpret_cast<double *>(base + kHeaderBytes)};
-  (void) off;
 
   const int s = m->s;
-  dev_method dm;
-  fill_dev_method(*m, dm);
-  state hs{};
-  hs.t = t0;
-  hs.te = te;
-  hs.tol = tol;
-  hs.h = initial_h(te - t0, tol, o.step_limit, o.h0);
-  hs.step_limit = o.step_limit;
-  hs.ord = m->ord;
-  hs.ctrl = o.ctrl;
-  hs.s = s;
-  hs.meth = dm_dev;
-  hs.coef = cf_dev;
-  hs.cur = 0;
-  hs.done = !(t0 < te);
-  dev_coef hc{};
-  premult(dm, s, hs.h, hc);
+  header hh{};
+  fill_dev_method(*m, hh.meth);
+  step_vars &v = hh.st.v;
+  v.t = t0;
+  v.te = te;
+  v.tol = tol;
+  v.h = initial_h(te - t0, tol, o.step_limit, o.h0);
+  v.step_limit = o.step_limit;
+  v.ord = m->ord;
+  v.done = !(t0 < te);
+  hh.st.ring = ref.ring;
+  hh.ring = make_ring(v);
 
   sweep_cfg cfg{1, 1};
   const int pattern = sweep_pattern(*m);
-  int ntiles = 0;
   bool gen_rows = false;   // the general ghost-row form (sweep_inst_single_reflect)
-  sweep_inst si{};
-  chain_inst ci{};
+  fused_launch<sweep_inst> sl{};
+  fused_launch<chain_inst> cl{};
   if (chain) {
-    ci = make_chain_inst(dp, *m, st_dev, ybuf[0], ybuf[1]);
-    ntiles = ci.nwg;
+    cl.one = make_chain_inst(dp, *m, ref, ybuf[0], ybuf[1]);
+    cl.ntiles = cl.one.nwg;
   } else if (!pairs) {
     cfg = sweep_default_cfg(dp, *m);
     if (o.tile_rows > 0)
@@ -164,42 +151,41 @@ int rkx_solve_noalloc(const rkx_ode *p, const rkx_method *m, double t0, double t
         sweep_resident_blocks(pattern, cfg.waves) < 1)
       return fail(RKX_EINVAL, "rkx_solve_noalloc: tile_waves must fit this table's fused kernel "
                               "(1..4, DOPRI87 1..2, wider than 2s), tile_rows >= 1");
-    si = make_sweep_inst(dp, *m, cfg, st_dev, ybuf[0], ybuf[1]);
-    ntiles = si.ntiles;
-    gen_rows = !sweep_inst_single_reflect(pattern, s, si);
+    sl.one = make_sweep_inst(dp, *m, cfg, ref, ybuf[0], ybuf[1]);
+    sl.ntiles = sl.one.ntiles;
+    gen_rows = !sweep_inst_single_reflect(pattern, s, sl.one);
   }
   // everything the kernels read is written before the first launch
   if (y0_dev != y_dev)
     RKX_HIP(hipMemcpyAsync(ybuf[0], y0_dev, n * sizeof(double), hipMemcpyDeviceToDevice, stream));
-  RKX_HIP(hipMemcpyAsync(dm_dev, &dm, sizeof(dm), hipMemcpyHostToDevice, stream));
-  RKX_HIP(hipMemcpyAsync(cf_dev, &hc, sizeof(hc), hipMemcpyHostToDevice, stream));
-  RKX_HIP(hipMemcpyAsync(st_dev, &hs, sizeof(hs), hipMemcpyHostToDevice, stream));
-  if (chain)
-    RKX_HIP(hipMemcpyAsync(inst_dev, &ci, sizeof(ci), hipMemcpyHostToDevice, stream));
-  else if (!pairs)
-    RKX_HIP(hipMemcpyAsync(inst_dev, &si, sizeof(si), hipMemcpyHostToDevice, stream));
+  RKX_HIP(hipMemcpyAsync(hd, &hh, sizeof(hh), hipMemcpyHostToDevice, stream));
   RKX_HIP(hipStreamSynchronize(stream));
 
-  auto step = [&]() -> hipError_t {
+  auto step = [&](int r) -> hipError_t {
     if (pairs)
-      return launch_lv_step(dp, cf_dev, s, st_dev, ybuf[0], ybuf[1], stream);
-    if (chain)
-      return launch_chain(pattern, static_cast<const chain_inst *>(inst_dev), nullptr, ntiles,
-                          stream);
-    return launch_sweep(pattern, cfg.waves, gen_rows, static_cast<const sweep_inst *>(inst_dev),
-                        nullptr, ntiles, stream);
+      return launch_lv_step(dp, s, ref, ybuf[0], ybuf[1], r, stream);
+    if (chain) {
+      cl.r = r;
+      return launch_chain(pattern, cl, stream);
+    }
+    sl.r = r;
+    return launch_sweep(pattern, cfg.waves, gen_rows, sl, stream);
   };
 
   const auto t_start = std::chrono::steady_clock::now();
-  state cur = hs;
+  step_vars cur = v;
   if (!cur.done && o.ctrl == RKX_CTRL_HOST) {
-    while (!cur.done) {
-      RKX_HIP(step());
-      RKX_HIP(hipMemcpyAsync(&cur, st_dev, sizeof(state), hipMemcpyDeviceToHost, stream));
+    for (int r = 0; !cur.done;) {
+      RKX_HIP(step(r));
+      r = (r + 1) & (kRing - 1);
+      double err = 0.0;
+      RKX_HIP(hipMemcpyAsync(&err, &ref.ring->err[r].bits, sizeof(err), hipMemcpyDeviceToHost,
+                             stream));
       RKX_HIP(hipStreamSynchronize(stream));
-      host_finish(cur, dm, hc);
-      RKX_HIP(hipMemcpyAsync(cf_dev, &hc, sizeof(hc), hipMemcpyHostToDevice, stream));
-      RKX_HIP(hipMemcpyAsync(st_dev, &cur, sizeof(state), hipMemcpyHostToDevice, stream));
+      host_finish(cur, err);
+      const step_slot next{cur, 0};
+      RKX_HIP(hipMemcpyAsync(&ref.ring->slot[r], &next, sizeof(next), hipMemcpyHostToDevice,
+                             stream));
       RKX_HIP(hipStreamSynchronize(stream));
     }
   } else if (!cur.done) {
@@ -208,8 +194,9 @@ int rkx_solve_noalloc(const rkx_ode *p, const rkx_method *m, double t0, double t
     int last = -1, stalled = 0;
     for (;;) {
       for (int k = 0; k < kChunk; ++k)
-        RKX_HIP(step());
-      RKX_HIP(hipMemcpyAsync(&cur, st_dev, sizeof(state), hipMemcpyDeviceToHost, stream));
+        RKX_HIP(step(k & (kRing - 1)));
+      RKX_HIP(launch_step_flush(ref.st, 1, kChunk & (kRing - 1), stream));
+      RKX_HIP(hipMemcpyAsync(&cur, &ref.st->v, sizeof(cur), hipMemcpyDeviceToHost, stream));
       RKX_HIP(hipStreamSynchronize(stream));
       if (cur.done)
         break;

@@ -36,13 +36,19 @@ namespace rkx {
 struct pow_tables {
   double logt[128][3];            // invc, logc, logctail
   unsigned long long expt[256];   // bits of tail T_k, bits of H_k - (k << 45)
+  __host__ __device__ double log_at(int i, int c) const { return logt[i][c]; }
+  __host__ __device__ unsigned long long exp_at(int k, int c) const { return expt[2 * k + c]; }
 };
 
 __host__ __device__ inline double pow_asd(uint64_t u) { return __builtin_bit_cast(double, u); }
 __host__ __device__ inline uint64_t pow_asu(double x) { return __builtin_bit_cast(uint64_t, x); }
 
+// The functions below read the tables through log_at / exp_at of T: pow_tables
+// itself, or the step kernels' copy spread over a wavefront's lanes.
+
 // log(x) as hi + *tail for the bits ix of a normal positive x (e_pow.c log_inline)
-__host__ __device__ inline double pow_log_inline(uint64_t ix, double *tail, const pow_tables &T)
+template <class TAB>
+__host__ __device__ inline double pow_log_inline(uint64_t ix, double *tail, const TAB &T)
 {
   constexpr double Ln2hi = 0x1.62e42fefa3800p-1, Ln2lo = 0x1.ef35793c76730p-45;
   // polynomial coefficients, scaled as the evaluation below uses them
@@ -56,7 +62,7 @@ __host__ __device__ inline double pow_log_inline(uint64_t ix, double *tail, cons
   const uint64_t iz = ix - (tmp & (0xfffULL << 52));
   const double z = pow_asd(iz);
   const double kd = static_cast<double>(k);
-  const double invc = T.logt[i][0], logc = T.logt[i][1], logctail = T.logt[i][2];
+  const double invc = T.log_at(i, 0), logc = T.log_at(i, 1), logctail = T.log_at(i, 2);
   const double r = __builtin_fma(z, invc, -1.0);        // exact: 1/c has few bits
   const double t1 = __builtin_fma(kd, Ln2hi, logc);
   const double t2 = t1 + r;
@@ -77,7 +83,8 @@ __host__ __device__ inline double pow_log_inline(uint64_t ix, double *tail, cons
 }
 
 // exp(x + xtail) for |x| < 512 (e_pow.c exp_inline, sign bias 0)
-__host__ __device__ inline double pow_exp_inline(double x, double xtail, const pow_tables &T)
+template <class TAB>
+__host__ __device__ inline double pow_exp_inline(double x, double xtail, const TAB &T)
 {
   constexpr double InvLn2N = 0x1.71547652b82fep0 * 128, NegLn2hiN = -0x1.62e42fefa0000p-8,
                    NegLn2loN = -0x1.cf79abc9e3b3ap-47, Shift = 0x1.8p52;
@@ -91,10 +98,10 @@ __host__ __device__ inline double pow_exp_inline(double x, double xtail, const p
   kd -= Shift;
   double r = __builtin_fma(kd, NegLn2loN, __builtin_fma(kd, NegLn2hiN, x));
   r += xtail;
-  const uint64_t idx = 2u * (ki % 128u);
+  const int idx = static_cast<int>(ki % 128u);
   const uint64_t top = ki << 45;
-  const double tail = pow_asd(T.expt[idx]);
-  const uint64_t sbits = T.expt[idx + 1] + top;
+  const double tail = pow_asd(T.exp_at(idx, 0));
+  const uint64_t sbits = T.exp_at(idx, 1) + top;
   const double r2 = r * r;
   const double p = __builtin_fma(r2 * r2, __builtin_fma(r, C5, C4),
                                  __builtin_fma(r2, __builtin_fma(r, C3, C2), tail + r));
@@ -103,7 +110,8 @@ __host__ __device__ inline double pow_exp_inline(double x, double xtail, const p
 }
 
 // pow(x, y) for x >= 0 and 0 < y <= 1/2 (e_pow.c __pow on that domain)
-__host__ __device__ inline double libm_pow(double x, double y, const pow_tables &T)
+template <class TAB>
+__host__ __device__ inline double libm_pow(double x, double y, const TAB &T)
 {
   uint64_t ix = pow_asu(x);
   if ((ix >> 52) - 1u >= 0x7feu) {     // zero, subnormal, inf or nan

@@ -48,8 +48,8 @@
 namespace rkx {
 
 // Internal linkage on purpose: each translation unit that includes this
-// header instantiates the kernels of its own tables (rkx_kernels_sweep.hip:
-// DOPRI54 ... SSPRK3; rkx_kernels_sweep_dopri87.hip: DOPRI87) and exports
+// header instantiates the kernels of its own tables (rkx_kernels_sweep.hip,
+// rkx_kernels_sweep_verner65.hip, rkx_kernels_sweep_dopri87.hip) and exports
 // only the launch and occupancy functions declared in rkx_internal.hpp.
 namespace {
 
@@ -66,8 +66,8 @@ __device__ __forceinline__ int reflect(int k, int N)
 // GEN: ghost rows by the general reflection loop (grids too short for
 // sweep_single_reflect); otherwise by a single reflection.
 template <class P, int K, bool GEN>
-__global__ __launch_bounds__(128 * K) __attribute__((amdgpu_waves_per_eu(P::occ))) void k_sweep(const sweep_inst *__restrict__ insts,
-                                                   const int2 *__restrict__ tiles, int ntiles)
+__global__ __launch_bounds__(128 * K) __attribute__((amdgpu_waves_per_eu(P::occ))) void
+k_sweep(fused_launch<sweep_inst> a)
 {
   constexpr int s = P::s;
   constexpr int L = 64 * K;          // columns per strip
@@ -77,35 +77,30 @@ __global__ __launch_bounds__(128 * K) __attribute__((amdgpu_waves_per_eu(P::occ)
   constexpr int PF = prefetch_rows(s);         // y rows loaded ahead of stage 0
   __shared__ double xch[2][s][2][LP];
   __shared__ double red[2 * K];
-  __shared__ unsigned int zred[2 * K];
+  __shared__ step_lds head;
 
   // XCD-aware tile order: consecutive workgroups are dispatched round-robin
   // over the 8 XCDs; give each XCD a contiguous run of tiles (adjacent bands
   // of a strip share halo rows in that XCD's L2).
-  const int T = ntiles;
+  const int T = a.ntiles;
   const int b = blockIdx.x;
   const int x = b & 7, q = T >> 3, rm = T & 7;
   const int tile = x * q + min(x, rm) + (b >> 3);
   // tile -> (instance, tile within the instance); no table: one instance
-  const int2 td = tiles ? tiles[tile] : make_int2(0, tile);
-  const sweep_inst &I = insts[td.x];
-  double *const y0p = I.y0, *const y1p = I.y1;
+  const int2 td = launch_tile(a, tile);
+  const sweep_inst I = launch_inst(a, td.x);
   const int N = I.N;
   const int R = I.R, OC = I.OC;
   const int nwide = I.nwide, nbands = I.nbands;
-  state *st = I.st;
-  const step_view sv = read_step(st);
-  if (sv.done)
+  const step_now sn = step_begin(I.ref, a.r, td.y == 0, head);
+  if (sn.done)
     return;                                      // uniform over the instance's tiles
-  // uniform, said explicitly: y, y_new and every row address below stay in
-  // scalar registers
-  const int cur = __builtin_amdgcn_readfirstlane(sv.cur);
-  gconst *__restrict__ y = as_global(cur ? y1p : y0p);
-  gmut *__restrict__ yn = as_global(cur ? y0p : y1p);
+  gconst *__restrict__ y = as_global(sn.cur ? I.y1 : I.y0);
+  gmut *__restrict__ yn = as_global(sn.cur ? I.y0 : I.y1);
   const int N2 = N + N;
   const double coef = I.coef;
-  gmethod *__restrict__ mt = as_global(sv.meth);
-  const double h = sv.h;                         // this step's h (uniform)
+  gmethod *__restrict__ mt = as_global(I.ref.meth);
+  const double h = sn.h;                         // this step's h (uniform)
   const int var = (threadIdx.x >= L) ? 1 : 0;   // wave-uniform: 0 = u, 1 = v
   const int cl = threadIdx.x - var * L;         // column lane within the strip
 
@@ -378,19 +373,16 @@ __global__ __launch_bounds__(128 * K) __attribute__((amdgpu_waves_per_eu(P::occ)
     rows(std::integral_constant<int, 0>{});
   else
     rows(std::integral_constant<int, 1>{});
-  block_finish(st, qmax, zero, red, zred, static_cast<unsigned int>(I.ntiles), false);
+  step_fold(head, qmax, zero, red);
 }
 
 template <class P, int K>
-hipError_t launch_one(bool gen, const sweep_inst *insts, const int2 *tiles, int ntiles,
-                      hipStream_t stream)
+hipError_t launch_one(bool gen, const fused_launch<sweep_inst> &a, hipStream_t stream)
 {
   if (gen)
-    hipLaunchKernelGGL((k_sweep<P, K, true>), dim3(ntiles), dim3(128 * K), 0, stream, insts,
-                       tiles, ntiles);
+    hipLaunchKernelGGL((k_sweep<P, K, true>), dim3(a.ntiles), dim3(128 * K), 0, stream, a);
   else
-    hipLaunchKernelGGL((k_sweep<P, K, false>), dim3(ntiles), dim3(128 * K), 0, stream, insts,
-                       tiles, ntiles);
+    hipLaunchKernelGGL((k_sweep<P, K, false>), dim3(a.ntiles), dim3(128 * K), 0, stream, a);
   return hipGetLastError();
 }
 
@@ -403,21 +395,20 @@ constexpr int max_waves()
 }
 
 template <class P>
-hipError_t launch_pat(int K, bool gen, const sweep_inst *insts, const int2 *tiles, int ntiles,
-                      hipStream_t stream)
+hipError_t launch_pat(int K, bool gen, const fused_launch<sweep_inst> &a, hipStream_t stream)
 {
   if (K < 1 || K > max_waves<P>())
     return hipErrorInvalidConfiguration;
   switch (K) {
-  case 1: return launch_one<P, 1>(gen, insts, tiles, ntiles, stream);
-  case 2: return launch_one<P, 2>(gen, insts, tiles, ntiles, stream);
+  case 1: return launch_one<P, 1>(gen, a, stream);
+  case 2: return launch_one<P, 2>(gen, a, stream);
   case 3:
     if constexpr (max_waves<P>() >= 3)
-      return launch_one<P, 3>(gen, insts, tiles, ntiles, stream);
+      return launch_one<P, 3>(gen, a, stream);
     return hipErrorInvalidConfiguration;
   default:
     if constexpr (max_waves<P>() >= 4)
-      return launch_one<P, 4>(gen, insts, tiles, ntiles, stream);
+      return launch_one<P, 4>(gen, a, stream);
     return hipErrorInvalidConfiguration;
   }
 }
