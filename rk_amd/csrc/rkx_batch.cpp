@@ -558,7 +558,7 @@ int rkx_batch_add(rkx_batch *b, const rkx_ode *p, const rkx_method *m, double t0
   step_ring hr{};
   if (storage == RKX_STORAGE_LOW) {
     hs.ring = b->rg_dev + slot;
-    hr = make_ring(hs.v);
+    hr = make_ring(hs.v, false);
     I.ref = step_refs{b->st_dev + slot, hs.ring, hs.meth};
   }
   dev_coef hc{};

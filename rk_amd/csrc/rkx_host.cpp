@@ -177,11 +177,79 @@ void host_finish(step_vars &v, double err)
   ctrl_finish(v, need, need ? std::pow(px, py) : 0.0);
 }
 
-step_ring make_ring(const step_vars &v)
+step_ring make_ring(const step_vars &v, bool traced)
 {
   step_ring g{};
   g.slot[0].v = v;
+  g.slot[0].traced = traced;
   return g;
+}
+
+hipError_t fused_plan::launch(int r, hipStream_t stream)
+{
+  switch (kind) {
+  case kPairs:
+    return launch_lv_step(dp, s, ref, y0, y1, r, stream);
+  case kChain:
+    chain.r = r;
+    return launch_chain(pattern, chain, stream);
+  case kTile:
+    tile.r = r;
+    return launch_tile_step(pattern, shape, general, tile, stream);
+  default:
+    sweep.r = r;
+    return launch_sweep(pattern, waves, general, sweep, stream);
+  }
+}
+
+int make_fused_plan(const rkx_ode &p, const rkx_method &m, int rows, int waves,
+                    const step_refs &ref, double *y0, double *y1, fused_plan *out)
+{
+  fused_plan f;
+  f.dp = make_dev_ode(p);
+  f.ref = ref;
+  f.y0 = y0;
+  f.y1 = y1;
+  f.s = m.s;
+  f.pattern = sweep_pattern(m);
+  const bool chosen = rows <= 0 && waves <= 0;
+  if (chain_supported(f.dp, m)) {
+    f.kind = fused_plan::kChain;
+    f.chain.one = make_chain_inst(f.dp, m, ref, y0, y1);
+    f.chain.ntiles = f.chain.one.nwg;
+  } else if (pairs_supported(f.dp, m)) {
+    f.kind = fused_plan::kPairs;
+  } else {
+    sweep_cfg cfg = sweep_default_cfg(f.dp, m);
+    if (rows > 0)
+      cfg.rows = rows;
+    if (waves > 0)
+      cfg.waves = waves;
+    if (cfg.waves < 1 || cfg.waves > 4 || cfg.rows < 1 || 64 * cfg.waves <= 2 * m.s)
+      return fail(RKX_EINVAL, "tile_waves must be 1..4 (and wider than 2s), tile_rows >= 1");
+    if (sweep_resident_blocks(f.pattern, cfg.waves) < 1)
+      return fail(RKX_EINVAL, "tile_waves wider than this table's fused kernel "
+                              "(DOPRI87: at most 2)");
+    // the tile kernel moves a cell's (u, v) in one 16-byte access: a caller's
+    // buffer that is not aligned for it stays with the row sweep
+    const bool aligned = ((reinterpret_cast<uintptr_t>(y0) | reinterpret_cast<uintptr_t>(y1)) &
+                          15u) == 0;
+    f.shape = chosen && aligned ? tile_default_shape(f.dp, m) : -1;
+    if (f.shape >= 0) {
+      f.kind = fused_plan::kTile;
+      f.tile.one = make_tile_inst(f.dp, m, f.shape, ref, y0, y1);
+      f.tile.ntiles = f.tile.one.ntiles;
+      f.general = tile_small(f.shape, p.grid);
+    } else {
+      f.kind = fused_plan::kSweep;
+      f.waves = cfg.waves;
+      f.sweep.one = make_sweep_inst(f.dp, m, cfg, ref, y0, y1);
+      f.sweep.ntiles = f.sweep.one.ntiles;
+      f.general = !sweep_inst_single_reflect(f.pattern, m.s, f.sweep.one);
+    }
+  }
+  *out = f;
+  return RKX_OK;
 }
 
 // The control block of a solve: everything small that its kernels read, in
@@ -521,18 +589,16 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
   const dev_ode dp = make_dev_ode(*p);
   const int s = m->s;
   int impl = o.impl;
-  // fused forms: the row sweep for BRUSS2D, the segment kernel for the LV
+  // fused forms: the row sweep or the tile form for BRUSS2D, the segment kernel for the LV
   // chain, the per-pair kernel for LV pairs; anything else (tables without a
   // compiled pattern or stage count) runs the full-storage loop order with
   // the least traffic.  D, A, E and F run as asked on every problem.
   bool fused = impl == RKX_IMPL_PIPED || impl == RKX_IMPL_PIPEDLS;
-  const bool chain = fused && chain_supported(dp, *m);
-  const bool pairs = fused && !chain && pairs_supported(dp, *m);
-  if (fused && !chain && !pairs && !sweep_supported(dp, *m)) {
+  if (fused && !chain_supported(dp, *m) && !pairs_supported(dp, *m) &&
+      !sweep_supported(dp, *m)) {
     impl = least_traffic_form(*m);
     fused = false;
   }
-  const bool sweep = fused && !chain && !pairs;
   const bool gather = impl == RKX_IMPL_A || impl == RKX_IMPL_E || impl == RKX_IMPL_F;
   const size_t n = static_cast<size_t>(p->n);
   const size_t vec = n * sizeof(double);
@@ -590,53 +656,27 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
   hs.coef = cf_dev;
   if (fused) {
     hs.ring = ref.ring;
-    hc.ring = make_ring(hs.v);
+    hc.ring = make_ring(hs.v, trace_dev != nullptr);
   }
   premult(hc.meth, s, hs.v.h, hc.coef);
   RKX_HIP(hipMemcpyAsync(ctl_dev, &hc, sizeof(hc), hipMemcpyHostToDevice, stream));
   RKX_HIP(hipMemcpyAsync(ybuf[0], y0_dev, vec, hipMemcpyDeviceToDevice, stream));
 
-  sweep_cfg cfg{1, 1};
-  if (sweep)
-    cfg = sweep_default_cfg(dp, *m);
-  if (o.tile_rows > 0)
-    cfg.rows = o.tile_rows;
-  if (o.tile_waves > 0)
-    cfg.waves = o.tile_waves;
-  if (cfg.waves < 1 || cfg.waves > 4 || cfg.rows < 1 || 64 * cfg.waves <= 2 * s)
-    return fail(RKX_EINVAL, "rkx_solve: tile_waves must be 1..4 (and wider than 2s), "
-                            "tile_rows >= 1");
-  fused_launch<sweep_inst> sl{};
-  fused_launch<chain_inst> cl{};
-  bool gen_rows = false;   // the general ghost-row form (sweep_inst_single_reflect)
-  const int pattern = sweep_pattern(*m);
-  if (sweep && sweep_resident_blocks(pattern, cfg.waves) < 1)
-    return fail(RKX_EINVAL, "rkx_solve: tile_waves wider than this table's fused kernel "
-                            "(DOPRI87: at most 2)");
-  if (chain) {
-    cl.one = make_chain_inst(dp, *m, ref, ybuf[0], ybuf[1]);
-    cl.ntiles = cl.one.nwg;
-  } else if (sweep) {
-    sl.one = make_sweep_inst(dp, *m, cfg, ref, ybuf[0], ybuf[1]);
-    sl.ntiles = sl.one.ntiles;
-    gen_rows = !sweep_inst_single_reflect(pattern, s, sl.one);
+  if (o.tile_waves > 4)
+    return fail(RKX_EINVAL, "rkx_solve: tile_waves must be 1..4");
+  fused_plan plan;
+  if (fused) {
+    if (int rc = make_fused_plan(*p, *m, o.tile_rows, o.tile_waves, ref, ybuf[0], ybuf[1], &plan))
+      return fail(rc, std::string("rkx_solve: ") + rkx_last_error());
   }
 
   // one attempted step; r: the ring slot a fused kernel reads
   auto enqueue_step = [&](int r) -> hipError_t {
+    if (fused)
+      return plan.launch(r, stream);
     if (impl == RKX_IMPL_D)
       return launch_d_step(dp, cf_dev, s, st_dev, ybuf[0], ybuf[1], w, dy, err, stream);
-    if (gather)
-      return launch_gather_step(impl, dp, cf_dev, s, nz, st_dev, ybuf[0], ybuf[1], v, w, w1,
-                                stream);
-    if (pairs)
-      return launch_lv_step(dp, s, ref, ybuf[0], ybuf[1], r, stream);
-    if (chain) {
-      cl.r = r;
-      return launch_chain(pattern, cl, stream);
-    }
-    sl.r = r;
-    return launch_sweep(pattern, cfg.waves, gen_rows, sl, stream);
+    return launch_gather_step(impl, dp, cf_dev, s, nz, st_dev, ybuf[0], ybuf[1], v, w, w1, stream);
   };
 
   state *hs_pinned = nullptr;   // [0], [1]: snapshots of two chunks in flight
@@ -687,7 +727,7 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
       }
       host_finish(cur, step_err);
       if (fused) {
-        const step_slot next{cur, 0};
+        const step_slot next{cur, 0, 0};
         RKX_HIP(hipMemcpyAsync(&ref.ring->slot[r], &next, sizeof(next), hipMemcpyHostToDevice,
                                stream));
       } else {

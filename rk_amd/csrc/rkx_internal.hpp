@@ -89,6 +89,7 @@ constexpr int kRing = 4;
 struct alignas(64) step_slot {
   step_vars v;
   int pending;                       // the attempt from v awaits its control
+  int traced;                        // state::trace is set
 };
 struct step_ring {
   step_slot slot[kRing];
@@ -186,7 +187,7 @@ struct step_refs {
   const dev_method *meth;
 };
 // Rings of instances about to run their first step (nothing pending).
-step_ring make_ring(const step_vars &v);
+step_ring make_ring(const step_vars &v, bool traced);
 
 // Kernel launchers (rkx_kernels_*.hip).  All return hipError_t of the launch.
 hipError_t launch_eval_rng(const dev_ode &p, int i, int j, const double *y, double *f,
@@ -293,6 +294,31 @@ int resident_blocks_dopri87(int K);
 // width; 0: the strip is too wide for that table's kernel
 int sweep_resident_blocks(int pattern, int K);
 
+// One BRUSS2D instance as the tile kernel sees it.  Strips of 64 columns and
+// bands of W*C rows that overlap by their halos; the last ones end at the
+// grid's edge, so the grid's own edges cost no halo.
+struct tile_inst {
+  int N;
+  int nstrips, nbands;
+  int ntiles;            // nstrips * nbands workgroups
+  double coef;
+  double *y0, *y1;
+  step_refs ref;
+};
+// Tile shapes of the kernel: C rows in each of 8 waves of 64 columns.
+constexpr int kTileWaves = 8;
+constexpr int kTileRows[] = {2, 3, 4, 6};
+constexpr int kNumTileShapes = sizeof(kTileRows) / sizeof(kTileRows[0]);
+bool tile_supported(int pattern);            // tables of up to 8 stages
+tile_inst make_tile_inst(const dev_ode &p, const rkx_method &m, int shape, const step_refs &ref,
+                         double *y0, double *y1);
+// The shape a single grid runs in, or -1: the row sweep is the faster form.
+int tile_default_shape(const dev_ode &p, const rkx_method &m);
+// Whether some grid's last row or column lies inside a tile (see k_tile's SMALL).
+bool tile_small(int shape, int N);
+hipError_t launch_tile_step(int pattern, int shape, bool small, const fused_launch<tile_inst> &a,
+                            hipStream_t stream);
+
 // One LV chain instance as the fused chain kernel sees it (device memory).
 struct chain_inst {
   int cells;             // M
@@ -308,5 +334,26 @@ bool chain_supported(const dev_ode &p, const rkx_method &m);
 chain_inst make_chain_inst(const dev_ode &p, const rkx_method &m, const step_refs &ref,
                            double *y0, double *y1);
 hipError_t launch_chain(int pattern, const fused_launch<chain_inst> &a, hipStream_t stream);
+
+// The fused step of one instance: which kernel, and its launch.
+struct fused_plan {
+  enum kind_t { kPairs, kChain, kTile, kSweep } kind = kSweep;
+  dev_ode dp{};
+  step_refs ref{};
+  double *y0 = nullptr, *y1 = nullptr;
+  int s = 0, pattern = 0;
+  int shape = 0;           // tile
+  bool general = false;    // tile: small grid; sweep: general ghost rows
+  int waves = 0;           // sweep
+  fused_launch<chain_inst> chain{};
+  fused_launch<tile_inst> tile{};
+  fused_launch<sweep_inst> sweep{};
+  // one attempted step; r: the ring slot the kernel reads
+  hipError_t launch(int r, hipStream_t stream);
+};
+// The plan of a problem and table with a fused kernel.  rows, waves: the
+// caller's row-sweep tile (0: chosen); y0, y1: the two y buffers.
+int make_fused_plan(const rkx_ode &p, const rkx_method &m, int rows, int waves,
+                    const step_refs &ref, double *y0, double *y1, fused_plan *out);
 
 }  // namespace rkx

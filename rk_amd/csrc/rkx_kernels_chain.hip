@@ -49,6 +49,8 @@ __global__ __launch_bounds__(kCB) void k_chain(fused_launch<chain_inst> a)
   const int2 td = launch_tile(a, tile);
   const chain_inst I = launch_inst(a, td.x);
   const int M = I.cells;
+  step_coefs<P> kc;
+  kc.load(as_global(I.ref.meth));
   const step_now sn = step_begin(I.ref, a.r, td.y == 0, head);
   if (sn.done)
     return;
@@ -60,26 +62,9 @@ __global__ __launch_bounds__(kCB) void k_chain(fused_launch<chain_inst> a)
   p.d1 = I.d1;
   p.c1 = I.c1;
   const double D = I.diff;
-  gmethod *__restrict__ mt = as_global(I.ref.meth);
-  const double h = sn.h;                         // this step's h (uniform)
-
   const int t = threadIdx.x;
 
-  // h * col[i]: the premultiplied coefficients of stage i (premult's products)
-  double kv[s][s + 1];
-  static_for<s>([&](auto it) {
-    constexpr int i = decltype(it)::value;
-    static_for<s>([&](auto lt) {
-      constexpr int l = decltype(lt)::value;
-      if constexpr (l > i)
-        kv[i][l - i - 1] = nzA<P>(l, i) ? wave_uniform(h * mt->col[i][l - i - 1]) : 0.0;
-    });
-    if constexpr (P::fsal && i < s - 1)
-      kv[i][s - i - 1] = kv[i][s - i - 2];
-    else
-      kv[i][s - i - 1] = ((P::b >> i) & 1u) ? wave_uniform(h * mt->col[i][s - i - 1]) : 0.0;
-    kv[i][s - i] = ((P::e >> i) & 1u) ? wave_uniform(h * mt->col[i][s - i]) : 0.0;
-  });
+  kc.scale(sn.h);
 
   double qmax = 0.0;
   unsigned int zero = 0u;
@@ -117,31 +102,31 @@ __global__ __launch_bounds__(kCB) void k_chain(fused_launch<chain_inst> a)
       lv_pair(p, v.x, v.y, gx, gy);
       const double fx = gx + D * __builtin_fma(-2.0, v.x, l.x + r.x);
       const double fy = gy + D * __builtin_fma(-2.0, v.y, l.y + r.y);
-      const double *kc = kv[i];
+      const double *ki = kc.k[i];
       if constexpr (i == 0) {
         static_for<s>([&](auto ltg) {
           constexpr int lq = decltype(ltg)::value;
           if constexpr (lq >= 1)
-            acc[c][lq] = nzA<P>(lq, 0) ? make_double2(v.x + kc[lq - 1] * fx, v.y + kc[lq - 1] * fy)
+            acc[c][lq] = nzA<P>(lq, 0) ? make_double2(v.x + ki[lq - 1] * fx, v.y + ki[lq - 1] * fy)
                                        : v;
         });
-        acc[c][0] = make_double2(kc[s - 1] * fx, kc[s - 1] * fy);
-        acc[c][s] = make_double2(kc[s] * fx, kc[s] * fy);
+        acc[c][0] = make_double2(ki[s - 1] * fx, ki[s - 1] * fy);
+        acc[c][s] = make_double2(ki[s] * fx, ki[s] * fy);
       } else {
         static_for<s>([&](auto ltg) {
           constexpr int lq = decltype(ltg)::value;
           if constexpr (lq > i && nzA<P>(lq, i)) {
-            acc[c][lq].x += kc[lq - i - 1] * fx;
-            acc[c][lq].y += kc[lq - i - 1] * fy;
+            acc[c][lq].x += ki[lq - i - 1] * fx;
+            acc[c][lq].y += ki[lq - i - 1] * fy;
           }
         });
         if constexpr ((P::b >> i) & 1u) {
-          acc[c][0].x += kc[s - i - 1] * fx;
-          acc[c][0].y += kc[s - i - 1] * fy;
+          acc[c][0].x += ki[s - i - 1] * fx;
+          acc[c][0].y += ki[s - i - 1] * fy;
         }
         if constexpr ((P::e >> i) & 1u) {
-          acc[c][s].x += kc[s - i] * fx;
-          acc[c][s].y += kc[s - i] * fy;
+          acc[c][s].x += ki[s - i] * fx;
+          acc[c][s].y += ki[s - i] * fy;
         }
       }
       if constexpr (i == s - 1) {
@@ -161,7 +146,7 @@ __global__ __launch_bounds__(kCB) void k_chain(fused_launch<chain_inst> a)
   });
   __syncthreads();                       // the next segment reuses the edge buffers
   }
-  step_fold(head, qmax, zero, red);
+  step_fold<kCB / 64>(head, qmax, zero, red);
 }
 
 }  // namespace

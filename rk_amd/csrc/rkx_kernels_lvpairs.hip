@@ -94,7 +94,7 @@ __global__ __launch_bounds__(kPBlock) void k_lv_step(dev_ode p, step_refs R, int
     err_term(ex, yn.x, Y.x, qmax, zero);
     err_term(ey, yn.y, Y.y, qmax, zero);
   }
-  step_fold(head, qmax, zero, red);
+  step_fold<kPBlock / 64>(head, qmax, zero, red);
 }
 
 template <int S>

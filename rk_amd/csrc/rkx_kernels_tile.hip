@@ -1,0 +1,76 @@
+// Host side of the tile form of the BRUSS2D step (rkx_tile_kernel.hpp): tile
+// geometry, and the launches.
+#include "rkx_tile_kernel.hpp"
+
+namespace rkx {
+
+tile_inst make_tile_inst(const dev_ode &p, const rkx_method &m, int shape, const step_refs &ref,
+                         double *y0, double *y1)
+{
+  tile_inst I{};
+  const int s = m.s, H = kTileRows[shape] * kTileWaves;
+  // the first and the last strip lose one halo, those between lose two
+  auto pieces = [](int n, int full, int halo) {
+    const int rest = n - 2 * (full - halo);
+    return n <= full ? 1 : 2 + (rest > 0 ? (rest + full - 2 * halo - 1) / (full - 2 * halo) : 0);
+  };
+  I.N = p.N;
+  I.nstrips = pieces(p.N, 64, s);
+  I.nbands = pieces(p.N, H, s - 1);
+  I.ntiles = I.nstrips * I.nbands;
+  I.coef = p.coef;
+  I.y0 = y0;
+  I.y1 = y1;
+  I.ref = ref;
+  return I;
+}
+
+bool tile_supported(int pattern) { return pattern >= 1 && pattern <= 6; }
+
+bool tile_small(int shape, int N) { return N < 64 || N < kTileRows[shape] * kTileWaves; }
+
+// The shape with the fewest rows per wave whose workgroups all run at once,
+// one to a compute unit: a step then takes the time of one tile, which grows
+// with its rows, and a second round would double it.  Grids beyond the
+// tallest tile's one round belong to the row sweep, whose bands waste less
+// on halos.  Measured, us per step, tile against sweep: DOPRI54 N=32 9.7 /
+// 11.0, N=128 9.3 / 11.5, N=301 11.9 / 14.6, N=512 14.9 / 17.6 (tallest tile
+// in two rounds at N=717: 30.6 / 21.0); VERNER65 N=128 11.1 / 17.9, N=301
+// 13.6 / 22.4; RKF23 N=128 6.9 / 7.6, N=512 10.1 / 11.4.
+int tile_default_shape(const dev_ode &p, const rkx_method &m)
+{
+  if (!tile_supported(sweep_pattern(m)))
+    return -1;
+  int cus = 0, dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      cus < 1) {
+    (void) hipGetLastError();
+    cus = 256;
+  }
+  for (int k = 0; k < kNumTileShapes; ++k) {
+    if (kTileRows[k] * kTileWaves <= 2 * (m.s - 1) && p.N > kTileRows[k] * kTileWaves)
+      continue;                                  // no rows left between the halos
+    if (make_tile_inst(p, m, k, {}, nullptr, nullptr).ntiles <= cus)
+      return k;
+  }
+  return -1;
+}
+
+hipError_t launch_tile_step(int pattern, int shape, bool small, const fused_launch<tile_inst> &a,
+                            hipStream_t stream)
+{
+  if (a.ntiles <= 0)
+    return hipSuccess;
+  switch (pattern) {
+  case 1: return launch_tile_pat<pat_dopri54>(shape, small, a, stream);
+  case 2: return launch_tile_pat<pat_verner65>(shape, small, a, stream);
+  case 3: return launch_tile_pat<pat_rkf23>(shape, small, a, stream);
+  case 4: return launch_tile_pat<pat_heun2>(shape, small, a, stream);
+  case 5: return launch_tile_pat<pat_rk4>(shape, small, a, stream);
+  case 6: return launch_tile_pat<pat_ssprk3>(shape, small, a, stream);
+  default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace rkx

@@ -89,9 +89,7 @@ int rkx_solve_noalloc(const rkx_ode *p, const rkx_method *m, double t0, double t
   if (o.trace_cap != 0 || o.dump_path)
     return fail(RKX_EINVAL, "rkx_solve_noalloc: trace and dump output need rkx_solve");
   const dev_ode dp = make_dev_ode(*p);
-  const bool chain = chain_supported(dp, *m);
-  const bool pairs = !chain && pairs_supported(dp, *m);
-  if (!chain && !pairs && !sweep_supported(dp, *m))
+  if (!chain_supported(dp, *m) && !pairs_supported(dp, *m) && !sweep_supported(dp, *m))
     return fail(RKX_EINVAL, "rkx_solve_noalloc: no fused kernel for this problem and method "
                             "(the D form needs full storage: use rkx_solve)");
   const size_t n = static_cast<size_t>(p->n);
@@ -119,7 +117,6 @@ int rkx_solve_noalloc(const rkx_ode *p, const rkx_method *m, double t0, double t
   const step_refs ref{&hd->st, &hd->ring, &hd->meth};
   double *ybuf[2] = {y_dev, reinterpret_cast<double *>(base + kHeaderBytes)};
 
-  const int s = m->s;
   header hh{};
   fill_dev_method(*m, hh.meth);
   step_vars &v = hh.st.v;
@@ -131,46 +128,18 @@ int rkx_solve_noalloc(const rkx_ode *p, const rkx_method *m, double t0, double t
   v.ord = m->ord;
   v.done = !(t0 < te);
   hh.st.ring = ref.ring;
-  hh.ring = make_ring(v);
+  hh.ring = make_ring(v, false);
 
-  sweep_cfg cfg{1, 1};
-  const int pattern = sweep_pattern(*m);
-  bool gen_rows = false;   // the general ghost-row form (sweep_inst_single_reflect)
-  fused_launch<sweep_inst> sl{};
-  fused_launch<chain_inst> cl{};
-  if (chain) {
-    cl.one = make_chain_inst(dp, *m, ref, ybuf[0], ybuf[1]);
-    cl.ntiles = cl.one.nwg;
-  } else if (!pairs) {
-    cfg = sweep_default_cfg(dp, *m);
-    if (o.tile_rows > 0)
-      cfg.rows = o.tile_rows;
-    if (o.tile_waves > 0)
-      cfg.waves = o.tile_waves;
-    if (cfg.waves < 1 || cfg.waves > 4 || cfg.rows < 1 || 64 * cfg.waves <= 2 * s ||
-        sweep_resident_blocks(pattern, cfg.waves) < 1)
-      return fail(RKX_EINVAL, "rkx_solve_noalloc: tile_waves must fit this table's fused kernel "
-                              "(1..4, DOPRI87 1..2, wider than 2s), tile_rows >= 1");
-    sl.one = make_sweep_inst(dp, *m, cfg, ref, ybuf[0], ybuf[1]);
-    sl.ntiles = sl.one.ntiles;
-    gen_rows = !sweep_inst_single_reflect(pattern, s, sl.one);
-  }
+  fused_plan plan;
+  if (int rc = make_fused_plan(*p, *m, o.tile_rows, o.tile_waves, ref, ybuf[0], ybuf[1], &plan))
+    return fail(rc, std::string("rkx_solve_noalloc: ") + rkx_last_error());
   // everything the kernels read is written before the first launch
   if (y0_dev != y_dev)
     RKX_HIP(hipMemcpyAsync(ybuf[0], y0_dev, n * sizeof(double), hipMemcpyDeviceToDevice, stream));
   RKX_HIP(hipMemcpyAsync(hd, &hh, sizeof(hh), hipMemcpyHostToDevice, stream));
   RKX_HIP(hipStreamSynchronize(stream));
 
-  auto step = [&](int r) -> hipError_t {
-    if (pairs)
-      return launch_lv_step(dp, s, ref, ybuf[0], ybuf[1], r, stream);
-    if (chain) {
-      cl.r = r;
-      return launch_chain(pattern, cl, stream);
-    }
-    sl.r = r;
-    return launch_sweep(pattern, cfg.waves, gen_rows, sl, stream);
-  };
+  auto step = [&](int r) -> hipError_t { return plan.launch(r, stream); };
 
   const auto t_start = std::chrono::steady_clock::now();
   step_vars cur = v;
@@ -183,7 +152,7 @@ int rkx_solve_noalloc(const rkx_ode *p, const rkx_method *m, double t0, double t
                              stream));
       RKX_HIP(hipStreamSynchronize(stream));
       host_finish(cur, err);
-      const step_slot next{cur, 0};
+      const step_slot next{cur, 0, 0};
       RKX_HIP(hipMemcpyAsync(&ref.ring->slot[r], &next, sizeof(next), hipMemcpyHostToDevice,
                              stream));
       RKX_HIP(hipStreamSynchronize(stream));

@@ -107,6 +107,66 @@ __device__ __forceinline__ constexpr bool nzA(int l, int i)
   return (P::rowA[l] >> i) & 1u;
 }
 
+template <int I>
+using int_c = std::integral_constant<int, I>;
+
+// The step's premultiplied coefficients (uniform, scalar registers):
+// k[i] = h * col[i] = {hA[i+1..s-1][i], hb[i], he[i]} for the scatter of
+// stage i, the products premult forms (src/methods.c:43-58).  Only the
+// non-zero entries are formed; for a first-same-as-last table (A[s-1][j] ==
+// b[j], e.g. DOPRI54) h*A[s-1][j] and h*b[j] are the same product, so hb[j]
+// reuses the register of hA[s-1][j].  load() reads the raw columns and
+// scale(h) multiplies them: a kernel loads before it waits for its step's h,
+// so the columns' trip to memory overlaps the one of the state (1.3 us of
+// each step when it followed it).
+template <class P>
+struct step_coefs {
+  static constexpr int s = P::s;
+  double k[s][s + 1];
+  template <class F>
+  __device__ __forceinline__ void each(F &&f)
+  {
+    static_for<s>([&](auto it) {
+      constexpr int i = decltype(it)::value;
+      static_for<s + 1>([&](auto jt) {
+        constexpr int j = decltype(jt)::value;
+        if constexpr (j < s - 1 - i) {
+          if constexpr (nzA<P>(i + 1 + j, i))
+            f(it, jt);
+        } else if constexpr (j == s - 1 - i) {
+          if constexpr (((P::b >> i) & 1u) && !(P::fsal && i < s - 1))
+            f(it, jt);
+        } else if constexpr (j == s - i) {
+          if constexpr ((P::e >> i) & 1u)
+            f(it, jt);
+        }
+      });
+    });
+  }
+  __device__ __forceinline__ void load(gmethod *mt)
+  {
+    static_for<s>([&](auto it) {
+      static_for<s + 1>([&](auto jt) { k[decltype(it)::value][decltype(jt)::value] = 0.0; });
+    });
+    each([&](auto it, auto jt) {
+      constexpr int i = decltype(it)::value, j = decltype(jt)::value;
+      k[i][j] = mt->col[i][j];
+    });
+  }
+  __device__ __forceinline__ void scale(double h)
+  {
+    each([&](auto it, auto jt) {
+      constexpr int i = decltype(it)::value, j = decltype(jt)::value;
+      k[i][j] = wave_uniform(h * k[i][j]);
+    });
+    if constexpr (P::fsal)
+      static_for<s - 1>([&](auto it) {
+        constexpr int i = decltype(it)::value;
+        k[i][s - i - 1] = k[i][s - i - 2];
+      });
+  }
+};
+
 
 // Which compiled pattern a method table has (0: none -- the fused kernels do
 // not cover it and the stage kernels run instead).  Zero coefficients are

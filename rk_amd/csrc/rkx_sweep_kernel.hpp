@@ -92,6 +92,12 @@ k_sweep(fused_launch<sweep_inst> a)
   const int N = I.N;
   const int R = I.R, OC = I.OC;
   const int nwide = I.nwide, nbands = I.nbands;
+  // the table's columns are asked for before the control is waited for
+  // (13 stages' do not fit the scalar registers meanwhile)
+  constexpr bool kEarly = s <= 8;
+  step_coefs<P> kc;
+  if constexpr (kEarly)
+    kc.load(as_global(I.ref.meth));
   const step_now sn = step_begin(I.ref, a.r, td.y == 0, head);
   if (sn.done)
     return;                                      // uniform over the instance's tiles
@@ -99,7 +105,6 @@ k_sweep(fused_launch<sweep_inst> a)
   gmut *__restrict__ yn = as_global(sn.cur ? I.y0 : I.y1);
   const int N2 = N + N;
   const double coef = I.coef;
-  gmethod *__restrict__ mt = as_global(I.ref.meth);
   const double h = sn.h;                         // this step's h (uniform)
   const int var = (threadIdx.x >= L) ? 1 : 0;   // wave-uniform: 0 = u, 1 = v
   const int cl = threadIdx.x - var * L;         // column lane within the strip
@@ -194,26 +199,9 @@ k_sweep(fused_launch<sweep_inst> a)
     static_for<s + 1>([&](auto et) { acc[d][decltype(et)::value] = 0.0; });
   });
 
-  // The step's premultiplied coefficients, formed once (uniform, SGPRs):
-  // kv[i] = h * col[i] = {hA[i+1..s-1][i], hb[i], he[i]} for the scatter of
-  // stage i, the products premult forms (src/methods.c:43-58).  Only the
-  // non-zero entries are formed; for a first-same-as-last table (A[s-1][j]
-  // == b[j], e.g. DOPRI54) h*A[s-1][j] and h*b[j] are the same product, so
-  // hb[j] reuses the register of hA[s-1][j].
-  double kv[s][s + 1];
-  static_for<s>([&](auto it) {
-    constexpr int i = decltype(it)::value;
-    static_for<s>([&](auto lt) {
-      constexpr int l = decltype(lt)::value;
-      if constexpr (l > i)
-        kv[i][l - i - 1] = nzA<P>(l, i) ? wave_uniform(h * mt->col[i][l - i - 1]) : 0.0;
-    });
-    if constexpr (P::fsal && i < s - 1)
-      kv[i][s - i - 1] = kv[i][s - i - 2];
-    else
-      kv[i][s - i - 1] = ((P::b >> i) & 1u) ? wave_uniform(h * mt->col[i][s - i - 1]) : 0.0;
-    kv[i][s - i] = ((P::e >> i) & 1u) ? wave_uniform(h * mt->col[i][s - i]) : 0.0;
-  });
+  if constexpr (!kEarly)
+    kc.load(as_global(I.ref.meth));
+  kc.scale(h);
 
   double qmax = 0.0;
   unsigned int zero = 0u;
@@ -298,26 +286,26 @@ k_sweep(fused_launch<sweep_inst> a)
             const double uuv = (pt * pt) * c;
             f = (3.4 * pt - uuv) + coef * lap;
           }
-          const double *kc = kv[i];
+          const double *ki = kc.k[i];
           if constexpr (i == 0) {
             // first stage: w_l = y + hA[l][0] F, dy = hb0 F, err = he0 F
             static_for<s>([&](auto ltg) {
               constexpr int l = decltype(ltg)::value;
               if constexpr (l >= 1)
-                acc[sl][l] = nzA<P>(l, 0) ? c + kc[l - 1] * f : c;
+                acc[sl][l] = nzA<P>(l, 0) ? c + ki[l - 1] * f : c;
             });
-            acc[sl][0] = kc[s - 1] * f;
-            acc[sl][s] = kc[s] * f;
+            acc[sl][0] = ki[s - 1] * f;
+            acc[sl][s] = ki[s] * f;
           } else {
             static_for<s>([&](auto ltg) {
               constexpr int l = decltype(ltg)::value;
               if constexpr (l > i && nzA<P>(l, i))
-                acc[sl][l] += kc[l - i - 1] * f;
+                acc[sl][l] += ki[l - i - 1] * f;
             });
             if constexpr ((P::b >> i) & 1u)
-              acc[sl][0] += kc[s - i - 1] * f;
+              acc[sl][0] += ki[s - i - 1] * f;
             if constexpr ((P::e >> i) & 1u)
-              acc[sl][s] += kc[s - i] * f;
+              acc[sl][s] += ki[s - i] * f;
           }
           if constexpr (i + 1 < s)
             xch[buf ^ 1][i + 1][VAR][cl] = acc[sl][i + 1];
@@ -373,7 +361,7 @@ k_sweep(fused_launch<sweep_inst> a)
     rows(std::integral_constant<int, 0>{});
   else
     rows(std::integral_constant<int, 1>{});
-  step_fold(head, qmax, zero, red);
+  step_fold<2 * K>(head, qmax, zero, red);
 }
 
 template <class P, int K>
