@@ -1,5 +1,5 @@
-// Ensemble of independent Lotka-Volterra pairs: one thread integrates one
-// 2-component system x' = c0 x - d0 x y, y' = d1 x y - c1 y (src/problems/lv.c
+// Ensemble of independent Lotka-Volterra pairs: a lane integrates one
+// 2-component system at a time x' = c0 x - d0 x y, y' = d1 x y - c1 y (src/problems/lv.c
 // with per-system constants) over [t0, te] with its own step size and
 // accept/reject.  The arithmetic of every attempted step is that of the
 // reference's seq D (block-inline.h:253-320, tools.h:191-288) on a system of
@@ -9,6 +9,8 @@
 // every new h equals the reference's (thousands of systems step at once; no
 // host round trip).
 #include "rkx_device.hpp"
+
+#include <algorithm>
 
 namespace rkx {
 namespace {
@@ -24,35 +26,103 @@ struct lv_method {
   int s, ord;
 };
 
+// A wavefront runs as long as its slowest system, and the systems' step
+// counts differ widely (the benchmark's 262144: 148 on average, up to 567), so
+// with one system per thread more than half of all lane-steps were idle.
+// Here a wave owns every gridDim-th block of 64 systems and hands the next of
+// them to its lanes as those finish, kRefill at a time: a refill costs the
+// wave a trip to memory (about one step), idle lanes cost their share of every
+// step, and the two balance at about 7 lanes.  No counter is shared: the sum
+// over a wave's few hundred systems varies little.
+constexpr int kRefill = 8;
+
+// Keeps a uniform value in a vector register.
+__device__ __forceinline__ void in_vector(double &x) { __asm__("" : "+v"(x)); }
+
 template <int S>
-__global__ __launch_bounds__(kLvBlock) void k_lv_ensemble(int count, lv_method m,
-                                                          const double *__restrict__ prm,
-                                                          const double *__restrict__ y0,
-                                                          double *__restrict__ yout, double t0,
-                                                          double te, double tol, double h0,
-                                                          int step_limit, int *__restrict__ acc_out,
-                                                          int *__restrict__ rej_out)
+__global__ __launch_bounds__(kLvBlock) __attribute__((amdgpu_waves_per_eu(2))) void
+k_lv_ensemble(int count, lv_method m, const double *__restrict__ prm,
+              const double *__restrict__ y0, double *__restrict__ yout, double t0, double te,
+              double tol, double h0, int step_limit, int *__restrict__ acc_out,
+              int *__restrict__ rej_out)
 {
-  const int kt = blockIdx.x * kLvBlock + threadIdx.x;
-  if (kt >= count)
-    return;
-  const size_t k = static_cast<size_t>(kt);
+  __shared__ pow_tables tab;                     // lanes look up different entries
+  for (unsigned k = threadIdx.x; k < sizeof(pow_tables) / 8; k += kLvBlock)
+    reinterpret_cast<double *>(&tab)[k] = reinterpret_cast<const double *>(&dev_pow_tables)[k];
+  __syncthreads();
+
+  const int lane = threadIdx.x & 63;
+  const int nw = gridDim.x * (kLvBlock / 64);
+  const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (kLvBlock / 64) +
+                                                  static_cast<int>(threadIdx.x >> 6));
+  const int blocks = (count + 63) >> 6;
+  // this wave's systems are numbered 0 .. last-1; next: the first not handed out
+  const int last = wave < blocks ? 64 * ((blocks - wave + nw - 1) / nw) : 0;
+  int next = 0;
+  bool have = false, active = false;             // holds a system; still integrates it
+  size_t k = 0;
   dev_ode p{};
-  p.c0 = prm[4 * k + 0];
-  p.d0 = prm[4 * k + 1];
-  p.d1 = prm[4 * k + 2];
-  p.c1 = prm[4 * k + 3];
-  double y[2] = {y0[2 * k], y0[2 * k + 1]};
+  double y[2] = {0.0, 0.0};
   step_vars st{};
-  st.t = t0;
   st.te = te;
   st.tol = tol;
-  st.h = h0;
   st.ord = m.ord;
   st.step_limit = step_limit;
-  st.done = !(t0 < te);
-  int attempts = 0;
-  while (!st.done && attempts < kLvMaxAttempts) {
+  // The table: 44 coefficients for 8 stages do not fit the scalar registers
+  // beside the rest and came back from spills with two lane reads each; at
+  // one wave per SIMD vector registers are there for up to 8 stages.
+  double cA[S][S], cb[S], ce[S];
+#pragma unroll
+  for (int i = 0; i < S; ++i) {
+#pragma unroll
+    for (int l = 0; l < i; ++l)
+      cA[i][l] = m.A[i * RKX_MAX_STAGES + l];
+    cb[i] = m.b[i];
+    ce[i] = m.e[i];
+    if constexpr (S <= 8) {
+#pragma unroll
+      for (int l = 0; l < i; ++l)
+        in_vector(cA[i][l]);
+      in_vector(cb[i]);
+      in_vector(ce[i]);
+    }
+  }
+  for (;;) {
+    const unsigned long long idle = __ballot(!active);
+    const int nidle = __popcll(idle);
+    if (nidle == 64 || (nidle >= kRefill && next < last)) {
+      if (have && !active) {
+        yout[2 * k] = y[0];
+        yout[2 * k + 1] = y[1];
+        acc_out[k] = st.acc;
+        rej_out[k] = st.rej;
+        have = false;
+      }
+      if (next >= last)
+        break;                                   // nidle == 64: everything is stored
+      const int mine = next + static_cast<int>(__popcll(idle & ((1ull << lane) - 1ull)));
+      if (!active && mine < last) {
+        k = (static_cast<size_t>(mine >> 6) * nw + wave) * 64 + (mine & 63);
+        if (k < static_cast<size_t>(count)) {
+          p.c0 = prm[4 * k + 0];
+          p.d0 = prm[4 * k + 1];
+          p.d1 = prm[4 * k + 2];
+          p.c1 = prm[4 * k + 3];
+          y[0] = y0[2 * k];
+          y[1] = y0[2 * k + 1];
+          st.t = t0;
+          st.h = h0;
+          st.acc = st.rej = 0;
+          st.done = !(t0 < te);
+          have = true;
+          active = !st.done;
+        }
+      }
+      next += nidle;
+      continue;
+    }
+    if (!active)
+      continue;
     const double h = st.h;
     double w[S][2], dy[2], er[2];
     // first stage
@@ -60,31 +130,31 @@ __global__ __launch_bounds__(kLvBlock) void k_lv_ensemble(int count, lv_method m
     lv_pair(p, y[0], y[1], f0, f1);
 #pragma unroll
     for (int l = 1; l < S; ++l) {
-      const double a = h * m.A[l * RKX_MAX_STAGES];
+      const double a = h * cA[l][0];
       w[l][0] = y[0] + a * f0;
       w[l][1] = y[1] + a * f1;
     }
-    dy[0] = (h * m.b[0]) * f0;
-    dy[1] = (h * m.b[0]) * f1;
-    er[0] = (h * m.e[0]) * f0;
-    er[1] = (h * m.e[0]) * f1;
+    dy[0] = (h * cb[0]) * f0;
+    dy[1] = (h * cb[0]) * f1;
+    er[0] = (h * ce[0]) * f0;
+    er[1] = (h * ce[0]) * f1;
     // intermediate and last stages
 #pragma unroll
     for (int i = 1; i < S; ++i) {
       lv_pair(p, w[i][0], w[i][1], f0, f1);
 #pragma unroll
       for (int l = i + 1; l < S; ++l) {
-        const double a = h * m.A[l * RKX_MAX_STAGES + i];
+        const double a = h * cA[l][i];
         w[l][0] += a * f0;
         w[l][1] += a * f1;
       }
-      const double hb = h * m.b[i], he = h * m.e[i];
+      const double hb = h * cb[i], he = h * ce[i];
       dy[0] += hb * f0;
       dy[1] += hb * f1;
       er[0] += he * f0;
       er[1] += he * f1;
     }
-    double yn[2] = {y[0] + dy[0], y[1] + dy[1]};
+    const double yn[2] = {y[0] + dy[0], y[1] + dy[1]};
     double q = 0.0;
     unsigned int zero = 0u;
     err_term(er[0], yn[0], y[0], q, zero);
@@ -96,13 +166,9 @@ __global__ __launch_bounds__(kLvBlock) void k_lv_ensemble(int count, lv_method m
       y[0] = yn[0];
       y[1] = yn[1];
     }
-    ctrl_finish(st, need, need ? libm_pow(px, py, dev_pow_tables) : 0.0);
-    ++attempts;
+    ctrl_finish(st, need, need ? libm_pow(px, py, tab) : 0.0);
+    active = !st.done && st.acc + st.rej < kLvMaxAttempts;
   }
-  yout[2 * k] = y[0];
-  yout[2 * k + 1] = y[1];
-  acc_out[k] = st.acc;
-  rej_out[k] = st.rej;
 }
 
 }  // namespace
@@ -134,7 +200,14 @@ extern "C" int rkx_lv_ensemble(int count, const double *params_dev, const double
   if (!s)
     if (int rc = default_stream(&s))
       return rc;
-  const int grid = (count + kLvBlock - 1) / kLvBlock;
+  // At most one wave per SIMD; more systems than lanes take turns (see
+  // k_lv_ensemble).  One wave issues a step in 1.3 us (8 stages), two on a
+  // SIMD in about twice that: 262144 systems, VERNER65, tol 1e-8: 1.24 ms with
+  // one, 1.32 ms with two, 1.8 ms with one system per thread.
+  int cus = 0, dev = 0;
+  RKX_HIP(hipGetDevice(&dev));
+  RKX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  const int grid = std::min((count + kLvBlock - 1) / kLvBlock, cus);   // 4 waves a workgroup
 #define RKX_LV_CASE(S_)                                                                      \
   case S_:                                                                                   \
     hipLaunchKernelGGL(k_lv_ensemble<S_>, dim3(grid), dim3(kLvBlock), 0, s, count, lm,      \
