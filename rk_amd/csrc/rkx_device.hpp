@@ -369,21 +369,27 @@ struct step_lds {
 
 // The start of a fused step, called by every thread of every workgroup: the
 // pending control of the attempt before, in the first wavefront, handed to
-// the others through LDS (one barrier).  leader: the one workgroup of the
-// instance that writes the next slot and clears the accumulator of the launch
-// after next.
-__device__ inline step_now step_begin(const step_refs &R, int r, bool leader, step_lds &x)
+// the others through LDS (one barrier).  tile: the workgroup's tile within
+// the instance; tile 0 writes the next slot and clears the accumulators of
+// the launch after next.
+__device__ inline step_now step_begin(const step_refs &R, int r, int tile, step_lds &x)
 {
+  const bool leader = tile == 0;
   if (threadIdx.x < 64) {
     gslot *s = (gslot *) &R.ring->slot[r];
-    using gu64 = const __attribute__((address_space(1))) unsigned long long;
-    const unsigned long long bits = *(gu64 *) &R.ring->err[r].bits;
+    using gerr = const __attribute__((address_space(1))) double;
+    static_assert(kErrLines == 8, "half a row of lanes");
+    double err = *(gerr *) &R.ring->err[r][threadIdx.x & 7].bits;
     step_vars v = slot_vars(s);
     const int pending = s->pending, traced = s->traced;
     lane_pow_tables T;
     T.load();
     if (pending) {
-      const double err = __longlong_as_double(static_cast<long long>(bits));
+      err = fmax(err, dpp_keep<0x111>(err));
+      err = fmax(err, dpp_keep<0x112>(err));
+      err = fmax(err, dpp_keep<0x114>(err));     // lane 7: all eight
+      err = __builtin_bit_cast(
+          double, lane_pow_tables::lane_of(__builtin_bit_cast(unsigned long long, err), 7));
       if (traced && leader && threadIdx.x == 0)
         trace_attempt(R.st, v, err);
       double px = 0.0, py = 0.0;
@@ -396,16 +402,17 @@ __device__ inline step_now step_begin(const step_refs &R, int r, bool leader, st
       x.h = v.h;
       x.cur = v.cur;
       x.done = v.done;
-      x.err = &R.ring->err[(r + 1) & (kRing - 1)].bits;
+      x.err = &R.ring->err[(r + 1) & (kRing - 1)][tile & (kErrLines - 1)].bits;
       if (leader) {
         step_slot &o = R.ring->slot[(r + 1) & (kRing - 1)];
         o.v = v;
         o.pending = !v.done;
         o.traced = traced;
-        __hip_atomic_store(&R.ring->err[(r + 2) & (kRing - 1)].bits, 0ull, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
       }
     }
+    if (leader && threadIdx.x < kErrLines)
+      __hip_atomic_store(&R.ring->err[(r + 2) & (kRing - 1)][threadIdx.x].bits, 0ull,
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
   step_now n;

@@ -703,10 +703,9 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
       r = (r + 1) & (kRing - 1);
       double step_err;
       if (fused) {
-        RKX_HIP(hipMemcpyAsync(&hs_pinned->err, &ref.ring->err[r].bits, sizeof(double),
-                               hipMemcpyDeviceToHost, stream));
+        RKX_HIP(hipMemcpyAsync(&hc.ring, ref.ring, sizeof(hc.ring), hipMemcpyDeviceToHost, stream));
         RKX_HIP(hipStreamSynchronize(stream));
-        step_err = hs_pinned->err;
+        step_err = ring_err(hc.ring, r);
       } else {
         RKX_HIP(hipMemcpyAsync(hs_pinned, st_dev, sizeof(state), hipMemcpyDeviceToHost, stream));
         RKX_HIP(hipStreamSynchronize(stream));

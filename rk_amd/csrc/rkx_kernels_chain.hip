@@ -51,7 +51,7 @@ __global__ __launch_bounds__(kCB) void k_chain(fused_launch<chain_inst> a)
   const int M = I.cells;
   step_coefs<P> kc;
   kc.load(as_global(I.ref.meth));
-  const step_now sn = step_begin(I.ref, a.r, td.y == 0, head);
+  const step_now sn = step_begin(I.ref, a.r, td.y, head);
   if (sn.done)
     return;
   const double2 *__restrict__ y = reinterpret_cast<const double2 *>(sn.cur ? I.y1 : I.y0);

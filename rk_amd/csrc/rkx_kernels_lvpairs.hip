@@ -34,7 +34,7 @@ __global__ __launch_bounds__(kPBlock) void k_lv_step(dev_ode p, step_refs R, int
   __shared__ double red[kPBlock / 64];
   __shared__ step_lds head;
   __shared__ double cl[S * (S + 2)];
-  const step_now sn = step_begin(R, r, blockIdx.x == 0, head);
+  const step_now sn = step_begin(R, r, static_cast<int>(blockIdx.x), head);
   if (sn.done)
     return;                       // uniform: every block of the grid returns
   for (int k = threadIdx.x; k < S * (S + 2); k += kPBlock) {

@@ -16,7 +16,7 @@ __global__ __launch_bounds__(kFlushBlock) void k_step_flush(state *st, int n, in
   step_ring &g = *st[i].ring;
   step_slot s = g.slot[r];
   if (s.pending) {
-    const double err = __longlong_as_double(static_cast<long long>(g.err[r].bits));
+    const double err = ring_err(g, r);
     trace_attempt(st + i, s.v, err);
     double px = 0.0, py = 0.0;
     const bool need = ctrl_decide(s.v, err, px, py);
@@ -25,8 +25,8 @@ __global__ __launch_bounds__(kFlushBlock) void k_step_flush(state *st, int n, in
     s.pending = 0;
   }
   g.slot[0] = s;
-  for (int k = 0; k < kRing; ++k)
-    g.err[k].bits = 0ull;
+  for (int k = 0; k < kRing * kErrLines; ++k)
+    g.err[k / kErrLines][k % kErrLines].bits = 0ull;
 }
 
 }  // namespace

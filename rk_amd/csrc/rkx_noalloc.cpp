@@ -147,11 +147,9 @@ int rkx_solve_noalloc(const rkx_ode *p, const rkx_method *m, double t0, double t
     for (int r = 0; !cur.done;) {
       RKX_HIP(step(r));
       r = (r + 1) & (kRing - 1);
-      double err = 0.0;
-      RKX_HIP(hipMemcpyAsync(&err, &ref.ring->err[r].bits, sizeof(err), hipMemcpyDeviceToHost,
-                             stream));
+      RKX_HIP(hipMemcpyAsync(&hh.ring, ref.ring, sizeof(hh.ring), hipMemcpyDeviceToHost, stream));
       RKX_HIP(hipStreamSynchronize(stream));
-      host_finish(cur, err);
+      host_finish(cur, ring_err(hh.ring, r));
       const step_slot next{cur, 0, 0};
       RKX_HIP(hipMemcpyAsync(&ref.ring->slot[r], &next, sizeof(next), hipMemcpyHostToDevice,
                              stream));

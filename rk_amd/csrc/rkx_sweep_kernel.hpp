@@ -98,7 +98,7 @@ k_sweep(fused_launch<sweep_inst> a)
   step_coefs<P> kc;
   if constexpr (kEarly)
     kc.load(as_global(I.ref.meth));
-  const step_now sn = step_begin(I.ref, a.r, td.y == 0, head);
+  const step_now sn = step_begin(I.ref, a.r, td.y, head);
   if (sn.done)
     return;                                      // uniform over the instance's tiles
   gconst *__restrict__ y = as_global(sn.cur ? I.y1 : I.y0);

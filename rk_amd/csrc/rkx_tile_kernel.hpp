@@ -98,7 +98,7 @@ __global__ __launch_bounds__(64 * W) void k_tile(fused_launch<tile_inst> a)
     ya[0][c] = ((gcell *) I.y0)[at];
     ya[1][c] = ((gcell *) I.y1)[at];
   });
-  const step_now sn = step_begin(I.ref, a.r, td.y == 0, head);
+  const step_now sn = step_begin(I.ref, a.r, td.y, head);
   if (sn.done)
     return;                                      // uniform over the instance's tiles
   gout *__restrict__ yn = (gout *) (sn.cur ? I.y0 : I.y1);
