@@ -21,6 +21,7 @@ LIB = os.path.join(HERE, "librkx.so")
 
 SOURCES = [
     "rkx_host.cpp",
+    "rkx_pool.cpp",
     "rkx_batch.cpp",
     "rkx_methods.cpp",
     "rkx_kernels_step.hip",

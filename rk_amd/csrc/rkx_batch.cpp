@@ -41,6 +41,7 @@ struct batch_inst {
   sweep_cfg cfg{1, 1};                  // current shape (bands shortened as the batch drains)
   double *y[2] = {nullptr, nullptr};
   double *w = nullptr, *dy = nullptr, *err = nullptr;
+  std::vector<std::pair<void *, size_t>> blocks;   // what the vectors above lie in
   size_t bytes = 0;
   state snap{};
 };
@@ -82,11 +83,11 @@ struct rkx_batch {
 
 namespace {
 
+// The stream must be done with the instance.
 void free_inst(batch_inst &b)
 {
-  for (double *p : {b.y[0], b.y[1], b.w, b.dy, b.err})
-    if (p)
-      (void) hipFree(p);
+  for (const auto &q : b.blocks)
+    pool_give(q.first, q.second);
   b = batch_inst{};
 }
 
@@ -520,10 +521,12 @@ int rkx_batch_add(rkx_batch *b, const rkx_ode *p, const rkx_method *m, double t0
   fill_dev_method(*m, I.dm);
   const size_t vec = static_cast<size_t>(p->n) * sizeof(double);
   auto dalloc = [&](double **q, size_t bytes) -> int {
-    if (hipMalloc(reinterpret_cast<void **>(q), bytes) != hipSuccess) {
-      (void) hipGetLastError();
-      return fail(RKX_ENOMEM, "rkx_batch_add: device allocation failed");
-    }
+    void *p = nullptr;
+    size_t got = 0;
+    if (int rc = pool_take(&p, bytes, &got))
+      return rc;
+    I.blocks.push_back({p, got});
+    *q = static_cast<double *>(p);
     return RKX_OK;
   };
   int rc = dalloc(&I.y[0], vec);
@@ -559,7 +562,7 @@ int rkx_batch_add(rkx_batch *b, const rkx_ode *p, const rkx_method *m, double t0
   if (storage == RKX_STORAGE_LOW) {
     hs.ring = b->rg_dev + slot;
     hr = make_ring(hs.v, false);
-    I.ref = step_refs{b->st_dev + slot, hs.ring, hs.meth};
+    I.ref = step_refs{b->st_dev + slot, hs.ring, hs.meth, nullptr};
   }
   dev_coef hc{};
   premult(I.dm, m->s, hs.v.h, hc);

@@ -197,6 +197,18 @@ __device__ inline void premult_block(const dev_method &m, int s, double h, dev_c
   }
 }
 
+// The loop variables for the host's thread (one thread; see host_view).
+__device__ inline void show(host_view *w, const step_vars &v)
+{
+  __hip_atomic_store(&w->t, v.t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&w->h, v.h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&w->acc, v.acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&w->rej, v.rej, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&w->cur, v.cur, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (v.done)
+    __hip_atomic_store(&w->done, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // The trace of an attempt made from v (one thread).
 __device__ inline void trace_attempt(state *st, const step_vars &v, double err)
 {
@@ -229,6 +241,8 @@ __device__ inline bool dev_control(state *st)
   double px = 0.0, py = 0.0;
   const bool need = ctrl_decide(st->v, st->err, px, py);
   ctrl_finish(st->v, need, need ? libm_pow(px, py, dev_pow_tables) : 0.0);
+  if (st->view)
+    show(st->view, st->v);
   return true;
 }
 
@@ -395,8 +409,11 @@ __device__ inline step_now step_begin(const step_refs &R, int r, int tile, step_
       double px = 0.0, py = 0.0;
       const bool need = ctrl_decide(v, err, px, py);
       ctrl_finish(v, need, need ? libm_pow(px, py, T) : 0.0);
-      if (leader && threadIdx.x == 0)
+      if (leader && threadIdx.x == 0) {
         publish(R.st, v, err);
+        if (R.view)
+          show(R.view, v);
+      }
     }
     if (threadIdx.x == 0) {
       x.h = v.h;

@@ -134,24 +134,70 @@ double initial_h(double H, double tol, int limit, double h0)
 
 namespace {
 
-// All device memory of one solve, released on scope exit.
+// All device memory of one solve, returned to the pool on scope exit, once
+// the solve's stream (if any) is done with it.
 struct solve_mem {
-  std::vector<void *> ptrs;
+  struct held {
+    void *p;
+    size_t bytes;
+  };
+  std::vector<held> blocks;
+  hipStream_t stream = nullptr;
+  host_view *view = nullptr;         // pinned
   ~solve_mem()
   {
-    for (void *p : ptrs)
-      (void) hipFree(p);
+    const bool ok = !stream || hipStreamSynchronize(stream) == hipSuccess;
+    for (const held &b : blocks) {
+      if (ok)
+        pool_give(b.p, b.bytes);
+      else
+        (void) hipFree(b.p);
+    }
+    if (view)
+      give_view(view, ok);
   }
   int alloc(void **out, size_t bytes)
   {
-    void *p = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-      (void) hipGetLastError();
-      return fail(RKX_ENOMEM, "hipMalloc of " + std::to_string(bytes) + " bytes failed");
-    }
-    ptrs.push_back(p);
-    *out = p;
+    held b{};
+    if (int rc = pool_take(&b.p, bytes, &b.bytes))
+      return rc;
+    blocks.push_back(b);
+    *out = b.p;
     return RKX_OK;
+  }
+  // Views are a few words each; up to kViews of them are kept.
+  static constexpr size_t kViews = 64;
+  static std::mutex &view_mu()
+  {
+    static std::mutex *m = new std::mutex;
+    return *m;
+  }
+  static std::vector<host_view *> &views()
+  {
+    static auto *v = new std::vector<host_view *>;
+    return *v;
+  }
+  int take_view()
+  {
+    {
+      std::lock_guard<std::mutex> lk(view_mu());
+      if (!views().empty()) {
+        view = views().back();
+        views().pop_back();
+      }
+    }
+    if (!view)
+      RKX_HIP(hipHostMalloc(reinterpret_cast<void **>(&view), sizeof(host_view),
+                            hipHostMallocPortable));
+    return RKX_OK;
+  }
+  static void give_view(host_view *w, bool ok)
+  {
+    std::lock_guard<std::mutex> lk(view_mu());
+    if (ok && views().size() < kViews)
+      views().push_back(w);
+    else
+      (void) hipHostFree(w);
   }
 };
 
@@ -212,7 +258,6 @@ int make_fused_plan(const rkx_ode &p, const rkx_method &m, int rows, int waves,
   f.y1 = y1;
   f.s = m.s;
   f.pattern = sweep_pattern(m);
-  const bool chosen = rows <= 0 && waves <= 0;
   if (chain_supported(f.dp, m)) {
     f.kind = fused_plan::kChain;
     f.chain.one = make_chain_inst(f.dp, m, ref, y0, y1);
@@ -220,27 +265,27 @@ int make_fused_plan(const rkx_ode &p, const rkx_method &m, int rows, int waves,
   } else if (pairs_supported(f.dp, m)) {
     f.kind = fused_plan::kPairs;
   } else {
-    sweep_cfg cfg = sweep_default_cfg(f.dp, m);
-    if (rows > 0)
-      cfg.rows = rows;
-    if (waves > 0)
-      cfg.waves = waves;
-    if (cfg.waves < 1 || cfg.waves > 4 || cfg.rows < 1 || 64 * cfg.waves <= 2 * m.s)
-      return fail(RKX_EINVAL, "tile_waves must be 1..4 (and wider than 2s), tile_rows >= 1");
-    if (sweep_resident_blocks(f.pattern, cfg.waves) < 1)
-      return fail(RKX_EINVAL, "tile_waves wider than this table's fused kernel "
-                              "(DOPRI87: at most 2)");
     // the tile kernel moves a cell's (u, v) in one 16-byte access: a caller's
     // buffer that is not aligned for it stays with the row sweep
     const bool aligned = ((reinterpret_cast<uintptr_t>(y0) | reinterpret_cast<uintptr_t>(y1)) &
                           15u) == 0;
-    f.shape = chosen && aligned ? tile_default_shape(f.dp, m) : -1;
+    f.shape = rows <= 0 && waves <= 0 && aligned ? tile_default_shape(f.dp, m) : -1;
     if (f.shape >= 0) {
       f.kind = fused_plan::kTile;
       f.tile.one = make_tile_inst(f.dp, m, f.shape, ref, y0, y1);
       f.tile.ntiles = f.tile.one.ntiles;
       f.general = tile_small(f.shape, p.grid);
     } else {
+      sweep_cfg cfg = sweep_default_cfg(f.dp, m);
+      if (rows > 0)
+        cfg.rows = rows;
+      if (waves > 0)
+        cfg.waves = waves;
+      if (cfg.waves < 1 || cfg.waves > 4 || cfg.rows < 1 || 64 * cfg.waves <= 2 * m.s)
+        return fail(RKX_EINVAL, "tile_waves must be 1..4 (and wider than 2s), tile_rows >= 1");
+      if (sweep_resident_blocks(f.pattern, cfg.waves) < 1)
+        return fail(RKX_EINVAL, "tile_waves wider than this table's fused kernel "
+                                "(DOPRI87: at most 2)");
       f.kind = fused_plan::kSweep;
       f.waves = cfg.waves;
       f.sweep.one = make_sweep_inst(f.dp, m, cfg, ref, y0, y1);
@@ -288,6 +333,90 @@ struct dump_file {
 }  // namespace rkx
 
 using namespace rkx;
+
+namespace {
+
+// Keeps the GPU supplied with steps until the device's step control ends the
+// loop.  Steps past the end return at once but still cost a launch each, so
+// the host follows the solve through its view and launches no more than it
+// expects: the steps left at the current step size (most are limited by
+// stability and change little) or to the step limit, and the one launch whose
+// control ends the loop.  Long solves replay a graph of kChunk steps (1.7 us
+// of launch a step, 2.6 us launched one by one), captured while the first
+// steps run; it takes 85 us, so short solves do without.
+template <class STEP>
+int run_steps(STEP &&enqueue, const host_view &view, double te, int step_limit, hipStream_t stream)
+{
+  constexpr int kChunk = 32;          // a multiple of kRing
+  constexpr int kLow = 12;            // launches in flight below which more are made
+  constexpr int kGroup = 8;           // made at a time without the graph
+  constexpr int kGraphFrom = 160;     // expected steps worth a graph
+  const volatile host_view &w = view;
+  graph_holder gh;
+  long long launched = 0;
+  auto capture = [&]() -> int {
+    RKX_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+    hipError_t cap = hipSuccess;
+    for (int k = 0; k < kChunk && cap == hipSuccess; ++k)
+      cap = enqueue(k & (kRing - 1));
+    const hipError_t end = hipStreamEndCapture(stream, &gh.g);
+    if (cap != hipSuccess)
+      return fail(RKX_EDEVICE, std::string("kernel launch during capture failed: ") +
+                                   hipGetErrorString(cap));
+    RKX_HIP(end);
+    RKX_HIP(hipGraphInstantiate(&gh.ge, gh.g, nullptr, nullptr, 0));
+    return RKX_OK;
+  };
+  for (unsigned spin = 1;; ++spin) {
+    if (__atomic_load_n(&view.done, __ATOMIC_ACQUIRE))
+      return RKX_OK;
+    const long long made = static_cast<long long>(w.acc) + w.rej;
+    const double t = w.t, h = w.h;
+    double left = std::ceil((te - t) / h);
+    if (!(left >= 1.0))
+      left = 1.0;
+    if (step_limit > 0)
+      left = std::fmin(left, static_cast<double>(step_limit) - static_cast<double>(made));
+    const double want = std::fmin(left + 1.0, 1e9) - static_cast<double>(launched - made);
+    if (want >= 1.0 && launched - made < kLow) {
+      const bool chunks = want >= kChunk && launched % kRing == 0;
+      const bool graph = chunks && gh.ge;
+      const bool make = chunks && !gh.ge && launched > 0 && left >= kGraphFrom;
+      if (graph) {
+        RKX_HIP(hipGraphLaunch(gh.ge, stream));
+        launched += kChunk;
+      } else {
+        // twice as many before a graph is captured, to bridge that time
+        const double most = make ? 2 * kGroup : kGroup;
+        const int n = static_cast<int>(std::fmin(want, most));
+        for (int k = 0; k < n; ++k, ++launched)
+          RKX_HIP(enqueue(static_cast<int>(launched & (kRing - 1))));
+        if (make)
+          if (int rc = capture())
+            return rc;
+      }
+      spin = 0;
+      continue;
+    }
+    if (spin % 64 == 0) {
+      // every launch has run and the loop has not moved past the last but
+      // one: the device-side control is not running -- stop, do not spin
+      const hipError_t q = hipStreamQuery(stream);
+      if (q == hipSuccess) {
+        const long long now = static_cast<long long>(w.acc) + w.rej;
+        if (!__atomic_load_n(&view.done, __ATOMIC_ACQUIRE) && now + 1 < launched && now == made)
+          return fail(RKX_EDEVICE, "device step control made no progress");
+      } else if (q != hipErrorNotReady) {
+        return fail(RKX_EDEVICE, std::string("a step failed: ") + hipGetErrorString(q));
+      } else {
+        (void) hipGetLastError();
+      }
+      std::this_thread::yield();
+    }
+  }
+}
+
+}  // namespace
 
 extern "C" {
 
@@ -604,6 +733,9 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
   const size_t vec = n * sizeof(double);
 
   solve_mem mem;
+  mem.stream = stream;
+  if (int rc = mem.take_view())
+    return rc;
   double *ybuf[2] = {nullptr, nullptr};
   double *w = nullptr, *dy = nullptr, *err = nullptr, *trace_dev = nullptr;
   double *v = nullptr, *w1 = nullptr;   // gather forms: v_0..v_{s-1}; F's second w
@@ -612,7 +744,7 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
     return rc;
   state *st_dev = &ctl_dev->st;
   dev_coef *cf_dev = &ctl_dev->coef;
-  const step_refs ref{st_dev, &ctl_dev->ring, &ctl_dev->meth};
+  const step_refs ref{st_dev, &ctl_dev->ring, &ctl_dev->meth, mem.view};
   for (int b = 0; b < 2; ++b)
     if (int rc = mem.alloc(reinterpret_cast<void **>(&ybuf[b]), vec))
       return rc;
@@ -654,6 +786,8 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
   hs.s = s;
   hs.meth = &ctl_dev->meth;
   hs.coef = cf_dev;
+  hs.view = mem.view;
+  *mem.view = host_view{t0, hs.v.h, 0, 0, 0, 0};
   if (fused) {
     hs.ring = ref.ring;
     hc.ring = make_ring(hs.v, trace_dev != nullptr);
@@ -679,23 +813,17 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
     return launch_gather_step(impl, dp, cf_dev, s, nz, st_dev, ybuf[0], ybuf[1], v, w, w1, stream);
   };
 
-  state *hs_pinned = nullptr;   // [0], [1]: snapshots of two chunks in flight
-  RKX_HIP(hipHostMalloc(reinterpret_cast<void **>(&hs_pinned), 2 * sizeof(state),
-                        hipHostMallocDefault));
-  struct pinned_free {
-    state *p;
-    ~pinned_free() { (void) hipHostFree(p); }
-  } pf{hs_pinned};
-
+  // the copies above read hc, whose ring the host control below reuses
   RKX_HIP(hipStreamSynchronize(stream));
   const auto t_start = std::chrono::steady_clock::now();
+  step_vars fin = hs.v;
 
   if (hs.v.done) {
-    hs_pinned[0] = hs;
+    // nothing to integrate
   } else if (o.ctrl == RKX_CTRL_HOST) {
     // One host round trip per step: the device computes the error norm, the
     // host runs the reference's step control with the C library's pow.
-    step_vars cur = hs.v;
+    step_vars &cur = fin;
     dump_file dump;
     std::vector<double> ydump;
     for (int r = 0; !cur.done;) {
@@ -707,9 +835,9 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
         RKX_HIP(hipStreamSynchronize(stream));
         step_err = ring_err(hc.ring, r);
       } else {
-        RKX_HIP(hipMemcpyAsync(hs_pinned, st_dev, sizeof(state), hipMemcpyDeviceToHost, stream));
+        RKX_HIP(hipMemcpyAsync(&hs, st_dev, sizeof(state), hipMemcpyDeviceToHost, stream));
         RKX_HIP(hipStreamSynchronize(stream));
-        step_err = hs_pinned->err;
+        step_err = hs.err;
       }
       const int attempt = cur.acc + cur.rej;
       if (o.dump_path) {
@@ -725,86 +853,28 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
         o.trace[3 * attempt + 2] = step_err;
       }
       host_finish(cur, step_err);
+      const step_slot next{cur, 0, 0};
       if (fused) {
-        const step_slot next{cur, 0, 0};
         RKX_HIP(hipMemcpyAsync(&ref.ring->slot[r], &next, sizeof(next), hipMemcpyHostToDevice,
                                stream));
       } else {
         premult(hc.meth, s, cur.h, hc.coef);
         RKX_HIP(hipMemcpyAsync(cf_dev, &hc.coef, sizeof(hc.coef), hipMemcpyHostToDevice, stream));
-        hs_pinned->v = cur;
-        RKX_HIP(hipMemcpyAsync(st_dev, hs_pinned, sizeof(state), hipMemcpyHostToDevice, stream));
+        hs.v = cur;
+        RKX_HIP(hipMemcpyAsync(st_dev, &hs, sizeof(state), hipMemcpyHostToDevice, stream));
       }
       RKX_HIP(hipStreamSynchronize(stream));
     }
-    hs_pinned[0].v = cur;
   } else {
-    // Chunks of steps captured once as a graph.  The host keeps two chunks in
-    // flight: it enqueues chunk k+1 (and a snapshot copy of the state) before
-    // waiting on the snapshot taken after chunk k.  The snapshot copy leaves
-    // the GPU idle for about 18 us, so a solve that is still running after
-    // its first kChunkGrowAfter chunks launches the graph kChunkReps times
-    // per snapshot (a short solve keeps short chunks: after the last step
-    // every launch in flight returns at once, but still costs its launch).
-    constexpr int kChunkGrowAfter = 8, kChunkReps = 4;
-    const int chunk = fused ? 32 : 16;   // a multiple of kRing: every chunk starts at slot 0
-    graph_holder gh;
-    RKX_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-    hipError_t cap_err = hipSuccess;
-    for (int k = 0; k < chunk && cap_err == hipSuccess; ++k)
-      cap_err = enqueue_step(k & (kRing - 1));
-    hipError_t end_err = hipStreamEndCapture(stream, &gh.g);
-    if (cap_err != hipSuccess)
-      return fail(RKX_EDEVICE, std::string("kernel launch during capture failed: ") +
-                                   hipGetErrorString(cap_err));
-    RKX_HIP(end_err);
-    RKX_HIP(hipGraphInstantiate(&gh.ge, gh.g, nullptr, nullptr, 0));
-    hipEvent_t ev[2];
-    RKX_HIP(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
-    RKX_HIP(hipEventCreateWithFlags(&ev[1], hipEventDisableTiming));
-    struct ev_free {
-      hipEvent_t *e;
-      ~ev_free()
-      {
-        (void) hipEventDestroy(e[0]);
-        (void) hipEventDestroy(e[1]);
-      }
-    } evf{ev};
-    int launched = 0;
-    auto launch_chunk = [&](int slot) -> int {
-      const int reps = (launched++ < kChunkGrowAfter) ? 1 : kChunkReps;
-      for (int r = 0; r < reps; ++r)
-        RKX_HIP(hipGraphLaunch(gh.ge, stream));
-      RKX_HIP(hipMemcpyAsync(&hs_pinned[slot], st_dev, sizeof(state), hipMemcpyDeviceToHost,
-                             stream));
-      RKX_HIP(hipEventRecord(ev[slot], stream));
-      return RKX_OK;
-    };
-    if (int rc = launch_chunk(0))
+    if (int rc = run_steps(enqueue_step, *mem.view, te, o.step_limit, stream))
       return rc;
-    int last_attempts = -1, stalled = 0;
-    for (int k = 0;; ++k) {
-      const int a = k & 1, b = a ^ 1;
-      if (int rc = launch_chunk(b))
-        return rc;
-      RKX_HIP(hipEventSynchronize(ev[a]));
-      if (hs_pinned[a].v.done)
-        break;
-      // every chunk must advance the attempt counter; a chunk that does not
-      // means the device-side step control is not running -- stop, do not spin
-      const int att = hs_pinned[a].v.acc + hs_pinned[a].v.rej;
-      stalled = (att == last_attempts) ? stalled + 1 : 0;
-      last_attempts = att;
-      if (stalled >= 3) {
-        (void) hipStreamSynchronize(stream);
-        return fail(RKX_EDEVICE, "device step control made no progress");
-      }
-    }
-    RKX_HIP(hipStreamSynchronize(stream));
-    RKX_HIP(hipMemcpy(&hs_pinned[0], st_dev, sizeof(state), hipMemcpyDeviceToHost));
+    fin.t = mem.view->t;
+    fin.h = mem.view->h;
+    fin.acc = mem.view->acc;
+    fin.rej = mem.view->rej;
+    fin.cur = mem.view->cur;
   }
   const auto t_end = std::chrono::steady_clock::now();
-  const step_vars fin = hs_pinned[0].v;
   RKX_HIP(hipMemcpyAsync(y_dev, ybuf[fin.cur], vec, hipMemcpyDeviceToDevice, stream));
   if (o.trace_cap > 0 && o.ctrl != RKX_CTRL_HOST) {
     const int ntr = std::min(o.trace_cap, fin.acc + fin.rej);

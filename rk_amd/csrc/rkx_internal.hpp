@@ -114,6 +114,16 @@ __host__ __device__ inline double ring_err(const step_ring &g, int r)
 
 struct state;
 
+// A solve's loop variables in pinned host memory, where its thread watches
+// them while it keeps the GPU supplied with steps: written by the step
+// control of every step (a posted write, no copy and no wait on the GPU's
+// side; a copy of the state after every chunk of steps left the GPU idle for
+// 18 us).  done is written last, after the others are visible.
+struct host_view {
+  double t, h;
+  int acc, rej, cur, done;
+};
+
 // Integration state of one solve, resident in device memory.  Written only by
 // the step control (the last workgroup of a full-storage step, the first
 // workgroup of a fused one, or the host).
@@ -130,6 +140,7 @@ struct alignas(64) state {
   const dev_method *meth;            // raw coefficients for the premultiplication
   dev_coef *coef;                    // premultiplied coefficients of the next step
   step_ring *ring;                   // fused kernels (nullptr: full storage)
+  host_view *view;                   // full-storage forms: as step_refs::view
 };
 
 // premult of the raw table by h (identical on host and device)
@@ -194,11 +205,17 @@ int default_stream(hipStream_t *out);
 // the step control on the host: ctrl_decide/ctrl_finish with the C library's pow
 void host_finish(step_vars &v, double err);
 
+// Device blocks kept between solves (rkx_pool.cpp): take a block of at least
+// `bytes` (its size in *got), give it back once no stream uses it.
+int pool_take(void **out, size_t bytes, size_t *got);
+void pool_give(void *p, size_t bytes);
+
 // What a fused kernel is given of an instance's device-side step state.
 struct step_refs {
   state *st;             // published loop variables, trace buffer
   step_ring *ring;
   const dev_method *meth;
+  host_view *view;       // nullptr: nobody watches
 };
 // Rings of instances about to run their first step (nothing pending).
 step_ring make_ring(const step_vars &v, bool traced);

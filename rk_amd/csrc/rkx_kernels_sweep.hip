@@ -10,7 +10,7 @@ namespace rkx {
 
 namespace {
 
-int resident_blocks(int pattern, int K)
+int query_resident_blocks(int pattern, int K)
 {
   switch (pattern) {
   case 1: return blocks_per_cu_k<pat_dopri54>(K);
@@ -22,6 +22,22 @@ int resident_blocks(int pattern, int K)
   case 7: return resident_blocks_dopri87(K);
   default: return 0;
   }
+}
+
+// A property of the built kernels, asked of the runtime once each (a solve's
+// default tile would otherwise ask for every strip width).
+int resident_blocks(int pattern, int K)
+{
+  constexpr int kPat = 8, kWidth = 5;
+  static std::atomic<int> known[kPat][kWidth];   // 1 + the answer; 0: not asked yet
+  if (pattern < 0 || pattern >= kPat || K < 0 || K >= kWidth)
+    return 0;
+  int v = known[pattern][K].load(std::memory_order_relaxed);
+  if (v == 0) {
+    v = 1 + query_resident_blocks(pattern, K);
+    known[pattern][K].store(v, std::memory_order_relaxed);
+  }
+  return v - 1;
 }
 
 }  // namespace

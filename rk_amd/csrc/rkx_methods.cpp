@@ -149,10 +149,23 @@ extern "C" int rkx_method_get(const char *name, rkx_method *m)
 {
   if (!name || !m)
     return rkx::fail(RKX_EINVAL, "rkx_method_get: null argument");
-  for (const auto &t : kTables)
-    if (std::strcmp(t.name, name) == 0) {
-      if (!parse_table(t, m))
+  // every table, parsed once
+  constexpr size_t n = sizeof(kTables) / sizeof(kTables[0]);
+  struct parsed {
+    rkx_method m[n];
+    bool ok[n];
+    parsed()
+    {
+      for (size_t i = 0; i < n; ++i)
+        ok[i] = parse_table(kTables[i], &m[i]);
+    }
+  };
+  static const parsed tables;
+  for (size_t i = 0; i < n; ++i)
+    if (std::strcmp(kTables[i].name, name) == 0) {
+      if (!tables.ok[i])
         return rkx::fail(RKX_EINVAL, "rkx_method_get: malformed table");
+      *m = tables.m[i];
       return RKX_OK;
     }
   return rkx::fail(RKX_EINVAL, std::string("rkx_method_get: unknown method ") + name);

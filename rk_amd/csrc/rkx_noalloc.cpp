@@ -114,7 +114,7 @@ int rkx_solve_noalloc(const rkx_ode *p, const rkx_method *m, double t0, double t
   };
   static_assert(sizeof(header) <= kHeaderBytes, "scratch header too small");
   header *hd = reinterpret_cast<header *>(base);
-  const step_refs ref{&hd->st, &hd->ring, &hd->meth};
+  const step_refs ref{&hd->st, &hd->ring, &hd->meth, nullptr};
   double *ybuf[2] = {y_dev, reinterpret_cast<double *>(base + kHeaderBytes)};
 
   header hh{};
