@@ -242,6 +242,9 @@ hipError_t fused_plan::launch(int r, hipStream_t stream)
   case kTile:
     tile.r = r;
     return launch_tile_step(pattern, shape, general, tile, stream);
+  case kGroups:
+    groups.r = r;
+    return launch_d_groups(groups, stream);
   default:
     sweep.r = r;
     return launch_sweep(pattern, waves, general, sweep, stream);
@@ -636,8 +639,14 @@ int rkx_eval_comp_host(const rkx_ode *p, int i, double t, const double *y, doubl
 // and E gather each stage from the stage derivatives (A skipping the zero
 // entries of the table), F fuses each RHS with the next stage's gather.  All
 // give the same results bitwise.  Counts: reads + writes of n doubles.
-static int least_traffic_form(const rkx_method &m)
+//
+// On BRUSS2D, D runs up to four stages to a kernel (rkx_kernels_dgroup.hip)
+// and moves the fewest vectors for every table: 13 for 7 stages against F's
+// 49 (N = 2000: 250 us a step against 588).
+static int least_traffic_form(const rkx_ode &p, const rkx_method &m)
 {
+  if (p.kind == RKX_BRUSS2D)
+    return RKX_IMPL_D;
   const int s = m.s;
   int d = (s + 2) + 5;                                   // first and last stage
   for (int i = 1; i < s - 1; ++i)
@@ -677,7 +686,7 @@ size_t rkx_solve_footprint(const rkx_ode *p, const rkx_method *m, int impl)
       sweep_supported(dp, *m) || chain_supported(dp, *m) || pairs_supported(dp, *m);
   const size_t s = static_cast<size_t>(m->s);
   if ((impl == RKX_IMPL_PIPED || impl == RKX_IMPL_PIPEDLS) && !fused)
-    impl = least_traffic_form(*m);
+    impl = least_traffic_form(*p, *m);
   if (impl == RKX_IMPL_A || impl == RKX_IMPL_E)
     return (2 + s + 1) * vec + fixed;            // y x2, v_0..v_{s-1}, w
   if (impl == RKX_IMPL_F)
@@ -725,10 +734,14 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
   bool fused = impl == RKX_IMPL_PIPED || impl == RKX_IMPL_PIPEDLS;
   if (fused && !chain_supported(dp, *m) && !pairs_supported(dp, *m) &&
       !sweep_supported(dp, *m)) {
-    impl = least_traffic_form(*m);
+    impl = least_traffic_form(*p, *m);
     fused = false;
   }
   const bool gather = impl == RKX_IMPL_A || impl == RKX_IMPL_E || impl == RKX_IMPL_F;
+  // D on BRUSS2D runs its stages in groups; these and the fused forms start
+  // each step with the control of the one before (step_ring)
+  const bool grouped = impl == RKX_IMPL_D && dp.kind == RKX_BRUSS2D;
+  const bool ringed = fused || grouped;
   const size_t n = static_cast<size_t>(p->n);
   const size_t vec = n * sizeof(double);
 
@@ -788,7 +801,7 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
   hs.coef = cf_dev;
   hs.view = mem.view;
   *mem.view = host_view{t0, hs.v.h, 0, 0, 0, 0};
-  if (fused) {
+  if (ringed) {
     hs.ring = ref.ring;
     hc.ring = make_ring(hs.v, trace_dev != nullptr);
   }
@@ -802,11 +815,15 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
   if (fused) {
     if (int rc = make_fused_plan(*p, *m, o.tile_rows, o.tile_waves, ref, ybuf[0], ybuf[1], &plan))
       return fail(rc, std::string("rkx_solve: ") + rkx_last_error());
+  } else if (grouped) {
+    plan.kind = fused_plan::kGroups;
+    plan.groups = stage_group{dp.N,    s,       0, 0, 0,  0,   0,  dp.coef,
+                              ybuf[0], ybuf[1], w, dy, err, ref};
   }
 
   // one attempted step; r: the ring slot a fused kernel reads
   auto enqueue_step = [&](int r) -> hipError_t {
-    if (fused)
+    if (ringed)
       return plan.launch(r, stream);
     if (impl == RKX_IMPL_D)
       return launch_d_step(dp, cf_dev, s, st_dev, ybuf[0], ybuf[1], w, dy, err, stream);
@@ -830,7 +847,7 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
       RKX_HIP(enqueue_step(r));
       r = (r + 1) & (kRing - 1);
       double step_err;
-      if (fused) {
+      if (ringed) {
         RKX_HIP(hipMemcpyAsync(&hc.ring, ref.ring, sizeof(hc.ring), hipMemcpyDeviceToHost, stream));
         RKX_HIP(hipStreamSynchronize(stream));
         step_err = ring_err(hc.ring, r);
@@ -854,7 +871,7 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
       }
       host_finish(cur, step_err);
       const step_slot next{cur, 0, 0};
-      if (fused) {
+      if (ringed) {
         RKX_HIP(hipMemcpyAsync(&ref.ring->slot[r], &next, sizeof(next), hipMemcpyHostToDevice,
                                stream));
       } else {

@@ -350,6 +350,29 @@ bool tile_small(int shape, int N);
 hipError_t launch_tile_step(int pattern, int shape, bool small, const fused_launch<tile_inst> &a,
                             hipStream_t stream);
 
+// Pieces of n rows or columns in tiles of `full` of them with a halo on either
+// inner side: the first and the last piece lose one halo, those between two.
+inline int tile_pieces(int n, int full, int halo)
+{
+  const int rest = n - 2 * (full - halo);
+  return n <= full ? 1 : 2 + (rest > 0 ? (rest + full - 2 * halo - 1) / (full - 2 * halo) : 0);
+}
+
+// The D form of a BRUSS2D step, stages in groups (rkx_kernels_dgroup.hip).
+struct stage_group {
+  int N, s;
+  int i0;                // the launch's first stage
+  int nstrips, nbands, ntiles;
+  int r;                 // ring slot, the same for every kernel of a step
+  double coef;
+  double *y0, *y1;
+  double *w, *dy, *err;  // w_1..w_{s-1} one after another
+  step_refs ref;
+};
+constexpr int kGroupBlocks = 512;   // two workgroups on a compute unit
+// all of a step's kernels; a: without i0 and the tile counts
+hipError_t launch_d_groups(stage_group a, hipStream_t stream);
+
 // One LV chain instance as the fused chain kernel sees it (device memory).
 struct chain_inst {
   int cells;             // M
@@ -366,9 +389,10 @@ chain_inst make_chain_inst(const dev_ode &p, const rkx_method &m, const step_ref
                            double *y0, double *y1);
 hipError_t launch_chain(int pattern, const fused_launch<chain_inst> &a, hipStream_t stream);
 
-// The fused step of one instance: which kernel, and its launch.
+// The step of one instance with a step ring: which kernel (kernels, for the D
+// form in groups of stages), and its launch.
 struct fused_plan {
-  enum kind_t { kPairs, kChain, kTile, kSweep } kind = kSweep;
+  enum kind_t { kPairs, kChain, kTile, kSweep, kGroups } kind = kSweep;
   dev_ode dp{};
   step_refs ref{};
   double *y0 = nullptr, *y1 = nullptr;
@@ -379,6 +403,7 @@ struct fused_plan {
   fused_launch<chain_inst> chain{};
   fused_launch<tile_inst> tile{};
   fused_launch<sweep_inst> sweep{};
+  stage_group groups{};    // the D form of BRUSS2D
   // one attempted step; r: the ring slot the kernel reads
   hipError_t launch(int r, hipStream_t stream);
 };

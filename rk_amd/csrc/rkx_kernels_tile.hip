@@ -9,14 +9,9 @@ tile_inst make_tile_inst(const dev_ode &p, const rkx_method &m, int shape, const
 {
   tile_inst I{};
   const int s = m.s, H = kTileRows[shape] * kTileWaves;
-  // the first and the last strip lose one halo, those between lose two
-  auto pieces = [](int n, int full, int halo) {
-    const int rest = n - 2 * (full - halo);
-    return n <= full ? 1 : 2 + (rest > 0 ? (rest + full - 2 * halo - 1) / (full - 2 * halo) : 0);
-  };
   I.N = p.N;
-  I.nstrips = pieces(p.N, 64, s);
-  I.nbands = pieces(p.N, H, s - 1);
+  I.nstrips = tile_pieces(p.N, 64, s);
+  I.nbands = tile_pieces(p.N, H, s - 1);
   I.ntiles = I.nstrips * I.nbands;
   I.coef = p.coef;
   I.y0 = y0;

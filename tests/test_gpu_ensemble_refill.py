@@ -4,6 +4,7 @@ enough for one system per lane: bitwise the same results and counts.  Ragged
 counts, an empty interval, a step limit, and every stage count."""
 import numpy as np
 import pytest
+import torch  # before the library: both load the HIP runtime
 
 pytestmark = pytest.mark.gpu
 

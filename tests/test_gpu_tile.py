@@ -5,6 +5,7 @@ or column around each tile height and strip width, one size per tile shape
 that the default rule picks, and the last sizes before the row sweep."""
 import numpy as np
 import pytest
+import torch  # before the library: both load the HIP runtime
 
 pytestmark = pytest.mark.gpu
 
@@ -14,7 +15,6 @@ SIZES = [2, 3, 7, 15, 16, 17, 24, 31, 32, 33, 47, 48, 49, 57, 58, 63, 64, 65, 11
 
 
 def run(n, meth, impl, **kw):
-    import torch
     import rk_amd
     p = rk_amd.Bruss2D(n)
     y0 = torch.from_numpy(p.ode_start_seeded(5, n, 0.01)).cuda()
@@ -46,7 +46,6 @@ def test_tile_host_control_equals_device_control():
 def test_tile_zero_divisor_and_overflow():
     """Zero components raise the error sentinel, and a step far too long
     overflows: the tile form gives the D form's values there too."""
-    import torch
     import rk_amd
     for n in (4, 40, 70, 130):
         for h0, fill in ((1e-3, 0.0), (1e60, 1.0), (1e200, 3.0)):
