@@ -65,6 +65,8 @@ CFLAGS = [
     "-O3", "-fPIC", "-std=c++17", "--offload-arch=" + ARCH,
     "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # leading scalar kernel arguments arrive in registers (see k_tile)
+    "-mllvm", "-amdgpu-kernarg-preload-count=16",
     "-Wall", "-Wno-unused-function", "-Wno-unused-command-line-argument",
     "-I" + os.path.join(REPO, "include"),
 ]

@@ -240,8 +240,7 @@ hipError_t fused_plan::launch(int r, hipStream_t stream)
     chain.r = r;
     return launch_chain(pattern, chain, stream);
   case kTile:
-    tile.r = r;
-    return launch_tile_step(pattern, shape, general, tile, stream);
+    return launch_tile_step(pattern, shape, tile, r, stream);
   case kGroups:
     groups.r = r;
     return launch_d_groups(groups, stream);
@@ -275,9 +274,7 @@ int make_fused_plan(const rkx_ode &p, const rkx_method &m, int rows, int waves,
     f.shape = rows <= 0 && waves <= 0 && aligned ? tile_default_shape(f.dp, m) : -1;
     if (f.shape >= 0) {
       f.kind = fused_plan::kTile;
-      f.tile.one = make_tile_inst(f.dp, m, f.shape, ref, y0, y1);
-      f.tile.ntiles = f.tile.one.ntiles;
-      f.general = tile_small(f.shape, p.grid);
+      f.tile = make_tile_inst(f.dp, m, f.shape, ref, y0, y1);
     } else {
       sweep_cfg cfg = sweep_default_cfg(f.dp, m);
       if (rows > 0)

@@ -345,10 +345,7 @@ tile_inst make_tile_inst(const dev_ode &p, const rkx_method &m, int shape, const
                          double *y0, double *y1);
 // The shape a single grid runs in, or -1: the row sweep is the faster form.
 int tile_default_shape(const dev_ode &p, const rkx_method &m);
-// Whether some grid's last row or column lies inside a tile (see k_tile's SMALL).
-bool tile_small(int shape, int N);
-hipError_t launch_tile_step(int pattern, int shape, bool small, const fused_launch<tile_inst> &a,
-                            hipStream_t stream);
+hipError_t launch_tile_step(int pattern, int shape, const tile_inst &I, int r, hipStream_t stream);
 
 // Pieces of n rows or columns in tiles of `full` of them with a halo on either
 // inner side: the first and the last piece lose one halo, those between two.
@@ -398,10 +395,10 @@ struct fused_plan {
   double *y0 = nullptr, *y1 = nullptr;
   int s = 0, pattern = 0;
   int shape = 0;           // tile
-  bool general = false;    // tile: small grid; sweep: general ghost rows
+  bool general = false;    // sweep: general ghost rows
   int waves = 0;           // sweep
   fused_launch<chain_inst> chain{};
-  fused_launch<tile_inst> tile{};
+  tile_inst tile{};
   fused_launch<sweep_inst> sweep{};
   stage_group groups{};    // the D form of BRUSS2D
   // one attempted step; r: the ring slot the kernel reads

@@ -4,6 +4,13 @@
 
 namespace rkx {
 
+namespace {
+
+// Whether the grid's last row or column may lie anywhere in a tile.
+bool tile_small(int shape, int N) { return N < 64 || N < kTileRows[shape] * kTileWaves; }
+
+}  // namespace
+
 tile_inst make_tile_inst(const dev_ode &p, const rkx_method &m, int shape, const step_refs &ref,
                          double *y0, double *y1)
 {
@@ -21,8 +28,6 @@ tile_inst make_tile_inst(const dev_ode &p, const rkx_method &m, int shape, const
 }
 
 bool tile_supported(int pattern) { return pattern >= 1 && pattern <= 6; }
-
-bool tile_small(int shape, int N) { return N < 64 || N < kTileRows[shape] * kTileWaves; }
 
 // The shape with the fewest rows per wave whose workgroups all run at once,
 // one to a compute unit: a step then takes the time of one tile, which grows
@@ -52,18 +57,16 @@ int tile_default_shape(const dev_ode &p, const rkx_method &m)
   return -1;
 }
 
-hipError_t launch_tile_step(int pattern, int shape, bool small, const fused_launch<tile_inst> &a,
-                            hipStream_t stream)
+hipError_t launch_tile_step(int pattern, int shape, const tile_inst &I, int r, hipStream_t stream)
 {
-  if (a.ntiles <= 0)
-    return hipSuccess;
+  const bool small = tile_small(shape, I.N);
   switch (pattern) {
-  case 1: return launch_tile_pat<pat_dopri54>(shape, small, a, stream);
-  case 2: return launch_tile_pat<pat_verner65>(shape, small, a, stream);
-  case 3: return launch_tile_pat<pat_rkf23>(shape, small, a, stream);
-  case 4: return launch_tile_pat<pat_heun2>(shape, small, a, stream);
-  case 5: return launch_tile_pat<pat_rk4>(shape, small, a, stream);
-  case 6: return launch_tile_pat<pat_ssprk3>(shape, small, a, stream);
+  case 1: return launch_tile_pat<pat_dopri54>(shape, small, I, r, stream);
+  case 2: return launch_tile_pat<pat_verner65>(shape, small, I, r, stream);
+  case 3: return launch_tile_pat<pat_rkf23>(shape, small, I, r, stream);
+  case 4: return launch_tile_pat<pat_heun2>(shape, small, I, r, stream);
+  case 5: return launch_tile_pat<pat_rk4>(shape, small, I, r, stream);
+  case 6: return launch_tile_pat<pat_ssprk3>(shape, small, I, r, stream);
   default: return hipErrorInvalidValue;
   }
 }

@@ -47,8 +47,15 @@ __device__ __forceinline__ double from_right(double v) { return wave_shift<0x130
 
 // SMALL: grids narrower or shorter than a tile, whose last row and column may
 // lie anywhere in it.
+//
+// The arguments are scalars, the ones the first loads need in front: the
+// hardware hands a kernel its leading scalar arguments in registers
+// (build.py asks for 16), so those loads do not wait for a trip to the
+// argument block first.
 template <class P, int C, int W, bool SMALL>
-__global__ __launch_bounds__(64 * W) void k_tile(fused_launch<tile_inst> a)
+__global__ __launch_bounds__(64 * W) void
+k_tile(step_ring *ring, const dev_method *meth, double *y0, double *y1, int r, int ntiles, int N,
+       int nbands, int nstrips, double coef, state *st, host_view *view)
 {
   constexpr int s = P::s;
   constexpr int H = W * C;
@@ -56,25 +63,24 @@ __global__ __launch_bounds__(64 * W) void k_tile(fused_launch<tile_inst> a)
   __shared__ double red[W];
   __shared__ step_lds head;
 
-  // XCD-aware tile order, as in the row sweep
-  const int T = a.ntiles;
+  // XCD-aware tile order, as in the row sweep (N = 512: 11.7 us per step, and
+  // 12.6 with the tiles in grid order)
   const int b = blockIdx.x;
-  const int x = b & 7, q = T >> 3, rm = T & 7;
-  const int2 td = launch_tile(a, x * q + min(x, rm) + (b >> 3));
-  const tile_inst I = launch_inst(a, td.x);
-  const int N = I.N;
+  const int x = b & 7, q = ntiles >> 3, rm = ntiles & 7;
+  const int tile = x * q + min(x, rm) + (b >> 3);
+  const int strip = tile / nbands, band = tile - strip * nbands;
+  const step_refs ref{st, ring, meth, view};
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
-  const int strip = td.y / I.nbands, band = td.y - strip * I.nbands;
   // columns [c0, c1) and rows [r0, r1) of y_new; the tile starts at (tr, tc)
   constexpr int SC = 64 - 2 * s, SR = H - 2 * (s - 1);
   const int tc = SMALL ? 0 : min(strip * SC, N - 64);
   const int c0 = strip == 0 ? 0 : strip * SC + s;
-  const int c1 = strip == I.nstrips - 1 ? N : strip * SC + 64 - s;
+  const int c1 = strip == nstrips - 1 ? N : strip * SC + 64 - s;
   const int tr = N < H ? 0 : min(band * SR, N - H);
   const int r0 = band == 0 ? 0 : band * SR + (s - 1);
-  const int r1 = band == I.nbands - 1 ? N : band * SR + H - (s - 1);
+  const int r1 = band == nbands - 1 ? N : band * SR + H - (s - 1);
   const int col = tc + lane;
   const int row = tr + wv * C;                   // the wave's first row
   const bool left = col == 0, right = col == N - 1;
@@ -87,7 +93,7 @@ __global__ __launch_bounds__(64 * W) void k_tile(fused_launch<tile_inst> a)
   using gcell = const __attribute__((address_space(1))) cell2;
   using gout = __attribute__((address_space(1))) cell2;
   step_coefs<P> kc;
-  kc.load(as_global(I.ref.meth));
+  kc.load(as_global(meth));
   const int ccol = SMALL ? min(col, N - 1) : col;
   cell2 ya[2][C + 2];
   static_for<C + 2>([&](auto ct) {
@@ -95,14 +101,13 @@ __global__ __launch_bounds__(64 * W) void k_tile(fused_launch<tile_inst> a)
     const int k = max(0, min(row + c - 1, N - 1));
     const unsigned at = static_cast<unsigned>(k) * static_cast<unsigned>(N) +
                         static_cast<unsigned>(ccol);
-    ya[0][c] = ((gcell *) I.y0)[at];
-    ya[1][c] = ((gcell *) I.y1)[at];
+    ya[0][c] = ((gcell *) y0)[at];
+    ya[1][c] = ((gcell *) y1)[at];
   });
-  const step_now sn = step_begin(I.ref, a.r, td.y, head);
+  const step_now sn = step_begin(ref, r, tile, head);
   if (sn.done)
     return;                                      // uniform over the instance's tiles
-  gout *__restrict__ yn = (gout *) (sn.cur ? I.y0 : I.y1);
-  const double coef = I.coef;
+  gout *__restrict__ yn = (gout *) (sn.cur ? y0 : y1);
   double yu[C + 2], yv[C + 2];
   static_for<C + 2>([&](auto ct) {
     constexpr int c = decltype(ct)::value;
@@ -242,26 +247,28 @@ __global__ __launch_bounds__(64 * W) void k_tile(fused_launch<tile_inst> a)
 }
 
 template <class P, int C>
-hipError_t launch_tile_shape(bool small, const fused_launch<tile_inst> &a, hipStream_t stream)
+hipError_t launch_tile_shape(bool small, const tile_inst &I, int r, hipStream_t stream)
 {
   constexpr int W = kTileWaves;
+  const dim3 g(I.ntiles), b(64 * W);
   if (small)
-    hipLaunchKernelGGL((k_tile<P, C, W, true>), dim3(a.ntiles), dim3(64 * W), 0, stream, a);
+    hipLaunchKernelGGL((k_tile<P, C, W, true>), g, b, 0, stream, I.ref.ring, I.ref.meth, I.y0,
+                       I.y1, r, I.ntiles, I.N, I.nbands, I.nstrips, I.coef, I.ref.st, I.ref.view);
   else
-    hipLaunchKernelGGL((k_tile<P, C, W, false>), dim3(a.ntiles), dim3(64 * W), 0, stream, a);
+    hipLaunchKernelGGL((k_tile<P, C, W, false>), g, b, 0, stream, I.ref.ring, I.ref.meth, I.y0,
+                       I.y1, r, I.ntiles, I.N, I.nbands, I.nstrips, I.coef, I.ref.st, I.ref.view);
   return hipGetLastError();
 }
 
 template <class P>
-hipError_t launch_tile_pat(int shape, bool small, const fused_launch<tile_inst> &a,
-                           hipStream_t stream)
+hipError_t launch_tile_pat(int shape, bool small, const tile_inst &I, int r, hipStream_t stream)
 {
   static_assert(kNumTileShapes == 4, "one case per shape");
   switch (shape) {
-  case 0: return launch_tile_shape<P, kTileRows[0]>(small, a, stream);
-  case 1: return launch_tile_shape<P, kTileRows[1]>(small, a, stream);
-  case 2: return launch_tile_shape<P, kTileRows[2]>(small, a, stream);
-  case 3: return launch_tile_shape<P, kTileRows[3]>(small, a, stream);
+  case 0: return launch_tile_shape<P, kTileRows[0]>(small, I, r, stream);
+  case 1: return launch_tile_shape<P, kTileRows[1]>(small, I, r, stream);
+  case 2: return launch_tile_shape<P, kTileRows[2]>(small, I, r, stream);
+  case 3: return launch_tile_shape<P, kTileRows[3]>(small, I, r, stream);
   default: return hipErrorInvalidConfiguration;
   }
 }
