@@ -221,7 +221,7 @@ int rebuild_tables(rkx_batch *b)
     g.K = I.K;
     int nt = 0;
     if (I.K == 0) {
-      nt = make_chain_inst(I.dp, I.m, {}, nullptr, nullptr).nwg;
+      nt = make_chain_inst(I.dp, I.m, kChainBatchCells, {}, nullptr, nullptr).nwg;
     } else {
       const sweep_inst si = make_sweep_inst(I.dp, I.m, I.cfg, {}, nullptr, nullptr);
       nt = si.ntiles;
@@ -265,7 +265,7 @@ int enqueue_batched_step(rkx_batch *b, int r)
     if (nt == 0)
       continue;
     if (g.K == 0)
-      RKX_HIP(launch_chain(g.pattern, {{}, b->ci_dev, g.dev, nt, r}, b->stream));
+      RKX_HIP(launch_chain(g.pattern, kChainBatchCells, {{}, b->ci_dev, g.dev, nt, r}, b->stream));
     else
       RKX_HIP(launch_sweep(g.pattern, g.K, g.gen, {{}, b->si_dev, g.dev, nt, r}, b->stream));
   }
@@ -575,7 +575,7 @@ int rkx_batch_add(rkx_batch *b, const rkx_ode *p, const rkx_method *m, double t0
     I.pattern = sweep_pattern(*m);
     I.K = 0;
     const chain_inst ci =
-        make_chain_inst(dp, *m, I.ref, I.y[0], I.y[1]);
+        make_chain_inst(dp, *m, kChainBatchCells, I.ref, I.y[0], I.y[1]);
     RKX_HIP(hipMemcpyAsync(b->ci_dev + slot, &ci, sizeof(ci), hipMemcpyHostToDevice, b->stream));
   } else if (storage == RKX_STORAGE_LOW) {
     I.pattern = sweep_pattern(*m);

@@ -238,7 +238,7 @@ hipError_t fused_plan::launch(int r, hipStream_t stream)
     return launch_lv_step(dp, s, ref, y0, y1, r, stream);
   case kChain:
     chain.r = r;
-    return launch_chain(pattern, chain, stream);
+    return launch_chain(pattern, shape, chain, stream);
   case kTile:
     return launch_tile_step(pattern, shape, tile, r, stream);
   case kGroups:
@@ -262,7 +262,8 @@ int make_fused_plan(const rkx_ode &p, const rkx_method &m, int rows, int waves,
   f.pattern = sweep_pattern(m);
   if (chain_supported(f.dp, m)) {
     f.kind = fused_plan::kChain;
-    f.chain.one = make_chain_inst(f.dp, m, ref, y0, y1);
+    f.shape = chain_default_cells(f.dp, m);
+    f.chain.one = make_chain_inst(f.dp, m, f.shape, ref, y0, y1);
     f.chain.ntiles = f.chain.one.nwg;
   } else if (pairs_supported(f.dp, m)) {
     f.kind = fused_plan::kPairs;

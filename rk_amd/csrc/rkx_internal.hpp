@@ -374,17 +374,21 @@ hipError_t launch_d_groups(stage_group a, hipStream_t stream);
 struct chain_inst {
   int cells;             // M
   int tile_out;          // output cells per segment
-  int ntiles;            // segments of 1024 cells per step
-  int nwg;               // workgroups per step (each loops over segments)
+  int ntiles;            // segments (a wavefront each) per step
+  int nwg;               // workgroups per step (their waves loop over segments)
   double c0, d0, d1, c1, diff;
   double *y0, *y1;
   step_refs ref;         // the kernel forms h*A etc. from ref.meth
 };
 
 bool chain_supported(const dev_ode &p, const rkx_method &m);
-chain_inst make_chain_inst(const dev_ode &p, const rkx_method &m, const step_refs &ref,
+// C: cells per lane, 2..4 (the kernel's instance)
+chain_inst make_chain_inst(const dev_ode &p, const rkx_method &m, int C, const step_refs &ref,
                            double *y0, double *y1);
-hipError_t launch_chain(int pattern, const fused_launch<chain_inst> &a, hipStream_t stream);
+int chain_default_cells(const dev_ode &p, const rkx_method &m);
+// many chains in one launch fill the chip whatever C is: the least halo
+constexpr int kChainBatchCells = 4;
+hipError_t launch_chain(int pattern, int C, const fused_launch<chain_inst> &a, hipStream_t stream);
 
 // The step of one instance with a step ring: which kernel (kernels, for the D
 // form in groups of stages), and its launch.
@@ -394,7 +398,7 @@ struct fused_plan {
   step_refs ref{};
   double *y0 = nullptr, *y1 = nullptr;
   int s = 0, pattern = 0;
-  int shape = 0;           // tile
+  int shape = 0;           // tile; chain: cells per lane
   bool general = false;    // sweep: general ghost rows
   int waves = 0;           // sweep
   fused_launch<chain_inst> chain{};
