@@ -274,7 +274,8 @@ int enqueue_batched_step(rkx_batch *b, int r)
     if (!I.used || I.done)
       continue;
     if (I.storage == RKX_STORAGE_LOW && I.K < 0)
-      RKX_HIP(launch_lv_step(I.dp, I.m.s, I.ref, I.y[0], I.y[1], r, b->stream));
+      RKX_HIP(launch_lv_step(I.dp, I.m.s, I.ref, b->cf_dev + i, I.y[0], I.y[1], r,
+                             b->stream));
     else if (I.storage == RKX_STORAGE_FULL)
       RKX_HIP(launch_d_step(I.dp, b->cf_dev + i, I.m.s, b->st_dev + i, I.y[0], I.y[1], I.w,
                             I.dy, I.err, b->stream));

@@ -235,7 +235,7 @@ hipError_t fused_plan::launch(int r, hipStream_t stream)
 {
   switch (kind) {
   case kPairs:
-    return launch_lv_step(dp, s, ref, y0, y1, r, stream);
+    return launch_lv_step(dp, s, ref, coef, y0, y1, r, stream);
   case kChain:
     chain.r = r;
     return launch_chain(pattern, shape, chain, stream);
@@ -251,11 +251,12 @@ hipError_t fused_plan::launch(int r, hipStream_t stream)
 }
 
 int make_fused_plan(const rkx_ode &p, const rkx_method &m, int rows, int waves,
-                    const step_refs &ref, double *y0, double *y1, fused_plan *out)
+                    const step_refs &ref, dev_coef *coef, double *y0, double *y1, fused_plan *out)
 {
   fused_plan f;
   f.dp = make_dev_ode(p);
   f.ref = ref;
+  f.coef = coef;
   f.y0 = y0;
   f.y1 = y1;
   f.s = m.s;
@@ -811,7 +812,8 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
     return fail(RKX_EINVAL, "rkx_solve: tile_waves must be 1..4");
   fused_plan plan;
   if (fused) {
-    if (int rc = make_fused_plan(*p, *m, o.tile_rows, o.tile_waves, ref, ybuf[0], ybuf[1], &plan))
+    if (int rc = make_fused_plan(*p, *m, o.tile_rows, o.tile_waves, ref, cf_dev, ybuf[0], ybuf[1],
+                                 &plan))
       return fail(rc, std::string("rkx_solve: ") + rkx_last_error());
   } else if (grouped) {
     plan.kind = fused_plan::kGroups;

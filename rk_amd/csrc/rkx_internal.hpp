@@ -229,8 +229,9 @@ hipError_t launch_d_step(const dev_ode &p, const dev_coef *cf, int s, state *st,
 // Stage-fused step of independent LV pairs (rkx_kernels_lvpairs.hip): every
 // table with 2, 3, 4, 7, 8 or 13 stages
 bool pairs_supported(const dev_ode &p, const rkx_method &m);
-hipError_t launch_lv_step(const dev_ode &p, int s, const step_refs &R, double *y0, double *y1,
-                          int r, hipStream_t stream);
+// cf: room for the step's products, used by tables of 13 stages
+hipError_t launch_lv_step(const dev_ode &p, int s, const step_refs &R, dev_coef *cf, double *y0,
+                          double *y1, int r, hipStream_t stream);
 // Runs the pending step control of n states (those without a ring are left
 // alone), publishes it, and moves each ring on to slot 0 (rkx_kernels_step.hip):
 // after launches that ended on ring slot r, before the host reads the states
@@ -396,6 +397,7 @@ struct fused_plan {
   enum kind_t { kPairs, kChain, kTile, kSweep, kGroups } kind = kSweep;
   dev_ode dp{};
   step_refs ref{};
+  dev_coef *coef = nullptr;
   double *y0 = nullptr, *y1 = nullptr;
   int s = 0, pattern = 0;
   int shape = 0;           // tile; chain: cells per lane
@@ -411,6 +413,6 @@ struct fused_plan {
 // The plan of a problem and table with a fused kernel.  rows, waves: the
 // caller's row-sweep tile (0: chosen); y0, y1: the two y buffers.
 int make_fused_plan(const rkx_ode &p, const rkx_method &m, int rows, int waves,
-                    const step_refs &ref, double *y0, double *y1, fused_plan *out);
+                    const step_refs &ref, dev_coef *coef, double *y0, double *y1, fused_plan *out);
 
 }  // namespace rkx

@@ -106,11 +106,12 @@ int rkx_solve_noalloc(const rkx_ode *p, const rkx_method *m, double t0, double t
   if (int rc = scratch_ptr(&base))
     return rc;
 
-  // scratch layout: state, ring and method | second y buffer
+  // scratch layout: state, ring, method and coefficients | second y buffer
   struct header {
     state st;
     step_ring ring;
     dev_method meth;
+    dev_coef coef;
   };
   static_assert(sizeof(header) <= kHeaderBytes, "scratch header too small");
   header *hd = reinterpret_cast<header *>(base);
@@ -131,7 +132,8 @@ int rkx_solve_noalloc(const rkx_ode *p, const rkx_method *m, double t0, double t
   hh.ring = make_ring(v, false);
 
   fused_plan plan;
-  if (int rc = make_fused_plan(*p, *m, o.tile_rows, o.tile_waves, ref, ybuf[0], ybuf[1], &plan))
+  if (int rc = make_fused_plan(*p, *m, o.tile_rows, o.tile_waves, ref, &hd->coef, ybuf[0], ybuf[1],
+                               &plan))
     return fail(rc, std::string("rkx_solve_noalloc: ") + rkx_last_error());
   // everything the kernels read is written before the first launch
   if (y0_dev != y_dev)
