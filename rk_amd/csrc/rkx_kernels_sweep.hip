@@ -47,12 +47,6 @@ bool sweep_supported(const dev_ode &p, const rkx_method &m)
   return p.kind == RKX_BRUSS2D && p.N >= 2 && pattern_of(m) != 0;
 }
 
-// Relative cost of one lane x row iteration of k_sweep for strips of 1..4
-// waves per component, measured on MI355X (DOPRI54, N = 2000, one dispatch
-// round): 1 wave pays a barrier and an LDS exchange for few lanes, 3 waves
-// (6 per workgroup) do not pack two workgroups per CU.
-constexpr double kTileCost[4] = {1.36, 1.0, 1.67, 0.97};
-
 namespace {
 
 // Strips of an N-column grid for strips of 64K lanes: as many full-width
@@ -80,25 +74,16 @@ strip_geom strips_of(int N, int s, int K)
   return strip_geom{nstrips, (N + nstrips - 1) / nstrips, 0};
 }
 
-// Relative cost of one step of an N x N instance with strips of 64K columns
-// and bands of R rows: lanes x row iterations (the balanced band height plus
-// the 2(s-1) halo iterations and a prologue of about 4) x the measured
-// per-lane factor of the strip width.  trip > 0 rounds a band's row
-// iterations after the pro peeled ones up to whole trips of that many rows.
-double tile_work(int N, int s, int K, int R, int trip, int pro)
+// Relative time of one step whose workgroups all run at once: the row
+// iterations of a band (plus about 5 for the step's start and end) times what
+// one costs at the waves per SIMD that per_cu workgroups of a compute unit
+// come to.  Measured, DOPRI54: 0.53 us an iteration at one wave per SIMD, 0.70
+// at two, whatever the strip width that makes them up, and in proportion
+// beyond (FP64 issue).
+double sweep_time(int K, int per_cu, long long iters)
 {
-  const int L = 64 * K;
-  const int oc = L - 2 * s;
-  if (oc < 1 || R < 1 || N < 1)
-    return 1e300;
-  const strip_geom g = strips_of(N, s, K);
-  const long long nbands = (N + R - 1) / R;
-  const long long reff = g.split ? R : (N + nbands - 1) / nbands;
-  long long iters = reff + 2 * (s - 1);
-  if (trip > 0)
-    iters = pro + (iters - pro + trip - 1) / trip * trip;
-  return kTileCost[K - 1] * static_cast<double>(g.wgs(nbands) * L) *
-         static_cast<double>(iters + 4);
+  const int wps = (2 * K * per_cu + 3) / 4;
+  return static_cast<double>(iters + 5) * (wps < 2 ? 0.76 : 0.5 * wps);
 }
 
 // Most bands per strip whose workgroups fit `slots`.
@@ -165,15 +150,14 @@ int sweep_band_rows(int pattern, int s, int rows)
 
 // Default tile: strips of 64*K columns (2K waves per workgroup) and the band
 // height R for which all strips x bands tiles are resident at once (one
-// dispatch round: a second, partial round would leave most CUs idle while
-// it runs), with bands as tall as that allows (the s-1 halo rows a band
-// recomputes are a smaller share of taller bands).  Where more than one
-// workgroup fits a CU, every count from the one that gives two waves per
-// SIMD up to the resident maximum is a candidate: on MI355X the FP64 row
-// loop gains little from more than two waves per SIMD (RKF23 at N = 2000:
-// 58 us per step either way with the same bands), so the taller bands of
-// fewer workgroups per CU can win (RKF23: 54.7 us with one per CU against
-// 58.6 us filling both).  The candidate with the lowest modelled cost wins.
+// dispatch round: a second, partial round would leave most CUs idle while it
+// runs), with bands as tall as that allows (the s-1 halo rows a band
+// recomputes are a smaller share of taller bands).  Every count of workgroups
+// per CU up to the resident maximum is a candidate, and the one with the
+// shortest modelled step (sweep_time) wins.  The model it replaces priced
+// lanes x iterations, as if a wider strip's idle lanes lengthened the step:
+// VERNER65 N=717 33.2 us per step with its choice and 22.6 with this one,
+// DOPRI54 N=1000 29.4 / 27.0, DOPRI87 N=300 65.9 / 45.3.
 // A grid so wide that one band per strip gives fewer tiles than CUs (N =
 // 32767, K = 4: 136 strips) or more than fit at once (DOPRI87, N = 32767:
 // 322 strips of 2 waves) instead takes shorter bands over several rounds
@@ -209,11 +193,16 @@ sweep_cfg sweep_default_cfg(const dev_ode &p, const rkx_method &m)
     const int res = resident_blocks(pat, K);
     if (res < 1)
       continue;                                     // too wide for this table's kernel
-    const int per_cu_min = std::min(res, (4 + K - 1) / K);   // 2K waves each: 2 per SIMD
-    for (int per_cu = per_cu_min; per_cu <= res; ++per_cu) {
+    for (int per_cu = 1; per_cu <= res; ++per_cu) {
       const int rows = band_rows_for(bands_for_slots(g, static_cast<long long>(cus) * per_cu));
-      const double cost = tile_work(N, s, K, rows, trip, pro);
-      if (cost < best_cost) {
+      long long iters = rows + 2 * (s - 1);
+      if (trip > 0)
+        iters = pro + (iters - pro + trip - 1) / trip * trip;
+      const long long tiles = g.wgs((N + rows - 1) / rows);
+      const long long rounds = (tiles + cus * per_cu - 1) / (cus * per_cu);
+      const int there = static_cast<int>(std::min<long long>(per_cu, (tiles + cus - 1) / cus));
+      const double cost = static_cast<double>(rounds) * sweep_time(K, there, iters);
+      if (cost <= best_cost) {                      // wider strips: less halo traffic
         best_cost = cost;
         best = sweep_cfg{K, rows};
       }
