@@ -97,8 +97,8 @@ int rkx_method_get(const char *name, rkx_method *m);
 
 /* ---- single solve (replaces solver(), include/solver.h:47) --------------- */
 enum {
-  RKX_IMPL_D = 0,        /* stage kernels, full storage (src/impl/seq/D.c); on BRUSS2D up
-                            to four stages to a kernel */
+  RKX_IMPL_D = 0,        /* stage kernels, full storage (src/impl/seq/D.c); on BRUSS2D this
+                            and A, E, F below run up to four stages to a kernel */
   RKX_IMPL_PIPED = 1,    /* the same stage-fused sweep as RKX_IMPL_PIPEDLS: the fused form
                             keeps every stage vector of src/impl/seq/PipeD.c in registers,
                             so it has no full-storage variant (two vectors of n) */

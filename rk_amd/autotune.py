@@ -63,13 +63,15 @@ def solve_form(problem, meth, y0, tol, t0=0.0, te=1.0, h0=1e-3, window=(20, 120)
     reference (src/impl/seq/D.c, A.c, E.c, F.c).  All of them give the same
     steps and results bitwise, so per-step times compare directly; each is
     the difference of two solves capped at window[0] and window[1] attempted
-    steps (set-up excluded).  y0: device tensor.  Returns (fastest form,
-    {form: seconds per attempted step})."""
+    steps (set-up excluded), after one that is not timed: a kernel's first
+    launch in a process loads its code within the step loop.  y0: device
+    tensor.  Returns (fastest form, {form: seconds per attempted step})."""
     import torch
     from .solver import solve
     y = torch.empty_like(y0)
     times = {}
     for f in forms:
+        solve(problem, meth, t0, te, y0, y, tol, h0=h0, impl=f, step_limit=window[0])
         a, _ = solve(problem, meth, t0, te, y0, y, tol, h0=h0, impl=f, step_limit=window[0])
         b, _ = solve(problem, meth, t0, te, y0, y, tol, h0=h0, impl=f, step_limit=window[1])
         if b.steps > a.steps:

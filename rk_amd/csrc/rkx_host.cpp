@@ -243,7 +243,7 @@ hipError_t fused_plan::launch(int r, hipStream_t stream)
     return launch_tile_step(pattern, shape, tile, r, stream);
   case kGroups:
     groups.r = r;
-    return launch_d_groups(groups, stream);
+    return launch_groups(form, groups, nz, stream);
   default:
     sweep.r = r;
     return launch_sweep(pattern, waves, general, sweep, stream);
@@ -639,13 +639,15 @@ int rkx_eval_comp_host(const rkx_ode *p, int i, double t, const double *y, doubl
 // entries of the table), F fuses each RHS with the next stage's gather.  All
 // give the same results bitwise.  Counts: reads + writes of n doubles.
 //
-// On BRUSS2D, D runs up to four stages to a kernel (rkx_kernels_dgroup.hip)
-// and moves the fewest vectors for every table: 13 for 7 stages against F's
-// 49 (N = 2000: 250 us a step against 588).
+// On BRUSS2D they run up to four stages to a kernel (rkx_kernels_groups.hip)
+// and move 13 (D) and 11 vectors a step for 7 stages.
 static int least_traffic_form(const rkx_ode &p, const rkx_method &m)
 {
+  // BRUSS2D, stages in groups: up to two groups D and E cost the same (N = 1000,
+  // DOPRI54: 51 and 50 us a step), beyond that D's partial sums cost more
+  // than E's stage derivatives (13 stages: 179 and 130 us)
   if (p.kind == RKX_BRUSS2D)
-    return RKX_IMPL_D;
+    return m.s <= 8 ? RKX_IMPL_D : RKX_IMPL_E;
   const int s = m.s;
   int d = (s + 2) + 5;                                   // first and last stage
   for (int i = 1; i < s - 1; ++i)
@@ -737,9 +739,9 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
     fused = false;
   }
   const bool gather = impl == RKX_IMPL_A || impl == RKX_IMPL_E || impl == RKX_IMPL_F;
-  // D on BRUSS2D runs its stages in groups; these and the fused forms start
-  // each step with the control of the one before (step_ring)
-  const bool grouped = impl == RKX_IMPL_D && dp.kind == RKX_BRUSS2D;
+  // on BRUSS2D the full-storage forms run their stages in groups; these and the
+  // fused forms start each step with the control of the one before (step_ring)
+  const bool grouped = !fused && dp.kind == RKX_BRUSS2D;
   const bool ringed = fused || grouped;
   const size_t n = static_cast<size_t>(p->n);
   const size_t vec = n * sizeof(double);
@@ -817,8 +819,10 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
       return fail(rc, std::string("rkx_solve: ") + rkx_last_error());
   } else if (grouped) {
     plan.kind = fused_plan::kGroups;
-    plan.groups = stage_group{dp.N,    s,       0, 0, 0,  0,   0,  dp.coef,
-                              ybuf[0], ybuf[1], w, dy, err, ref};
+    plan.form = impl;
+    plan.nz = nz;
+    plan.groups = stage_group{dp.N,    s,       0, 0, 0, 0, 0, dp.coef, ybuf[0], ybuf[1],
+                              gather ? v : w, dy, err, ref};
   }
 
   // one attempted step; r: the ring slot a fused kernel reads

@@ -356,7 +356,8 @@ inline int tile_pieces(int n, int full, int halo)
   return n <= full ? 1 : 2 + (rest > 0 ? (rest + full - 2 * halo - 1) / (full - 2 * halo) : 0);
 }
 
-// The D form of a BRUSS2D step, stages in groups (rkx_kernels_dgroup.hip).
+// A full-storage form of a BRUSS2D step, stages in groups
+// (rkx_kernels_groups.hip).
 struct stage_group {
   int N, s;
   int i0;                // the launch's first stage
@@ -364,12 +365,13 @@ struct stage_group {
   int r;                 // ring slot, the same for every kernel of a step
   double coef;
   double *y0, *y1;
-  double *w, *dy, *err;  // w_1..w_{s-1} one after another
+  double *w, *dy, *err;  // D: w_1..w_{s-1} one after another; A, E, F: w holds v_0..
   step_refs ref;
 };
 constexpr int kGroupBlocks = 512;   // two workgroups on a compute unit
-// all of a step's kernels; a: without i0 and the tile counts
-hipError_t launch_d_groups(stage_group a, hipStream_t stream);
+// all of a step's kernels, form RKX_IMPL_D, A, E or F; a: without i0 and the
+// tile counts
+hipError_t launch_groups(int form, stage_group a, const gather_masks &nz, hipStream_t stream);
 
 // One LV chain instance as the fused chain kernel sees it (device memory).
 struct chain_inst {
@@ -391,8 +393,8 @@ int chain_default_cells(const dev_ode &p, const rkx_method &m);
 constexpr int kChainBatchCells = 4;
 hipError_t launch_chain(int pattern, int C, const fused_launch<chain_inst> &a, hipStream_t stream);
 
-// The step of one instance with a step ring: which kernel (kernels, for the D
-// form in groups of stages), and its launch.
+// The step of one instance with a step ring: which kernel (kernels, for the
+// full-storage forms in groups of stages), and its launch.
 struct fused_plan {
   enum kind_t { kPairs, kChain, kTile, kSweep, kGroups } kind = kSweep;
   dev_ode dp{};
@@ -406,7 +408,9 @@ struct fused_plan {
   fused_launch<chain_inst> chain{};
   tile_inst tile{};
   fused_launch<sweep_inst> sweep{};
-  stage_group groups{};    // the D form of BRUSS2D
+  int form = 0;            // groups: RKX_IMPL_D, A, E, F on BRUSS2D
+  stage_group groups{};
+  gather_masks nz{};
   // one attempted step; r: the ring slot the kernel reads
   hipError_t launch(int r, hipStream_t stream);
 };

@@ -14,8 +14,9 @@
 // Every w_l, dy and err receives the same terms in the same ascending order as
 // the scatter form of D (block-inline.h:253-320), so all three give D's
 // results bitwise.  They differ in traffic: per DOPRI54 step A and E move
-// about 54 vectors of n, F about 49, D 69 -- candidates for problems without
-// a fused kernel (LV pairs, tables without a compiled pattern).  The output
+// about 54 vectors of n, F about 49, D 69 -- candidates for LV problems
+// without a fused kernel for the table.  BRUSS2D solves run these orders in
+// groups of stages instead (rkx_kernels_groups.hip).  The output
 // kernel also forms y_new = y + dy into the other y buffer and the error
 // max-norm (A.c:85-92), and its last workgroup runs the step control.
 #include "rkx_device.hpp"

@@ -1,4 +1,4 @@
-"""The D form of BRUSS2D in groups of stages (rkx_kernels_dgroup.hip) against
+"""The D form of BRUSS2D in groups of stages (rkx_kernels_groups.hip) against
 the E form's kernels, bitwise: every attempted step's (t, h, err), the counts
 and the final vector.  Sizes at the edges of the 64-column, 32-row tiles for
 every group size, tables of 2 to 16 stages (one, two, three and four groups),
