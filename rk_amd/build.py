@@ -32,6 +32,7 @@ SOURCES = [
     "rkx_kernels_sweep_verner65.hip",
     "rkx_kernels_sweep_dopri87.hip",
     "rkx_kernels_tile.hip",
+    "rkx_kernels_run.hip",
     "rkx_kernels_groups.hip",
     "rkx_kernels_lv.hip",
     "rkx_kernels_chain.hip",

@@ -250,6 +250,17 @@ hipError_t fused_plan::launch(int r, hipStream_t stream)
   }
 }
 
+namespace {
+// Attempts a launch of one workgroup makes: its start and end (4 us) are
+// spread over them, and a launch is short enough for the host to follow.
+constexpr int kRunSteps = 32;
+}  // namespace
+
+hipError_t fused_plan::launch_many(int r, hipStream_t stream)
+{
+  return launch_run(pattern, run, r, many, stream);
+}
+
 int make_fused_plan(const rkx_ode &p, const rkx_method &m, int rows, int waves,
                     const step_refs &ref, dev_coef *coef, double *y0, double *y1, fused_plan *out)
 {
@@ -273,7 +284,16 @@ int make_fused_plan(const rkx_ode &p, const rkx_method &m, int rows, int waves,
     // buffer that is not aligned for it stays with the row sweep
     const bool aligned = ((reinterpret_cast<uintptr_t>(y0) | reinterpret_cast<uintptr_t>(y1)) &
                           15u) == 0;
-    f.shape = rows <= 0 && waves <= 0 && aligned ? tile_default_shape(f.dp, m) : -1;
+    const bool free_tile = rows <= 0 && waves <= 0 && aligned;
+    f.shape = free_tile ? tile_default_shape(f.dp, m) : -1;
+    if (free_tile && run_supported(f.pattern, f.dp.N)) {
+      f.many = kRunSteps;
+      f.run.N = f.dp.N;
+      f.run.coef = f.dp.coef;
+      f.run.y0 = y0;
+      f.run.y1 = y1;
+      f.run.ref = ref;
+    }
     if (f.shape >= 0) {
       f.kind = fused_plan::kTile;
       f.tile = make_tile_inst(f.dp, m, f.shape, ref, y0, y1);
@@ -346,8 +366,13 @@ namespace {
 // control ends the loop.  Long solves replay a graph of kChunk steps (1.7 us
 // of launch a step, 2.6 us launched one by one), captured while the first
 // steps run; it takes 85 us, so short solves do without.
+//
+// many > 0: a launch makes up to that many attempts (and none pending: the
+// host sees the state after the last of them).  Two launches are kept in
+// flight then, the second covering the host's reaction to the first.
 template <class STEP>
-int run_steps(STEP &&enqueue, const host_view &view, double te, int step_limit, hipStream_t stream)
+int run_steps(STEP &&enqueue, int many, const host_view &view, double te, int step_limit,
+              hipStream_t stream)
 {
   constexpr int kChunk = 32;          // a multiple of kRing
   constexpr int kLow = 12;            // launches in flight below which more are made
@@ -380,7 +405,14 @@ int run_steps(STEP &&enqueue, const host_view &view, double te, int step_limit, 
     if (step_limit > 0)
       left = std::fmin(left, static_cast<double>(step_limit) - static_cast<double>(made));
     const double want = std::fmin(left + 1.0, 1e9) - static_cast<double>(launched - made);
-    if (want >= 1.0 && launched - made < kLow) {
+    if (many > 0) {
+      if (want >= 1.0 && launched - made <= many) {
+        RKX_HIP(enqueue(static_cast<int>(launched / many) & (kRing - 1)));
+        launched += many;
+        spin = 0;
+        continue;
+      }
+    } else if (want >= 1.0 && launched - made < kLow) {
       const bool chunks = want >= kChunk && launched % kRing == 0;
       const bool graph = chunks && gh.ge;
       const bool make = chunks && !gh.ge && launched > 0 && left >= kGraphFrom;
@@ -887,7 +919,10 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
       RKX_HIP(hipStreamSynchronize(stream));
     }
   } else {
-    if (int rc = run_steps(enqueue_step, *mem.view, te, o.step_limit, stream))
+    auto enqueue_many = [&](int r) { return plan.launch_many(r, stream); };
+    if (int rc = plan.many > 0
+                     ? run_steps(enqueue_many, plan.many, *mem.view, te, o.step_limit, stream)
+                     : run_steps(enqueue_step, 0, *mem.view, te, o.step_limit, stream))
       return rc;
     fin.t = mem.view->t;
     fin.h = mem.view->h;

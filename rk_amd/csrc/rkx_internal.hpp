@@ -347,6 +347,10 @@ tile_inst make_tile_inst(const dev_ode &p, const rkx_method &m, int shape, const
 // The shape a single grid runs in, or -1: the row sweep is the faster form.
 int tile_default_shape(const dev_ode &p, const rkx_method &m);
 hipError_t launch_tile_step(int pattern, int shape, const tile_inst &I, int r, hipStream_t stream);
+// Grids of one workgroup (rkx_kernels_run.hip): up to `steps` attempts in one
+// launch, each with its control; I: N, coef, the buffers and ref.
+bool run_supported(int pattern, int N);
+hipError_t launch_run(int pattern, const tile_inst &I, int r, int steps, hipStream_t stream);
 
 // Pieces of n rows or columns in tiles of `full` of them with a halo on either
 // inner side: the first and the last piece lose one halo, those between two.
@@ -413,6 +417,10 @@ struct fused_plan {
   gather_masks nz{};
   // one attempted step; r: the ring slot the kernel reads
   hipError_t launch(int r, hipStream_t stream);
+  // > 0: launch_many makes up to this many, each with its control
+  int many = 0;
+  tile_inst run{};
+  hipError_t launch_many(int r, hipStream_t stream);
 };
 // The plan of a problem and table with a fused kernel.  rows, waves: the
 // caller's row-sweep tile (0: chosen); y0, y1: the two y buffers.

@@ -45,6 +45,114 @@ __device__ __forceinline__ double wave_shift(double v)
 __device__ __forceinline__ double from_left(double v) { return wave_shift<0x138>(v); }    // wave_shr:1
 __device__ __forceinline__ double from_right(double v) { return wave_shift<0x130>(v); }   // wave_shl:1
 
+// Where a wave's cells lie, for a stage.
+struct tile_place {
+  int N, row;                  // the wave's (or half wave's) first row
+  bool left, right;            // the lane's column is 0, N - 1
+  double mE, mW, coef;
+};
+
+// Stage i of a wave's C rows: the derivatives, then their terms in the row's
+// accumulators ([0] dy, [1..s-1] w_l, [s] err).  yu, yv: y with the row on
+// either side; nu, nv, su, sv: the rows beyond the wave's of this stage's w.
+// HALVES: a wave holds two rows side by side, in 32 lanes each.
+template <class P, int C, int i, bool SMALL, bool HALVES>
+__device__ __forceinline__ void tile_stage(const tile_place &t, const double *ki,
+                                           const double (&yu)[C + 2], const double (&yv)[C + 2],
+                                           double nu, double nv, double su, double sv,
+                                           double (&au)[C][P::s + 1], double (&av)[C][P::s + 1])
+{
+  constexpr int s = P::s;
+  // stage i of every row of the wave, before its accumulators change
+  double fu[C], fv[C];
+  static_for<C>([&](auto ct) {
+    constexpr int c = decltype(ct)::value;
+    auto wu = [&](auto kt) -> double {
+      constexpr int k = decltype(kt)::value;
+      if constexpr (i == 0)
+        return yu[k + 1];
+      else if constexpr (k < 0)
+        return nu;
+      else if constexpr (k >= C)
+        return su;
+      else
+        return au[k][i];
+    };
+    auto wvv = [&](auto kt) -> double {
+      constexpr int k = decltype(kt)::value;
+      if constexpr (i == 0)
+        return yv[k + 1];
+      else if constexpr (k < 0)
+        return nv;
+      else if constexpr (k >= C)
+        return sv;
+      else
+        return av[k][i];
+    };
+    const double u = wu(int_c<c>{}), v = wvv(int_c<c>{});
+    double un = wu(int_c<c - 1>{}), vn = wvv(int_c<c - 1>{});
+    double us = wu(int_c<c + 1>{}), vs = wvv(int_c<c + 1>{});
+    if constexpr (c == 0) {
+      const bool top = t.row + c == 0;
+      un = top ? us : un;
+      vn = top ? vs : vn;
+    }
+    if constexpr (SMALL || c == C - 1) {
+      const bool bot = t.row + c == t.N - 1;
+      us = bot ? un : us;
+      vs = bot ? vn : vs;
+    }
+    double uE = from_right(u), vE = from_right(v);
+    double uW = from_left(u), vW = from_left(v);
+    if constexpr (HALVES) {                    // lane 32 starts a row of its own
+      uW = t.left ? 0.0 : uW;
+      vW = t.left ? 0.0 : vW;
+    }
+    if constexpr (SMALL) {                     // the column after the last
+      uE = t.right ? 0.0 : uE;
+      vE = t.right ? 0.0 : vE;
+    }
+    // ((vN + vS) + vW) + vE - 4c; 1, 2 and 4 times are exact
+    const double lu = __builtin_fma(
+        -4.0, u, __builtin_fma(t.mE, uE, __builtin_fma(t.mW, uW, un + us)));
+    const double lv = __builtin_fma(
+        -4.0, v, __builtin_fma(t.mE, vE, __builtin_fma(t.mW, vW, vn + vs)));
+    bruss_react(u, v, lu, lv, t.coef, fu[c], fv[c]);
+  });
+  static_for<C>([&](auto ct) {
+    constexpr int c = decltype(ct)::value;
+    if constexpr (i == 0) {
+      static_for<s>([&](auto lt) {
+        constexpr int l = decltype(lt)::value;
+        if constexpr (l >= 1) {
+          au[c][l] = nzA<P>(l, 0) ? yu[c + 1] + ki[l - 1] * fu[c] : yu[c + 1];
+          av[c][l] = nzA<P>(l, 0) ? yv[c + 1] + ki[l - 1] * fv[c] : yv[c + 1];
+        }
+      });
+      au[c][0] = ki[s - 1] * fu[c];
+      av[c][0] = ki[s - 1] * fv[c];
+      au[c][s] = ki[s] * fu[c];
+      av[c][s] = ki[s] * fv[c];
+    } else {
+      static_for<s>([&](auto lt) {
+        constexpr int l = decltype(lt)::value;
+        if constexpr (l > i && nzA<P>(l, i)) {
+          au[c][l] += ki[l - i - 1] * fu[c];
+          av[c][l] += ki[l - i - 1] * fv[c];
+        }
+      });
+      if constexpr ((P::b >> i) & 1u) {
+        au[c][0] += ki[s - i - 1] * fu[c];
+        av[c][0] += ki[s - i - 1] * fv[c];
+      }
+      if constexpr ((P::e >> i) & 1u) {
+        au[c][s] += ki[s - i] * fu[c];
+        av[c][s] += ki[s - i] * fv[c];
+      }
+    }
+  });
+}
+
 // SMALL: grids narrower or shorter than a tile, whose last row and column may
 // lie anywhere in it.
 //
@@ -84,7 +192,7 @@ k_tile(step_ring *ring, const dev_method *meth, double *y0, double *y1, int r, i
   const int col = tc + lane;
   const int row = tr + wv * C;                   // the wave's first row
   const bool left = col == 0, right = col == N - 1;
-  const double mE = left ? 2.0 : 1.0, mW = right ? 2.0 : 1.0;
+  const tile_place T{N, row, left, right, left ? 2.0 : 1.0, right ? 2.0 : 1.0, coef};
 
   // Everything that comes from memory is asked for before the control is
   // waited for: the table's columns, and y (the wave's rows and the row on
@@ -139,89 +247,9 @@ k_tile(step_ring *ring, const dev_method *meth, double *y0, double *y1, int r, i
     }
     if (!need)
       return;
-    // stage i of every row of the wave, before its accumulators change
-    double fu[C], fv[C];
+    tile_stage<P, C, i, SMALL, false>(T, kc.k[i], yu, yv, nu, nv, su, sv, au, av);
     static_for<C>([&](auto ct) {
       constexpr int c = decltype(ct)::value;
-      auto wu = [&](auto kt) -> double {
-        constexpr int k = decltype(kt)::value;
-        if constexpr (i == 0)
-          return yu[k + 1];
-        else if constexpr (k < 0)
-          return nu;
-        else if constexpr (k >= C)
-          return su;
-        else
-          return au[k][i];
-      };
-      auto wvv = [&](auto kt) -> double {
-        constexpr int k = decltype(kt)::value;
-        if constexpr (i == 0)
-          return yv[k + 1];
-        else if constexpr (k < 0)
-          return nv;
-        else if constexpr (k >= C)
-          return sv;
-        else
-          return av[k][i];
-      };
-      const double u = wu(int_c<c>{}), v = wvv(int_c<c>{});
-      double un = wu(int_c<c - 1>{}), vn = wvv(int_c<c - 1>{});
-      double us = wu(int_c<c + 1>{}), vs = wvv(int_c<c + 1>{});
-      if constexpr (SMALL || c == 0) {
-        const bool top = row + c == 0;
-        un = top ? us : un;
-        vn = top ? vs : vn;
-      }
-      if constexpr (SMALL || c == C - 1) {
-        const bool bot = row + c == N - 1;
-        us = bot ? un : us;
-        vs = bot ? vn : vs;
-      }
-      double uE = from_right(u), vE = from_right(v);
-      if constexpr (SMALL) {                     // the column after the last
-        uE = right ? 0.0 : uE;
-        vE = right ? 0.0 : vE;
-      }
-      // ((vN + vS) + vW) + vE - 4c; 1, 2 and 4 times are exact
-      const double lu = __builtin_fma(
-          -4.0, u, __builtin_fma(mE, uE, __builtin_fma(mW, from_left(u), un + us)));
-      const double lv = __builtin_fma(
-          -4.0, v, __builtin_fma(mE, vE, __builtin_fma(mW, from_left(v), vn + vs)));
-      bruss_react(u, v, lu, lv, coef, fu[c], fv[c]);
-    });
-    const double *ki = kc.k[i];
-    static_for<C>([&](auto ct) {
-      constexpr int c = decltype(ct)::value;
-      if constexpr (i == 0) {
-        static_for<s>([&](auto lt) {
-          constexpr int l = decltype(lt)::value;
-          if constexpr (l >= 1) {
-            au[c][l] = nzA<P>(l, 0) ? yu[c + 1] + ki[l - 1] * fu[c] : yu[c + 1];
-            av[c][l] = nzA<P>(l, 0) ? yv[c + 1] + ki[l - 1] * fv[c] : yv[c + 1];
-          }
-        });
-        au[c][0] = ki[s - 1] * fu[c];
-        av[c][0] = ki[s - 1] * fv[c];
-        au[c][s] = ki[s] * fu[c];
-        av[c][s] = ki[s] * fv[c];
-      } else {
-        static_for<s>([&](auto lt) {
-          constexpr int l = decltype(lt)::value;
-          if constexpr (l > i && nzA<P>(l, i)) {
-            au[c][l] += ki[l - i - 1] * fu[c];
-            av[c][l] += ki[l - i - 1] * fv[c];
-          }
-        });
-        if constexpr ((P::b >> i) & 1u) {
-          au[c][0] += ki[s - i - 1] * fu[c];
-          av[c][0] += ki[s - i - 1] * fv[c];
-        }
-        if constexpr ((P::e >> i) & 1u) {
-          au[c][s] += ki[s - i] * fu[c];
-          av[c][s] += ki[s - i] * fv[c];
-        }
-      }
       if constexpr (i + 1 < s) {
         if constexpr (c == 0)
           edge[(i + 1) & 1][wv][0][lane] = make_double2(au[c][i + 1], av[c][i + 1]);
