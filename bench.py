@@ -141,41 +141,32 @@ def gpu_c1():
     return {"steps": st.steps, "kernel_s": st.kernel_time, "wall_s": wall}
 
 
-def d_form_passes(s):
-    """Vector passes (reads + writes of n doubles) of one step of the stage
-    kernels of the D form: first stage reads y and writes w_1..w_{s-1}, dy,
-    err; intermediate stage i reads w_i and updates w_{i+1..s-1}, dy, err;
-    the last reads w_{s-1}, dy, err, y and writes y_new."""
-    return (s + 2) + sum(5 + 2 * (s - 1 - i) for i in range(1, s - 1)) + 5
-
-
-def gather_form_passes(meth, impl):
-    """Vector passes of one step of the gather forms.  A and E: stage 0 reads
-    y and writes v_0; stage l gathers (reads y and the v_i it adds, writes w)
-    then evaluates (reads w, writes v_l); the output reads the v_i it adds and
-    y, and writes y_new.  A adds only the non-zero coefficients of the table.
-    F: stage l < s-1 reads w_l (stage 0: y), y and v_0..v_{l-1}, and writes
-    v_l and w_{l+1}; the last stage reads w_{s-1} and writes v_{s-1}."""
-    from rk_amd.methods import method
-    m = method(meth)
-    s = m.s
-    A = [[m.A[l][i] for i in range(s)] for l in range(s)]
-    if impl == "F":
-        return 3 + sum(l + 4 for l in range(1, s - 1)) + 2 + (s + 2)
-    skip = impl == "A"
-    nnz = [sum(1 for i in range(l) if A[l][i] != 0.0 or not skip) for l in range(s)]
-    out = 1 + sum(1 for i in range(1, s)
-                  if not skip or m.b[i] != 0.0 or m.b[i] - m.b_hat[i] != 0.0)
-    return 2 + sum(2 + nnz[l] + 2 for l in range(1, s)) + out + 2
-
-
 def form_passes(meth, impl):
+    """Vector passes (reads + writes of n doubles) of one BRUSS2D step.  The
+    full-storage forms run their s stages in groups of up to four, a kernel
+    each.  D: a group reads its w (the first y), reads and writes (the first:
+    writes) every later w, dy and err; the last also reads y and writes y_new.
+    A, E, F: a group reads y and the v of the groups before and writes its
+    own; the last writes y_new instead.  Halo re-reads are not counted."""
     from rk_amd.methods import method
-    if impl == "D":
-        return d_form_passes(method(meth).s)
-    if impl in ("A", "E", "F"):
-        return gather_form_passes(meth, impl)
-    return 2
+    if impl not in ("D", "A", "E", "F"):
+        return 2
+    s = method(meth).s
+    groups = (s + 3) // 4
+    total = 0
+    for q in range(groups):
+        i0, i1 = q * s // groups, (q + 1) * s // groups
+        first, last = q == 0, q == groups - 1
+        if impl == "D":
+            later = s - i1 + 2
+            total += 1 if first else i1 - i0
+            if last:
+                total += 1 + (0 if first else 3)
+            else:
+                total += later if first else 2 * later
+        else:
+            total += 1 + i0 + (1 if last else i1 - i0)
+    return total
 
 
 def c2_matrix_leg(window=(300, 1300), impls=("D", "A", "E", "F", "PipeDls"),
@@ -211,8 +202,7 @@ def c2_matrix_leg(window=(300, 1300), impls=("D", "A", "E", "F", "PipeDls"),
 def loop_order_leg():
     """The step-form autotuner (rk_amd.autotune.solve_form) on three problems:
     BRUSS2D N=2000 (fused sweep), an LV chain of 5e5 cells (fused chain
-    kernel) and 4e6 independent LV pairs (no fused kernel: D, A, E, F only;
-    "PipeDls" runs D there); DOPRI54, per-step times over attempted steps
+    kernel) and 4e6 independent LV pairs (fused per-pair kernel); DOPRI54, per-step times over attempted steps
     20..120 and the form it picks."""
     import torch
     import rk_amd

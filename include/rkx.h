@@ -115,10 +115,12 @@ enum {
 };
 
 enum {
-  RKX_CTRL_DEVICE = 0,     /* step control on the device, in the last workgroup of each
-                              step; the one pow() of the new h (include/tools.h:226) is
-                              the C library's pow restated bitwise (rkx_pow_device), so
-                              every h equals the reference's (default) */
+  RKX_CTRL_DEVICE = 0,     /* step control on the device, at the start of the next step's
+                              kernels (LV full-storage forms: in the last workgroup of
+                              each step); the one pow() of the new h
+                              (include/tools.h:226) is the C library's pow restated
+                              bitwise (rkx_pow_device), so every h equals the
+                              reference's (default) */
   RKX_CTRL_HOST = 1        /* step control on the host after each step with the C
                               library's pow (one host round trip per step; bitwise the
                               same steps) */
@@ -129,11 +131,13 @@ typedef struct rkx_opts {
   int step_limit;        /* STEP_LIMIT (config.h:70-72); <= 0: unlimited */
   int impl;              /* RKX_IMPL_* */
   int ctrl;              /* RKX_CTRL_* */
-  int tile_rows;         /* sweep band height in grid rows (0: tuned default; VERNER65
+  int tile_rows;         /* BRUSS2D with either of these two set runs the row sweep;
+                            with both 0, small grids run in 64-column tiles or in one
+                            workgroup.  Band height in grid rows (0: chosen; VERNER65
                             rounds it up so that a band's row iterations after its
                             first 2(s-1) fill whole trips of its ring) */
   int tile_waves;        /* sweep strip width in wavefronts per component, 1..4 (DOPRI87:
-                            1..2, its kernel runs one wave per SIMD); 0: tuned default.
+                            1..2, its kernel runs one wave per SIMD); 0: chosen.
                             With an even width, columns left over after the full
                             strips that fit half a strip run as a narrow strip whose
                             bands share workgroups two at a time */

@@ -4,9 +4,10 @@
 // Instances with a fused kernel (BRUSS2D row sweep, LV chain segments; low
 // storage) are grouped by (method pattern, kernel and strip width); one
 // launch per group covers the tiles of all
-// of the group's active instances through an (instance, tile) table, and the
-// last tile of each instance runs that instance's step control.  Instances
-// without a fused kernel (full storage) run the stage kernels of the D form.
+// of the group's active instances through an (instance, tile) table; every
+// tile of an instance starts with the step control of that instance's attempt
+// before (step_ring).  Instances without a fused kernel (full storage) run the
+// stage kernels of the D form.
 // The host polls the instances' states every few batched steps, drops
 // finished instances from the tile tables and lets callers add new ones in
 // between (continuous batching).  An instance's arithmetic depends only on

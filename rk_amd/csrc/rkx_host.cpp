@@ -672,14 +672,16 @@ int rkx_eval_comp_host(const rkx_ode *p, int i, double t, const double *y, doubl
 // give the same results bitwise.  Counts: reads + writes of n doubles.
 //
 // On BRUSS2D they run up to four stages to a kernel (rkx_kernels_groups.hip)
-// and move 13 (D) and 11 vectors a step for 7 stages.
+// and move 15 (D) and 9 vectors a step for 7 stages, 57 and 32 for 13.
 static int least_traffic_form(const rkx_ode &p, const rkx_method &m)
 {
-  // BRUSS2D, stages in groups: up to two groups D and E cost the same (N = 1000,
-  // DOPRI54: 51 and 50 us a step), beyond that D's partial sums cost more
-  // than E's stage derivatives (13 stages: 179 and 130 us)
+  // BRUSS2D, stages in groups: one group of up to 4 stages moves y and y_new
+  // alone and D's kernel is the simpler (RK4, N = 1000: 17.4 us a step, A
+  // 18.9); with more, D's partial sums cost more than E's stage derivatives
+  // (DOPRI54 N = 1000 51 and 50 us, N = 2000 246 and 162; 13 stages, N = 1000,
+  // 179 and 130)
   if (p.kind == RKX_BRUSS2D)
-    return m.s <= 8 ? RKX_IMPL_D : RKX_IMPL_E;
+    return m.s <= 4 ? RKX_IMPL_D : RKX_IMPL_E;
   const int s = m.s;
   int d = (s + 2) + 5;                                   // first and last stage
   for (int i = 1; i < s - 1; ++i)
@@ -760,8 +762,8 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
   const dev_ode dp = make_dev_ode(*p);
   const int s = m->s;
   int impl = o.impl;
-  // fused forms: the row sweep or the tile form for BRUSS2D, the segment kernel for the LV
-  // chain, the per-pair kernel for LV pairs; anything else (tables without a
+  // fused forms: the row sweep, the tile form or the one-workgroup form for
+  // BRUSS2D, the segment kernel for the LV chain, the per-pair kernel for LV pairs; anything else (tables without a
   // compiled pattern or stage count) runs the full-storage loop order with
   // the least traffic.  D, A, E and F run as asked on every problem.
   bool fused = impl == RKX_IMPL_PIPED || impl == RKX_IMPL_PIPEDLS;

@@ -8,7 +8,9 @@
 // y_new = y + dy into the other y buffer, so a rejected step needs no copy,
 // and folds the relative error max-norm into the step state; the last
 // workgroup runs the step control.  Full storage: y (2 buffers), w_1..w_{s-1},
-// dy, err.
+// dy, err.  Solves of LV problems and every full-storage batch instance run
+// these; a single BRUSS2D solve runs its stages in groups
+// (rkx_kernels_groups.hip).
 #include "rkx_device.hpp"
 
 #include <algorithm>

@@ -11,10 +11,10 @@
 //
 //   D         the w of the group's own later stages are read with a halo, and
 //             each w_l behind the group is read and written once, receiving
-//             the G terms: 13 vectors a DOPRI54 step in two kernels;
+//             the G terms: 15 vectors a DOPRI54 step in two kernels;
 //   A, E, F   y and v_0 .. v_{i0-1} are read with a halo and gathered into the
 //             group's w, and the group's v are written; the step's last kernel
-//             also gathers dy and err, and writes y_new: 11 vectors.
+//             also gathers dy and err, and writes y_new: 9 vectors.
 //
 // Every sum receives its terms in the reference's order, in A without those
 // of zero coefficients (of the table), in D, E and F with them, so each equals

@@ -33,10 +33,11 @@ bool tile_supported(int pattern) { return pattern >= 1 && pattern <= 6; }
 // one to a compute unit: a step then takes the time of one tile, which grows
 // with its rows, and a second round would double it.  Grids beyond the
 // tallest tile's one round belong to the row sweep, whose bands waste less
-// on halos.  Measured, us per step, tile against sweep: DOPRI54 N=32 9.7 /
-// 11.0, N=128 9.3 / 11.5, N=301 11.9 / 14.6, N=512 14.9 / 17.6 (tallest tile
-// in two rounds at N=717: 30.6 / 21.0); VERNER65 N=128 11.1 / 17.9, N=301
-// 13.6 / 22.4; RKF23 N=128 6.9 / 7.6, N=512 10.1 / 11.4.
+// on halos.  Measured, us per step, tile against the best of 28 sweep shapes:
+// DOPRI54 N=48 8.6 / 10.1, N=128 8.3 / 10.2, N=301 10.1 / 11.0, N=512 12.2 /
+// 15.6, N=650 15.4 / 17.0 (tallest tile in two rounds at N=717: 30.6 / 21.0);
+// VERNER65 N=128 9.2 / 16.9, N=301 11.2 / 17.0, N=512 17.1 / 21.0; RKF23
+// N=128 5.9 / 6.4, N=512 7.5 / 8.6.
 int tile_default_shape(const dev_ode &p, const rkx_method &m)
 {
   if (!tile_supported(sweep_pattern(m)))
