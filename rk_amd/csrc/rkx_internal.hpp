@@ -375,7 +375,8 @@ struct stage_group {
 constexpr int kGroupBlocks = 512;   // two workgroups on a compute unit
 // all of a step's kernels, form RKX_IMPL_D, A, E or F; a: without i0 and the
 // tile counts
-hipError_t launch_groups(int form, stage_group a, const gather_masks &nz, hipStream_t stream);
+hipError_t launch_groups(int form, const stage_group &a, const gather_masks &nz,
+                         hipStream_t stream);
 
 // One LV chain instance as the fused chain kernel sees it (device memory).
 struct chain_inst {

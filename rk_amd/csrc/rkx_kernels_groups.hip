@@ -24,7 +24,7 @@
 // D 555 -> 179, A 404 -> 132, E 451 -> 130, F 379 -> 130.
 //
 // The tile is the one of rkx_tile_kernel.hpp: 64 columns (lane = column) x
-// 8 waves of C rows, u and v in one lane, horizontal neighbours by DPP,
+// 8 waves of C = 2 or 4 rows, u and v in one lane, horizontal neighbours by DPP,
 // vertical ones across waves through LDS; it yields 64 - 2G columns and
 // 8C - 2(G-1) rows.  Every kernel of the step starts with the control of the
 // attempt before it; the last one folds the error.
@@ -35,7 +35,11 @@
 namespace rkx {
 namespace {
 
-constexpr int kGroupRows = 4;                    // rows per wave
+// rows per wave: the fewer that still let all tiles of a kernel run at once
+// (halo rows are cheaper then than a second row's time in every wave), else 4.
+// us per step, 2 / 4 rows: DOPRI54 D N = 200 15.4 / 18.4, N = 500 25.7 / 27.6,
+// N = 700 36.9 / 34.0, N = 1000 59.5 / 51.9.
+constexpr int kGroupRows[] = {2, 4};
 
 using cell2 = double __attribute__((ext_vector_type(2)));
 using gcell = __attribute__((address_space(1))) cell2;
@@ -50,9 +54,9 @@ struct group_lds {
 };
 
 // One tile: where it lies, and the group's stages over it.
-template <int G, bool SMALL>
+template <int G, int C, bool SMALL>
 struct group_tile {
-  static constexpr int C = kGroupRows, W = kTileWaves, H = W * C;
+  static constexpr int W = kTileWaves, H = W * C;
   int N, lane, wv;
   int c0, c1, r0, r1;          // columns and rows of y_new
   int col, row;                // the lane's column, the wave's first row
@@ -158,10 +162,10 @@ struct group_tile {
   }
 };
 
-template <int G, bool FIRST, bool LAST, bool SMALL>
+template <int G, int C, bool FIRST, bool LAST, bool SMALL>
 __global__ __launch_bounds__(64 * kTileWaves) void k_d_group(stage_group a)
 {
-  constexpr int C = kGroupRows, W = kTileWaves;
+  constexpr int W = kTileWaves;
   __shared__ group_lds x;
   __shared__ double cl[G][RKX_MAX_STAGES + 2];   // h A[l][i0+g] (l < s), h b, h e
 
@@ -189,7 +193,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void k_d_group(stage_group a)
   // coefficients and the control are formed once per workgroup
   for (int t = blockIdx.x; t < a.ntiles; t += gridDim.x) {
     __syncthreads();                             // cl; the tile before is done with edge
-    const group_tile<G, SMALL> T(a, t);
+    const group_tile<G, C, SMALL> T(a, t);
     // the group's first vector (y or w_i0) with the row on either side
     cell2 v0[C + 2];
     cell2 wg[G][C];                              // [g >= 1]: w_{i0+g}
@@ -292,10 +296,10 @@ __global__ __launch_bounds__(64 * kTileWaves) void k_d_group(stage_group a)
 }
 
 // A (SKIP), E and F.  nz: the masks of the table's non-zero entries.
-template <int G, bool FIRST, bool LAST, bool SMALL, bool SKIP>
+template <int G, int C, bool FIRST, bool LAST, bool SMALL, bool SKIP>
 __global__ __launch_bounds__(64 * kTileWaves) void k_g_group(stage_group a, gather_masks nz)
 {
-  constexpr int C = kGroupRows, W = kTileWaves;
+  constexpr int W = kTileWaves;
   __shared__ group_lds x;
   __shared__ double cl[G][RKX_MAX_STAGES];       // h A[i0+g][j]
   __shared__ double cb[RKX_MAX_STAGES], ce[RKX_MAX_STAGES];
@@ -328,7 +332,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void k_g_group(stage_group a, gath
   unsigned int zero = 0u;
   for (int t = blockIdx.x; t < a.ntiles; t += gridDim.x) {
     __syncthreads();
-    const group_tile<G, SMALL> T(a, t);
+    const group_tile<G, C, SMALL> T(a, t);
     cell2 yo[C], north, south;                   // y; w_i0 beyond the wave's rows
     cell2 wg[G][C], F[G][C], d[C], e[C];
     north = y[T.at(T.row - 1)];
@@ -434,66 +438,78 @@ __global__ __launch_bounds__(64 * kTileWaves) void k_g_group(stage_group a, gath
     step_fold<W>(x.head, qmax, zero, x.red);
 }
 
-template <int G, bool FIRST, bool LAST, bool SMALL>
+template <int G, int C, bool FIRST, bool LAST, bool SMALL>
 void launch_kernel(int form, const stage_group &a, const gather_masks &nz, int grid,
                    hipStream_t stream)
 {
   const dim3 g(grid), b(64 * kTileWaves);
   if (form == RKX_IMPL_D)
-    hipLaunchKernelGGL((k_d_group<G, FIRST, LAST, SMALL>), g, b, 0, stream, a);
+    hipLaunchKernelGGL((k_d_group<G, C, FIRST, LAST, SMALL>), g, b, 0, stream, a);
   else if (form == RKX_IMPL_A)
-    hipLaunchKernelGGL((k_g_group<G, FIRST, LAST, SMALL, true>), g, b, 0, stream, a, nz);
+    hipLaunchKernelGGL((k_g_group<G, C, FIRST, LAST, SMALL, true>), g, b, 0, stream, a, nz);
   else
-    hipLaunchKernelGGL((k_g_group<G, FIRST, LAST, SMALL, false>), g, b, 0, stream, a, nz);
+    hipLaunchKernelGGL((k_g_group<G, C, FIRST, LAST, SMALL, false>), g, b, 0, stream, a, nz);
 }
 
-template <int G, bool FIRST, bool LAST>
+template <int G, int C, bool FIRST, bool LAST>
 hipError_t launch_group(int form, const stage_group &a, const gather_masks &nz, int grid,
                         hipStream_t stream)
 {
-  if (a.N < 64 || a.N < kTileWaves * kGroupRows)
-    launch_kernel<G, FIRST, LAST, true>(form, a, nz, grid, stream);
+  if (a.N < 64 || a.N < kTileWaves * C)
+    launch_kernel<G, C, FIRST, LAST, true>(form, a, nz, grid, stream);
   else
-    launch_kernel<G, FIRST, LAST, false>(form, a, nz, grid, stream);
+    launch_kernel<G, C, FIRST, LAST, false>(form, a, nz, grid, stream);
   return hipGetLastError();
 }
 
-template <int G>
+template <int G, int C>
 hipError_t launch_group(bool first, bool last, int form, const stage_group &a,
                         const gather_masks &nz, int grid, hipStream_t stream)
 {
   if (first)
-    return last ? launch_group<G, true, true>(form, a, nz, grid, stream)
-                : launch_group<G, true, false>(form, a, nz, grid, stream);
-  return last ? launch_group<G, false, true>(form, a, nz, grid, stream)
-              : launch_group<G, false, false>(form, a, nz, grid, stream);
+    return last ? launch_group<G, C, true, true>(form, a, nz, grid, stream)
+                : launch_group<G, C, true, false>(form, a, nz, grid, stream);
+  return last ? launch_group<G, C, false, true>(form, a, nz, grid, stream)
+              : launch_group<G, C, false, false>(form, a, nz, grid, stream);
 }
 
-}  // namespace
+// as few groups of up to four stages as there must be, of even sizes
+int stage_groups(int s) { return (s + 3) / 4; }
 
-hipError_t launch_groups(int form, stage_group a, const gather_masks &nz, hipStream_t stream)
+template <int C>
+hipError_t launch_shape(int form, stage_group a, const gather_masks &nz, hipStream_t stream)
 {
-  // as few groups of up to four stages as there must be, of even sizes
-  const int groups = (a.s + 3) / 4;
-  const int H = kTileWaves * kGroupRows;
+  const int groups = stage_groups(a.s);
   for (int q = 0; q < groups; ++q) {
     const int i0 = q * a.s / groups, G = (q + 1) * a.s / groups - i0;
     a.i0 = i0;
     a.nstrips = tile_pieces(a.N, 64, G);
-    a.nbands = tile_pieces(a.N, H, G - 1);
+    a.nbands = tile_pieces(a.N, kTileWaves * C, G - 1);
     a.ntiles = a.nstrips * a.nbands;
+    const bool first = q == 0, last = q == groups - 1;
     const int grid = std::min(a.ntiles, kGroupBlocks);
     hipError_t e = hipErrorInvalidValue;
     switch (G) {
-    case 2: e = launch_group<2>(q == 0, q == groups - 1, form, a, nz, grid, stream); break;
-    case 3: e = launch_group<3>(q == 0, q == groups - 1, form, a, nz, grid, stream); break;
-    case 4: e = launch_group<4>(q == 0, q == groups - 1, form, a, nz, grid, stream); break;
+    case 2: e = launch_group<2, C>(first, last, form, a, nz, grid, stream); break;
+    case 3: e = launch_group<3, C>(first, last, form, a, nz, grid, stream); break;
+    case 4: e = launch_group<4, C>(first, last, form, a, nz, grid, stream); break;
     default: break;
     }
     if (e != hipSuccess)
       return e;
   }
   return hipSuccess;
+}
+
+}  // namespace
+
+hipError_t launch_groups(int form, const stage_group &a, const gather_masks &nz, hipStream_t stream)
+{
+  // the largest group's tiles are the most
+  const int G = (a.s + stage_groups(a.s) - 1) / stage_groups(a.s);
+  const int tiles = tile_pieces(a.N, 64, G) * tile_pieces(a.N, kTileWaves * kGroupRows[0], G - 1);
+  return tiles <= kGroupBlocks ? launch_shape<kGroupRows[0]>(form, a, nz, stream)
+                               : launch_shape<kGroupRows[1]>(form, a, nz, stream);
 }
 
 }  // namespace rkx

@@ -1,8 +1,8 @@
 """The A, E and F forms of BRUSS2D in groups of stages
 (rkx_kernels_groups.hip) bitwise against kernels that share none of that code:
 the row sweep for compiled tables, the CPU oracle's seq D for others (tables
-with zeros, whose terms A leaves out).  Sizes at the edges of the 64-column,
-32-row tiles of every group size."""
+with zeros, whose terms A leaves out).  Sizes at the edges of the tiles of
+every group size."""
 import numpy as np
 import pytest
 import torch  # before the library: both load the HIP runtime
@@ -41,3 +41,14 @@ def test_custom_tables_equal_oracle(orc, s):
             st, tr, y = run(n, m, 1e-4, impl, ctrl="host")
             assert st[:2] == (so["acc"], so["rej"]), (n, impl)
             assert np.array_equal(tr, tro) and np.array_equal(y, yo), (n, impl)
+
+
+@pytest.mark.parametrize("meth", ["HEUN2", "RK4", "DOPRI54", "DOPRI87"])
+def test_taller_tiles_equal_row_sweep(meth):
+    """Grids whose two-row tiles do not all run at once: four rows to a wave."""
+    import rk_amd
+    tol = 1e-6 if rk_amd.method(meth).has_emb else 0.0
+    for n in (530, 641, 713):
+        ref = run(n, meth, tol, "PipeDls", tile_rows=32)
+        for impl in ("D", "A", "E"):
+            assert same(run(n, meth, tol, impl), ref), (n, impl)
