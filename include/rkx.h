@@ -134,8 +134,9 @@ typedef struct rkx_opts {
   int tile_rows;         /* BRUSS2D with either of these two set runs the row sweep;
                             with both 0, small grids run in 64-column tiles or in one
                             workgroup.  Band height in grid rows (0: chosen; VERNER65
-                            rounds it up so that a band's row iterations after its
-                            first 2(s-1) fill whole trips of its ring) */
+                            and DOPRI87 round it up so that a band's row iterations
+                            after its first 2(s-1) fill whole trips of their ring,
+                            DOPRI87's last trip also up to its 4th) */
   int tile_waves;        /* sweep strip width in wavefronts per component, 1..4 (DOPRI87:
                             1..2, its kernel runs one wave per SIMD); 0: chosen.
                             With an even width, columns left over after the full

@@ -142,10 +142,7 @@ int sweep_band_rows(int pattern, int s, int rows)
 {
   if (!full_trips_of(pattern))
     return rows;
-  const int ns = s + 1;
-  const int pro = peeled_iters(true, s);
-  const int it = rows + 2 * (s - 1) - pro;      // iterations in the loop
-  return (it + ns - 1) / ns * ns - 2 * (s - 1) + pro;
+  return trip_iters(s, rows + 2 * (s - 1)) - 2 * (s - 1);
 }
 
 // Default tile: strips of 64*K columns (2K waves per workgroup) and the band
@@ -168,8 +165,7 @@ sweep_cfg sweep_default_cfg(const dev_ode &p, const rkx_method &m)
   const int s = m.s;
   const int N = p.N;
   const int pat = pattern_of(m);
-  const int trip = full_trips_of(pat) ? s + 1 : 0;
-  const int pro = peeled_iters(true, s);      // used with trip only
+  const bool trips = full_trips_of(pat);
   int cus = 0, dev = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
@@ -196,8 +192,8 @@ sweep_cfg sweep_default_cfg(const dev_ode &p, const rkx_method &m)
     for (int per_cu = 1; per_cu <= res; ++per_cu) {
       const int rows = band_rows_for(bands_for_slots(g, static_cast<long long>(cus) * per_cu));
       long long iters = rows + 2 * (s - 1);
-      if (trip > 0)
-        iters = pro + (iters - pro + trip - 1) / trip * trip;
+      if (trips)
+        iters = trip_iters(s, static_cast<int>(iters));
       const long long tiles = g.wgs((N + rows - 1) / rows);
       const long long rounds = (tiles + cus * per_cu - 1) / (cus * per_cu);
       const int there = static_cast<int>(std::min<long long>(per_cu, (tiles + cus - 1) / cus));
@@ -213,8 +209,8 @@ sweep_cfg sweep_default_cfg(const dev_ode &p, const rkx_method &m)
   auto round_time = [&](int rows) {
     const long long tiles = g.wgs((N + rows - 1) / rows);
     long long iters = rows + 2 * (s - 1);
-    if (trip > 0)
-      iters = pro + (iters - pro + trip - 1) / trip * trip;
+    if (trips)
+      iters = trip_iters(s, static_cast<int>(iters));
     return static_cast<double>((tiles + cus - 1) / cus) * static_cast<double>(iters + 4);
   };
   const long long tiles = g.wgs((N + best.rows - 1) / best.rows);

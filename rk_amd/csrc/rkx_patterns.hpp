@@ -83,10 +83,23 @@ constexpr int prefetch_rows(int s) { return (s - 2 < 2) ? s - 2 : 2; }
 
 // Row iterations at the start of a band that the fused kernel runs outside
 // its loop (the first 2(s-1), in which the stages whose rows no stored row
-// needs are left out); none for the 13-stage tables, whose peeled code would
-// be too long.  Tables whose kernel runs whole trips of the ring then fill
-// whole trips with the rest of the band.
-constexpr int peeled_iters(bool full_trips, int s) { return (full_trips && s > 9) ? 0 : 2 * (s - 1); }
+// needs are left out).  Tables whose kernel runs whole trips of the ring then
+// fill whole trips with the rest of the band.
+constexpr int peeled_iters(int s) { return 2 * (s - 1); }
+
+// Iterations after which a whole-trip kernel may also leave its last trip (0:
+// none).  13 stages: with trips of 14 iterations alone, bands have 14 k rows
+// and small grids 14-row bands of 38 iterations, where 4-row bands take 28
+// (DOPRI87, us per step, no exit / after 4 / after 7: N = 300 39.1 / 23.9 /
+// 28.1, N = 600 59.6 / 44.4 / 49.1, N = 1000 82.1 / 83.0 / 84.6).
+constexpr int trip_exit(int s) { return s > 9 ? 4 : 0; }
+// A whole-trip kernel's iterations for a band that needs n of them.
+constexpr int trip_iters(int s, int n)
+{
+  const int pro = peeled_iters(s), trip = s + 1, mid = trip_exit(s);
+  const int loop = n - pro, q = loop / trip, r = loop % trip;
+  return pro + q * trip + (r == 0 ? 0 : r <= mid ? mid : trip);
+}
 
 // compile-time loop: f(integral_constant<int, I>) for I = 0 .. N-1, so ring
 // slots and stage indices are constants and the register ring stays in VGPRs
