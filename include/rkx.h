@@ -136,7 +136,7 @@ typedef struct rkx_opts {
                             workgroup.  Band height in grid rows (0: chosen; VERNER65
                             and DOPRI87 round it up so that a band's row iterations
                             after its first 2(s-1) fill whole trips of their ring,
-                            DOPRI87's last trip also up to its 4th) */
+                            the last trip up to an exit) */
   int tile_waves;        /* sweep strip width in wavefronts per component, 1..4 (DOPRI87:
                             1..2, its kernel runs one wave per SIMD); 0: chosen.
                             With an even width, columns left over after the full

@@ -284,7 +284,7 @@ sweep_cfg sweep_default_cfg(const dev_ode &p, const rkx_method &m);
 // Band height a tile gets for `rows` requested rows: unchanged, or for tables
 // whose fused kernel runs whole trips of its s+1-row ring, rounded up so that
 // the band's rows + 2(s-1) row iterations, less the peeled ones
-// (peeled_iters), fill whole trips, the last up to its exit (trip_iters).
+// (peeled_iters), fill whole trips, the last up to an exit (trip_iters).
 int sweep_band_rows(int pattern, int s, int rows);
 // Whether every ghost row a band of an N-row grid loads lies within a single
 // reflection about row 0 / N-1 (the kernel's fast form); false for grids

@@ -83,22 +83,24 @@ constexpr int prefetch_rows(int s) { return (s - 2 < 2) ? s - 2 : 2; }
 
 // Row iterations at the start of a band that the fused kernel runs outside
 // its loop (the first 2(s-1), in which the stages whose rows no stored row
-// needs are left out).  Tables whose kernel runs whole trips of the ring then
-// fill whole trips with the rest of the band.
+// needs are left out).
 constexpr int peeled_iters(int s) { return 2 * (s - 1); }
 
-// Iterations after which a whole-trip kernel may also leave its last trip (0:
-// none).  13 stages: with trips of 14 iterations alone, bands have 14 k rows
-// and small grids 14-row bands of 38 iterations, where 4-row bands take 28
-// (DOPRI87, us per step, no exit / after 4 / after 7: N = 300 39.1 / 23.9 /
-// 28.1, N = 600 59.6 / 44.4 / 49.1, N = 1000 82.1 / 83.0 / 84.6).
-constexpr int trip_exit(int s) { return s > 9 ? 4 : 0; }
-// A whole-trip kernel's iterations for a band that needs n of them.
+// A whole-trip kernel may leave its last trip of s + 1 iterations also
+// trip_step(s), 2 trip_step(s), ... iterations before its end: whole trips
+// alone round a band up by up to s rows.  us per step, whole trips / exits:
+// VERNER65 N = 800 31.1 / 24.5, N = 1300 50.0 / 43.0, N = 2000 85.4 / 80.2,
+// N = 4001 294 / 286; DOPRI87 N = 300 39.1 / 25.1, N = 600 59.6 / 45.8, N = 1400
+// 142.4 / 136.5.  More exits cost the 13-stage kernel registers (every 3
+// iterations: N = 2000 282 against 266); VERNER65's need fewer with exits than
+// without (246 VGPRs for 256 and spills).
+constexpr int trip_step(int s) { return s > 9 ? 5 : 2; }
+// Its iterations for a band that needs n of them.
 constexpr int trip_iters(int s, int n)
 {
-  const int pro = peeled_iters(s), trip = s + 1, mid = trip_exit(s);
-  const int loop = n - pro, q = loop / trip, r = loop % trip;
-  return pro + q * trip + (r == 0 ? 0 : r <= mid ? mid : trip);
+  const int trip = s + 1, step = trip_step(s), loop = n - peeled_iters(s);
+  const int left = trip - 1 - (loop + trip - 1) % trip;   // of the last trip, not needed
+  return n + left - left / step * step;
 }
 
 // compile-time loop: f(integral_constant<int, I>) for I = 0 .. N-1, so ring
@@ -112,6 +114,17 @@ template <int N, class F>
 __device__ __forceinline__ void static_for(F &&f)
 {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+// the same until f returns false
+template <class F, int... Is>
+__device__ __forceinline__ void static_while_impl(F &&f, std::integer_sequence<int, Is...>)
+{
+  (void) (f(std::integral_constant<int, Is>{}) && ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_while(F &&f)
+{
+  static_while_impl(f, std::make_integer_sequence<int, N>{});
 }
 
 template <class P>

@@ -339,32 +339,35 @@ k_sweep(fused_launch<sweep_inst> a)
     constexpr int JALL = 2 * (s - 1);
     // the peeled iterations (every band runs more: R >= 1); with whole
     // trips the band height makes the rest fill whole trips, the last up to
-    // its exit.  13 stages: 156 of 832 stage rows of a 40-row band are left
-    // out (DOPRI87 N = 1000, with the exit: 100.6 -> 83.0 us per step, N = 300
-    // 43.9 -> 23.9).
+    // an exit.  13 stages: 156 of 832 stage rows of a 40-row band are left out
+    // (DOPRI87 N = 1000, with the exits: 100.6 -> 83.0 us per step, N = 300
+    // 43.9 -> 25.1).
     constexpr int PRO = peeled_iters(s);
     static_for<PRO>([&](auto jt) {
       constexpr int j = decltype(jt)::value;
       iter(it0 + j, std::integral_constant<int, j % NS>{}, jt);
     });
-    constexpr int EXIT = P::full_trips ? trip_exit(s) : 0;
     for (int rb = it0 + PRO; rb < it1; rb += NS) {
-      auto part = [&](auto ut, auto off) {
-        constexpr int U = decltype(ut)::value + decltype(off)::value;
-        const int rr = rb + U;
-        if constexpr (!P::full_trips) {
-          if (rr >= it1)
-            return;
-        }
-        iter(rr, std::integral_constant<int, (U + PRO) % NS>{},
+      auto at = [&](auto ut) {
+        constexpr int U = decltype(ut)::value;
+        iter(rb + U, std::integral_constant<int, (U + PRO) % NS>{},
              std::integral_constant<int, JALL>{});
       };
-      if constexpr (EXIT > 0) {
-        static_for<EXIT>([&](auto ut) { part(ut, int_c<0>{}); });
-        if (rb + EXIT >= it1)
-          break;
-      }
-      static_for<NS - EXIT>([&](auto ut) { part(ut, int_c<EXIT>{}); });
+      if constexpr (P::full_trips)
+        static_while<NS>([&](auto ut) {
+          constexpr int U = decltype(ut)::value;
+          if constexpr (U > 0 && (NS - U) % trip_step(s) == 0)
+            if (rb + U >= it1)
+              return false;
+          at(ut);
+          return true;
+        });
+      else
+        static_for<NS>([&](auto ut) {
+          if (rb + decltype(ut)::value >= it1)
+            return;
+          at(ut);
+        });
     }
   };
   if (__builtin_amdgcn_readfirstlane(var) == 0)
