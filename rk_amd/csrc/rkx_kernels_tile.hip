@@ -36,8 +36,8 @@ bool tile_supported(int pattern) { return pattern >= 1 && pattern <= 6; }
 // on halos.  Measured, us per step, tile against the best of 28 sweep shapes:
 // DOPRI54 N=48 8.6 / 10.1, N=128 8.3 / 10.2, N=301 10.1 / 11.0, N=512 12.2 /
 // 15.6, N=650 15.4 / 17.0 (tallest tile in two rounds at N=717: 30.6 / 21.0);
-// VERNER65 N=128 9.2 / 16.9, N=301 11.2 / 17.0, N=512 17.1 / 21.0; RKF23
-// N=128 5.9 / 6.4, N=512 7.5 / 8.6.
+// VERNER65 N=128 9.2 / 11.9, N=301 11.1 / 13.4, N=512 17.2 / 18.6, N=640 17.7
+// / 21.5; RKF23 N=128 5.9 / 6.4, N=512 7.5 / 8.6.
 int tile_default_shape(const dev_ode &p, const rkx_method &m)
 {
   if (!tile_supported(sweep_pattern(m)))
