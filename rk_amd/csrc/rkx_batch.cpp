@@ -424,8 +424,10 @@ int rkx_batch_create(rkx_batch **out, const rkx_batch_opts *o)
     rkx_batch_destroy(b);
     return rc;
   }
-  // slots without a fused instance have no ring (launch_step_flush skips them)
-  if (hipMemset(b->st_dev, 0, sizeof(state) * kBatchCap) != hipSuccess) {
+  // slots without a fused instance have no ring (launch_step_flush skips them);
+  // cleared on the batch's stream, which later writes of the states follow
+  if (hipMemsetAsync(b->st_dev, 0, sizeof(state) * kBatchCap, b->stream) != hipSuccess ||
+      hipStreamSynchronize(b->stream) != hipSuccess) {
     (void) hipGetLastError();
     rkx_batch_destroy(b);
     return fail(RKX_EDEVICE, "rkx_batch_create: clearing the states failed");

@@ -1,0 +1,51 @@
+"""The library's host side against a recording HIP runtime on the CPU
+(tests/hip_record.c): what it orders, keeps and frees.  Each test runs in a
+process of its own that loads the recorder ahead of librkx.so; no kernel runs."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+CHILD = """
+import ctypes, json, os, sys
+sys.path.insert(0, %(repo)r)
+rec = ctypes.CDLL(%(rec)r, mode=ctypes.RTLD_GLOBAL)
+rec.rec_live_bytes.restype = rec.rec_copy_block.restype = ctypes.c_size_t
+rec.rec_limit.argtypes = rec.rec_watch_copy.argtypes = [ctypes.c_size_t]
+import numpy as np
+import rk_amd
+out = {}
+%(body)s
+sys.stdout.write(json.dumps(out))
+"""
+
+
+@pytest.fixture(scope="module")
+def child(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("rec") / "libhiprecord.so")
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-I" + os.path.join(ROCM, "include"), "-o",
+                    so, os.path.join(HERE, "hip_record.c")], check=True)
+
+    def run(body):
+        src = CHILD % dict(repo=os.path.dirname(HERE), rec=so, body=body)
+        r = subprocess.run([sys.executable, "-c", src], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stderr[-2000:]
+        return json.loads(r.stdout)
+    return run
+
+
+def test_new_batch_clears_its_states_in_order(child):
+    """rkx_batch_create clears the states before rkx_batch_add writes one: the
+    clear must not be left running on a stream the writes do not wait for."""
+    out = child("""
+p = rk_amd.Bruss2D(24)
+with rk_amd.Batch() as b:
+    b.add(p, "DOPRI54", 0.0, 1.0, p.ode_start(), 1e-6, h0=1e-3)
+    out["unordered"] = rec.rec_unordered_writes()
+""")
+    assert out["unordered"] == 0
