@@ -134,8 +134,21 @@ double initial_h(double H, double tol, int limit, double h0)
 
 namespace {
 
-// All device memory of one solve, returned to the pool on scope exit, once
-// the solve's stream (if any) is done with it.
+struct graph_holder {
+  hipGraph_t g = nullptr;
+  hipGraphExec_t ge = nullptr;
+  ~graph_holder()
+  {
+    if (ge)
+      (void) hipGraphExecDestroy(ge);
+    if (g)
+      (void) hipGraphDestroy(g);
+  }
+};
+
+// What the launches of one solve use: its device memory, returned to the pool
+// on scope exit, its view and its step graph.  All of it outlives the work on
+// the solve's stream (if any), which goes on behind the loop's last attempt.
 struct solve_mem {
   struct held {
     void *p;
@@ -144,6 +157,7 @@ struct solve_mem {
   std::vector<held> blocks;
   hipStream_t stream = nullptr;
   host_view *view = nullptr;         // pinned
+  graph_holder steps;                // destroyed after the wait below
   ~solve_mem()
   {
     const bool ok = !stream || hipStreamSynchronize(stream) == hipSuccess;
@@ -198,18 +212,6 @@ struct solve_mem {
       views().push_back(w);
     else
       (void) hipHostFree(w);
-  }
-};
-
-struct graph_holder {
-  hipGraph_t g = nullptr;
-  hipGraphExec_t ge = nullptr;
-  ~graph_holder()
-  {
-    if (ge)
-      (void) hipGraphExecDestroy(ge);
-    if (g)
-      (void) hipGraphDestroy(g);
   }
 };
 
@@ -365,21 +367,22 @@ namespace {
 // stability and change little) or to the step limit, and the one launch whose
 // control ends the loop.  Long solves replay a graph of kChunk steps (1.7 us
 // of launch a step, 2.6 us launched one by one), captured while the first
-// steps run; it takes 85 us, so short solves do without.
+// steps run; it takes 85 us, so short solves do without.  The caller keeps the
+// graph (gh) until the stream is done: replays are still queued when the view
+// shows the end.
 //
 // many > 0: a launch makes up to that many attempts (and none pending: the
 // host sees the state after the last of them).  Two launches are kept in
 // flight then, the second covering the host's reaction to the first.
 template <class STEP>
 int run_steps(STEP &&enqueue, int many, const host_view &view, double te, int step_limit,
-              hipStream_t stream)
+              graph_holder &gh, hipStream_t stream)
 {
   constexpr int kChunk = 32;          // a multiple of kRing
   constexpr int kLow = 12;            // launches in flight below which more are made
   constexpr int kGroup = 8;           // made at a time without the graph
   constexpr int kGraphFrom = 160;     // expected steps worth a graph
   const volatile host_view &w = view;
-  graph_holder gh;
   long long launched = 0;
   auto capture = [&]() -> int {
     RKX_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
@@ -923,8 +926,9 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
   } else {
     auto enqueue_many = [&](int r) { return plan.launch_many(r, stream); };
     if (int rc = plan.many > 0
-                     ? run_steps(enqueue_many, plan.many, *mem.view, te, o.step_limit, stream)
-                     : run_steps(enqueue_step, 0, *mem.view, te, o.step_limit, stream))
+                     ? run_steps(enqueue_many, plan.many, *mem.view, te, o.step_limit, mem.steps,
+                                 stream)
+                     : run_steps(enqueue_step, 0, *mem.view, te, o.step_limit, mem.steps, stream))
       return rc;
     fin.t = mem.view->t;
     fin.h = mem.view->h;

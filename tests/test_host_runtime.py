@@ -49,3 +49,22 @@ with rk_amd.Batch() as b:
     out["unordered"] = rec.rec_unordered_writes()
 """)
     assert out["unordered"] == 0
+
+
+@pytest.mark.parametrize("ends", [200, 333, 400])
+def test_step_graph_outlives_its_replays(child, ends):
+    """A solve sees its end in pinned memory while the launches behind the last
+    attempt are still queued: the graph they come from must not be destroyed
+    before they have run."""
+    out = child("""
+import ctypes as C
+p = rk_amd.Bruss2D(64)
+y0 = p.ode_start()
+rec.rec_next_solve(%d)
+y, st, _ = rk_amd.solve_host(p, "DOPRI54", 0.0, 1.0, y0, 1e-6, h0=1e-3)
+out["steps"] = st.steps
+out["replays"] = rec.rec_graph_replays()
+out["early"] = rec.rec_graph_destroyed_early()
+""" % ends)
+    assert out["replays"] > 0 and out["steps"] == ends
+    assert out["early"] == 0
