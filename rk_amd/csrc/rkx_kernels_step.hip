@@ -1,6 +1,7 @@
 // The control of the fused kernels' last attempt, run on its own: after the
 // last launch of a chunk the attempt it made still awaits its control (every
-// fused kernel starts with the control of the attempt before it).
+// fused kernel starts with the control of the attempt before it).  Instances
+// that have ended are left alone.
 #include "rkx_device.hpp"
 
 namespace rkx {
@@ -11,7 +12,9 @@ constexpr int kFlushBlock = 64;
 __global__ __launch_bounds__(kFlushBlock) void k_step_flush(state *st, int n, int r)
 {
   const int i = blockIdx.x * kFlushBlock + threadIdx.x;
-  if (i >= n || !st[i].ring)
+  // an instance that has ended is launched no more, and its older ring slots
+  // keep attempts whose control has long run: nothing is pending
+  if (i >= n || !st[i].ring || st[i].v.done)
     return;
   step_ring &g = *st[i].ring;
   step_slot s = g.slot[r];
