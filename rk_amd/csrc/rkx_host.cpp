@@ -200,9 +200,10 @@ struct solve_mem {
         views().pop_back();
       }
     }
+    // coherent: the host reads it while kernels write it
     if (!view)
       RKX_HIP(hipHostMalloc(reinterpret_cast<void **>(&view), sizeof(host_view),
-                            hipHostMallocPortable));
+                            hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent));
     return RKX_OK;
   }
   static void give_view(host_view *w, bool ok)

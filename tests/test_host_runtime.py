@@ -68,3 +68,17 @@ out["early"] = rec.rec_graph_destroyed_early()
 """ % ends)
     assert out["replays"] > 0 and out["steps"] == ends
     assert out["early"] == 0
+
+
+def test_solve_view_is_asked_for_coherent(child):
+    """The host reads a solve's progress and end from pinned memory while kernels
+    run, so that memory has to be fine-grained by request, not by the
+    runtime's default."""
+    out = child("""
+rec.rec_next_solve(20)
+p = rk_amd.Bruss2D(64)
+rk_amd.solve_host(p, "DOPRI54", 0.0, 1.0, p.ode_start(), 1e-6, h0=1e-3)
+out["flags"] = rec.rec_pinned_flags()
+""")
+    portable, mapped, coherent = 0x1, 0x2, 0x40000000
+    assert out["flags"] == portable | mapped | coherent
