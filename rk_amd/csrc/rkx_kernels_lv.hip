@@ -138,47 +138,7 @@ k_lv_ensemble(int count, lv_method m, const double *__restrict__ prm,
       in_vector(ce[i]);
     }
   }
-  for (;;) {
-    const unsigned long long idle = __ballot(!active);
-    const int nidle = __popcll(idle);
-    if (nidle == 64 || (nidle >= kRefill && next < last)) {
-      if (have && !active) {
-        yout[2 * k] = y[0];
-        yout[2 * k + 1] = y[1];
-        acc_out[k] = st.acc;
-        rej_out[k] = st.rej;
-        have = false;
-      }
-      if (next >= last)
-        break;                                   // nidle == 64: everything is stored
-      if (next == window_end) {
-        if (last > 64)                           // more systems than lanes
-          rank_window(next);
-        window_end = min(next + kWindow, last);
-      }
-      const int mine = next + static_cast<int>(__popcll(idle & ((1ull << lane) - 1ull)));
-      if (!active && mine < window_end) {
-        k = system_of(last > 64 ? (next & ~(kWindow - 1)) + turn[wid][mine & (kWindow - 1)] : mine);
-        if (k < static_cast<size_t>(count)) {
-          p.c0 = prm[4 * k + 0];
-          p.d0 = prm[4 * k + 1];
-          p.d1 = prm[4 * k + 2];
-          p.c1 = prm[4 * k + 3];
-          y[0] = y0[2 * k];
-          y[1] = y0[2 * k + 1];
-          st.t = t0;
-          st.h = h0;
-          st.acc = st.rej = 0;
-          st.done = !(t0 < te);
-          have = true;
-          active = !st.done;
-        }
-      }
-      next = min(next + nidle, window_end);
-      continue;
-    }
-    if (!active)
-      continue;
+  auto attempt = [&]() {
     const double h = st.h;
     double w[S][2], dy[2], er[2];
     // first stage
@@ -224,7 +184,58 @@ k_lv_ensemble(int count, lv_method m, const double *__restrict__ prm,
     }
     ctrl_finish(st, need, need ? libm_pow(px, py, tab) : 0.0);
     active = !st.done && st.acc + st.rej < kLvMaxAttempts;
+  };
+  auto store = [&]() {
+    yout[2 * k] = y[0];
+    yout[2 * k + 1] = y[1];
+    acc_out[k] = st.acc;
+    rej_out[k] = st.rej;
+    have = false;
+  };
+  // While systems are left to hand out, each attempt starts with a count of
+  // the idle lanes; behind that, and for a wave of 64 systems from the start,
+  // every lane just runs to its end (the count and the branches around it made
+  // 64 systems' attempts 10 % longer with 4 stages and 18 % with 2: 3000
+  // attempts 2303 -> 2103 us with RK4, 2022 -> 1714 with HEUN2).
+  while (next < last) {
+    const unsigned long long idle = __ballot(!active);
+    const int nidle = __popcll(idle);
+    if (nidle < kRefill) {
+      if (active)
+        attempt();
+      continue;
+    }
+    if (have && !active)
+      store();
+    if (next == window_end) {
+      if (last > 64)                             // more systems than lanes
+        rank_window(next);
+      window_end = min(next + kWindow, last);
+    }
+    const int mine = next + static_cast<int>(__popcll(idle & ((1ull << lane) - 1ull)));
+    if (!active && mine < window_end) {
+      k = system_of(last > 64 ? (next & ~(kWindow - 1)) + turn[wid][mine & (kWindow - 1)] : mine);
+      if (k < static_cast<size_t>(count)) {
+        p.c0 = prm[4 * k + 0];
+        p.d0 = prm[4 * k + 1];
+        p.d1 = prm[4 * k + 2];
+        p.c1 = prm[4 * k + 3];
+        y[0] = y0[2 * k];
+        y[1] = y0[2 * k + 1];
+        st.t = t0;
+        st.h = h0;
+        st.acc = st.rej = 0;
+        st.done = !(t0 < te);
+        have = true;
+        active = !st.done;
+      }
+    }
+    next = min(next + nidle, window_end);
   }
+  while (active)
+    attempt();
+  if (have)
+    store();
 }
 
 }  // namespace
