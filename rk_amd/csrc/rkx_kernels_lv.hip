@@ -121,7 +121,8 @@ k_lv_ensemble(int count, lv_method m, const double *__restrict__ prm,
   st.step_limit = step_limit;
   // The table: 44 coefficients for 8 stages do not fit the scalar registers
   // beside the rest and came back from spills with two lane reads each; at
-  // one wave per SIMD vector registers are there for up to 8 stages.
+  // one wave per SIMD vector registers are there for up to 8 stages.  Those of
+  // 4 fit, and leave vector registers for five waves (94 instead of 122).
   double cA[S][S], cb[S], ce[S];
 #pragma unroll
   for (int i = 0; i < S; ++i) {
@@ -130,7 +131,7 @@ k_lv_ensemble(int count, lv_method m, const double *__restrict__ prm,
       cA[i][l] = m.A[i * RKX_MAX_STAGES + l];
     cb[i] = m.b[i];
     ce[i] = m.e[i];
-    if constexpr (S <= 8) {
+    if constexpr (S > 4 && S <= 8) {
 #pragma unroll
       for (int l = 0; l < i; ++l)
         in_vector(cA[i][l]);
@@ -267,14 +268,22 @@ extern "C" int rkx_lv_ensemble(int count, const double *params_dev, const double
   if (!s)
     if (int rc = default_stream(&s))
       return rc;
-  // At most one wave per SIMD; more systems than lanes take turns (see
-  // k_lv_ensemble).  One wave issues a step in 1.3 us (8 stages), two on a
-  // SIMD in about twice that: 262144 systems, VERNER65, tol 1e-8: 1.24 ms with
-  // one, 1.32 ms with two, 1.8 ms with one system per thread.
+  // With error control, at most one wave per SIMD; more systems than lanes take
+  // turns (see k_lv_ensemble).  One wave issues a step in 1.3 us (8 stages),
+  // two on a SIMD in about twice that: 262144 systems, VERNER65, tol 1e-8:
+  // 1.24 ms with one, 1.32 ms with two, 1.8 ms with one system per thread.
+  // Fixed steps, and tables without an error estimate, give every system the
+  // same number of attempts: no lane waits for another, and waves that hide
+  // each other's latency are worth more, so each lane gets one system.  262144
+  // systems, 1000 fixed steps, us, taking turns / a system a lane: HEUN2 1518 /
+  // 786, RK4 2075 / 1219, RKF23 1723 / 1103, DOPRI54 2759 / 2245, VERNER65
+  // 3084 / 2549.
   int cus = 0, dev = 0;
   RKX_HIP(hipGetDevice(&dev));
   RKX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  const int grid = std::min((count + kLvBlock - 1) / kLvBlock, cus);   // 4 waves a workgroup
+  const bool even = tol <= 0.0 || !m->has_emb;
+  const int all = (count + kLvBlock - 1) / kLvBlock;   // 4 waves a workgroup
+  const int grid = even ? all : std::min(all, cus);
 #define RKX_LV_CASE(S_)                                                                      \
   case S_:                                                                                   \
     hipLaunchKernelGGL(k_lv_ensemble<S_>, dim3(grid), dim3(kLvBlock), 0, s, count, lm,      \

@@ -41,6 +41,7 @@ static int nblocks;
 static size_t live, limit;
 static int graph_launches[kMaxGraphs], ngraphs, capturing = -1;
 static view_t *view;
+static unsigned last_grid;
 static int attempts, done_after;
 
 static struct {
@@ -85,6 +86,7 @@ int rec_graph_destroyed_early(void) { return rec.graph_destroyed_early; }
 int rec_unordered_writes(void) { return rec.unordered_writes; }
 int rec_graph_replays(void) { return rec.graph_replays; }
 unsigned rec_pinned_flags(void) { return rec.pinned_flags; }
+unsigned rec_last_grid(void) { return last_grid; }   /* workgroups of the last launch */
 size_t rec_live_bytes(void) { return live; }
 void rec_limit(size_t bytes) { limit = bytes; }
 /* the next solve ends after this many attempts */
@@ -236,7 +238,8 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *l, hipStream_t *s
 }
 hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **a, size_t l, hipStream_t s)
 {
-  (void) f, (void) g, (void) b, (void) a, (void) l;
+  (void) f, (void) b, (void) a, (void) l;
+  last_grid = g.x;
   if (capturing >= 0) {
     ++graph_launches[capturing];
     return hipSuccess;

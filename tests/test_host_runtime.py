@@ -82,3 +82,22 @@ out["flags"] = rec.rec_pinned_flags()
 """)
     portable, mapped, coherent = 0x1, 0x2, 0x40000000
     assert out["flags"] == portable | mapped | coherent
+
+
+@pytest.mark.parametrize("meth,tol,even", [("DOPRI54", 1e-6, False), ("DOPRI87", 1e-8, False),
+                                           ("DOPRI54", 0.0, True), ("DOPRI87", 0.0, True),
+                                           ("RK4", 0.0, True), ("HEUN2", 1e-6, True)])
+def test_even_ensembles_get_a_lane_per_system(child, meth, tol, even):
+    """Systems that take their turns on a bounded number of waves lose where all
+    of them take the same number of attempts."""
+    out = child("""
+import ctypes as C
+buf, m = (C.c_double * 16)(), rk_amd.method(%r)
+p = C.addressof(buf)
+out["grid"] = []
+for count in (1, 256, 257, 65536, 65537, 262144):
+    rc = rk_amd.lib().rkx_lv_ensemble(count, p, p, p, 0.0, 1.0, C.byref(m), %r, 1e-3, 10, p, p, None)
+    assert rc == 0
+    out["grid"].append(rec.rec_last_grid())
+""" % (meth, tol))
+    assert out["grid"] == [1, 1, 2, 256] + ([257, 1024] if even else [256, 256])
