@@ -73,6 +73,14 @@ k_lv_ensemble(int count, lv_method m, const double *__restrict__ prm,
   __shared__ unsigned char turn[kLvBlock / 64][kWindow];
   for (unsigned k = threadIdx.x; k < sizeof(pow_tables) / 8; k += kLvBlock)
     reinterpret_cast<double *>(&tab)[k] = reinterpret_cast<const double *>(&dev_pow_tables)[k];
+  constexpr bool kInLds = S > 8;
+  __shared__ alignas(16) double table[kInLds ? S : 1][(S + 3) / 2 * 2];
+  auto table_at = [&](int i, int l) -> double {
+    return l < S ? m.A[l * RKX_MAX_STAGES + i] : l == S ? m.b[i] : m.e[i];
+  };
+  if constexpr (kInLds)
+    for (int q = threadIdx.x; q < S * (S + 2); q += kLvBlock)
+      table[q / (S + 2)][q % (S + 2)] = table_at(q / (S + 2), q % (S + 2));
   __syncthreads();
 
   const int lane = threadIdx.x & 63;
@@ -119,27 +127,35 @@ k_lv_ensemble(int count, lv_method m, const double *__restrict__ prm,
   st.tol = tol;
   st.ord = m.ord;
   st.step_limit = step_limit;
-  // The table: 44 coefficients for 8 stages do not fit the scalar registers
-  // beside the rest and came back from spills with two lane reads each; at
-  // one wave per SIMD vector registers are there for up to 8 stages.  Those of
-  // 4 fit, and leave vector registers for five waves (94 instead of 122).
-  double cA[S][S], cb[S], ce[S];
+  // Coefficient l of stage i: A[l][i] for i < l < S, b[i] for l = S, e[i] for
+  // S + 1.  Those of 4 stages fit the scalar registers, and leave vector
+  // registers for five waves (94 instead of 122).  The 44 of 8 stages do not
+  // fit beside the rest and came back from spills with two lane reads each;
+  // at one wave per SIMD vector registers are there for them.  The 104 of 13
+  // stages are read from LDS for every attempt: left to the compiler, 265
+  // scalar registers were spilled (262144 systems, tol 1e-6: 506 us, 363 from
+  // LDS; 1000 fixed steps 9615, 5703).
+  double kept[kInLds ? 1 : S][S + 2];
+  if constexpr (!kInLds) {
 #pragma unroll
-  for (int i = 0; i < S; ++i) {
+    for (int i = 0; i < S; ++i) {
 #pragma unroll
-    for (int l = 0; l < i; ++l)
-      cA[i][l] = m.A[i * RKX_MAX_STAGES + l];
-    cb[i] = m.b[i];
-    ce[i] = m.e[i];
-    if constexpr (S > 4 && S <= 8) {
-#pragma unroll
-      for (int l = 0; l < i; ++l)
-        in_vector(cA[i][l]);
-      in_vector(cb[i]);
-      in_vector(ce[i]);
+      for (int l = i + 1; l < S + 2; ++l) {
+        kept[i][l] = table_at(i, l);
+        if constexpr (S > 4)
+          in_vector(kept[i][l]);
+      }
     }
   }
+  auto coef = [&](int l, int i) -> double {
+    if constexpr (kInLds)
+      return table[i][l];
+    else
+      return kept[i][l];
+  };
   auto attempt = [&]() {
+    if constexpr (kInLds)
+      __asm__ volatile("" ::: "memory");          // not kept in registers between attempts
     const double h = st.h;
     double w[S][2], dy[2], er[2];
     // first stage
@@ -147,25 +163,25 @@ k_lv_ensemble(int count, lv_method m, const double *__restrict__ prm,
     lv_pair(p, y[0], y[1], f0, f1);
 #pragma unroll
     for (int l = 1; l < S; ++l) {
-      const double a = h * cA[l][0];
+      const double a = h * coef(l, 0);
       w[l][0] = y[0] + a * f0;
       w[l][1] = y[1] + a * f1;
     }
-    dy[0] = (h * cb[0]) * f0;
-    dy[1] = (h * cb[0]) * f1;
-    er[0] = (h * ce[0]) * f0;
-    er[1] = (h * ce[0]) * f1;
+    dy[0] = (h * coef(S, 0)) * f0;
+    dy[1] = (h * coef(S, 0)) * f1;
+    er[0] = (h * coef(S + 1, 0)) * f0;
+    er[1] = (h * coef(S + 1, 0)) * f1;
     // intermediate and last stages
 #pragma unroll
     for (int i = 1; i < S; ++i) {
       lv_pair(p, w[i][0], w[i][1], f0, f1);
 #pragma unroll
       for (int l = i + 1; l < S; ++l) {
-        const double a = h * cA[l][i];
+        const double a = h * coef(l, i);
         w[l][0] += a * f0;
         w[l][1] += a * f1;
       }
-      const double hb = h * cb[i], he = h * ce[i];
+      const double hb = h * coef(S, i), he = h * coef(S + 1, i);
       dy[0] += hb * f0;
       dy[1] += hb * f1;
       er[0] += he * f0;
