@@ -126,7 +126,13 @@ k_lv_ensemble(int count, lv_method m, const double *__restrict__ prm,
   st.te = te;
   st.tol = tol;
   st.ord = m.ord;
+  // Few stages: the bound on attempts is part of the step limit, one test less
+  // in each (64 systems, 1000 fixed steps: RK4 451 -> 415 us, RKF23 387 -> 365;
+  // the schedule of 7 stages is the worse for it, 639 -> 704).
+  constexpr bool kOneLimit = S <= 4;
   st.step_limit = step_limit;
+  if constexpr (kOneLimit)
+    st.step_limit = step_limit > 0 ? min(step_limit, kLvMaxAttempts) : kLvMaxAttempts;
   // Coefficient l of stage i: A[l][i] for i < l < S, b[i] for l = S, e[i] for
   // S + 1.  Those of 4 stages fit the scalar registers, and leave vector
   // registers for five waves (94 instead of 122).  The 44 of 8 stages do not
@@ -200,7 +206,7 @@ k_lv_ensemble(int count, lv_method m, const double *__restrict__ prm,
       y[1] = yn[1];
     }
     ctrl_finish(st, need, need ? libm_pow(px, py, tab) : 0.0);
-    active = !st.done && st.acc + st.rej < kLvMaxAttempts;
+    active = !st.done && (kOneLimit || st.acc + st.rej < kLvMaxAttempts);
   };
   auto store = [&]() {
     yout[2 * k] = y[0];
