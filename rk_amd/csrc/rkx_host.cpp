@@ -150,13 +150,21 @@ struct graph_holder {
 // on scope exit, its view and its step graph.  All of it outlives the work on
 // the solve's stream (if any), which goes on behind the loop's last attempt.
 struct solve_mem {
+  // Pinned: the view, and what the host's step control passes to and fro.
+  struct pinned {
+    host_view view;
+    step_slot slot;
+    err_line err[kErrLines];
+    state st;
+    dev_coef coef;
+  };
   struct held {
     void *p;
     size_t bytes;
   };
   std::vector<held> blocks;
   hipStream_t stream = nullptr;
-  host_view *view = nullptr;         // pinned
+  pinned *host = nullptr;
   graph_holder steps;                // destroyed after the wait below
   ~solve_mem()
   {
@@ -167,8 +175,8 @@ struct solve_mem {
       else
         (void) hipFree(b.p);
     }
-    if (view)
-      give_view(view, ok);
+    if (host)
+      give_pinned(host, ok);
   }
   int alloc(void **out, size_t bytes)
   {
@@ -179,38 +187,38 @@ struct solve_mem {
     *out = b.p;
     return RKX_OK;
   }
-  // Views are a few words each; up to kViews of them are kept.
-  static constexpr size_t kViews = 64;
-  static std::mutex &view_mu()
+  // Up to kPinned of these (8 KB each) are kept.
+  static constexpr size_t kPinned = 64;
+  static std::mutex &pinned_mu()
   {
     static std::mutex *m = new std::mutex;
     return *m;
   }
-  static std::vector<host_view *> &views()
+  static std::vector<pinned *> &pinned_kept()
   {
-    static auto *v = new std::vector<host_view *>;
+    static auto *v = new std::vector<pinned *>;
     return *v;
   }
-  int take_view()
+  int take_pinned()
   {
     {
-      std::lock_guard<std::mutex> lk(view_mu());
-      if (!views().empty()) {
-        view = views().back();
-        views().pop_back();
+      std::lock_guard<std::mutex> lk(pinned_mu());
+      if (!pinned_kept().empty()) {
+        host = pinned_kept().back();
+        pinned_kept().pop_back();
       }
     }
-    // coherent: the host reads it while kernels write it
-    if (!view)
-      RKX_HIP(hipHostMalloc(reinterpret_cast<void **>(&view), sizeof(host_view),
+    // coherent: the host reads the view while kernels write it
+    if (!host)
+      RKX_HIP(hipHostMalloc(reinterpret_cast<void **>(&host), sizeof(pinned),
                             hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent));
     return RKX_OK;
   }
-  static void give_view(host_view *w, bool ok)
+  static void give_pinned(pinned *w, bool ok)
   {
-    std::lock_guard<std::mutex> lk(view_mu());
-    if (ok && views().size() < kViews)
-      views().push_back(w);
+    std::lock_guard<std::mutex> lk(pinned_mu());
+    if (ok && pinned_kept().size() < kPinned)
+      pinned_kept().push_back(w);
     else
       (void) hipHostFree(w);
   }
@@ -786,7 +794,7 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
 
   solve_mem mem;
   mem.stream = stream;
-  if (int rc = mem.take_view())
+  if (int rc = mem.take_pinned())
     return rc;
   double *ybuf[2] = {nullptr, nullptr};
   double *w = nullptr, *dy = nullptr, *err = nullptr, *trace_dev = nullptr;
@@ -796,7 +804,7 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
     return rc;
   state *st_dev = &ctl_dev->st;
   dev_coef *cf_dev = &ctl_dev->coef;
-  const step_refs ref{st_dev, &ctl_dev->ring, &ctl_dev->meth, mem.view};
+  const step_refs ref{st_dev, &ctl_dev->ring, &ctl_dev->meth, &mem.host->view};
   for (int b = 0; b < 2; ++b)
     if (int rc = mem.alloc(reinterpret_cast<void **>(&ybuf[b]), vec))
       return rc;
@@ -838,8 +846,8 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
   hs.s = s;
   hs.meth = &ctl_dev->meth;
   hs.coef = cf_dev;
-  hs.view = mem.view;
-  *mem.view = host_view{t0, hs.v.h, 0, 0, 0, 0};
+  hs.view = &mem.host->view;
+  mem.host->view = host_view{t0, hs.v.h, 0, 0, 0, 0};
   if (ringed) {
     hs.ring = ref.ring;
     hc.ring = make_ring(hs.v, trace_dev != nullptr);
@@ -872,8 +880,7 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
     return launch_gather_step(impl, dp, cf_dev, s, nz, st_dev, ybuf[0], ybuf[1], v, w, w1, stream);
   };
 
-  // the copies above read hc, whose ring the host control below reuses
-  RKX_HIP(hipStreamSynchronize(stream));
+  RKX_HIP(hipStreamSynchronize(stream));           // the copies above read hc
   const auto t_start = std::chrono::steady_clock::now();
   step_vars fin = hs.v;
 
@@ -881,23 +888,24 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
     // nothing to integrate
   } else if (o.ctrl == RKX_CTRL_HOST) {
     // One host round trip per step: the device computes the error norm, the
-    // host runs the reference's step control with the C library's pow.
+    // host runs the reference's step control with the C library's pow.  All
+    // of it goes through pinned memory, with one wait: the stream has done
+    // what the host sent by the time the next step's error has come back.
     step_vars &cur = fin;
+    solve_mem::pinned &pin = *mem.host;
+    pin.coef = hc.coef;
     dump_file dump;
     std::vector<double> ydump;
     for (int r = 0; !cur.done;) {
       RKX_HIP(enqueue_step(r));
       r = (r + 1) & (kRing - 1);
-      double step_err;
-      if (ringed) {
-        RKX_HIP(hipMemcpyAsync(&hc.ring, ref.ring, sizeof(hc.ring), hipMemcpyDeviceToHost, stream));
-        RKX_HIP(hipStreamSynchronize(stream));
-        step_err = ring_err(hc.ring, r);
-      } else {
-        RKX_HIP(hipMemcpyAsync(&hs, st_dev, sizeof(state), hipMemcpyDeviceToHost, stream));
-        RKX_HIP(hipStreamSynchronize(stream));
-        step_err = hs.err;
-      }
+      if (ringed)
+        RKX_HIP(hipMemcpyAsync(&pin.err, &ref.ring->err[r], sizeof(pin.err), hipMemcpyDeviceToHost,
+                               stream));
+      else
+        RKX_HIP(hipMemcpyAsync(&pin.st, st_dev, sizeof(state), hipMemcpyDeviceToHost, stream));
+      RKX_HIP(hipStreamSynchronize(stream));
+      const double step_err = ringed ? ring_err(pin.err) : pin.st.err;
       const int attempt = cur.acc + cur.rej;
       if (o.dump_path) {
         // the step's new y is in the other buffer until the decision flips cur
@@ -912,30 +920,29 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
         o.trace[3 * attempt + 2] = step_err;
       }
       host_finish(cur, step_err);
-      const step_slot next{cur, 0, 0};
       if (ringed) {
-        RKX_HIP(hipMemcpyAsync(&ref.ring->slot[r], &next, sizeof(next), hipMemcpyHostToDevice,
-                               stream));
+        pin.slot = step_slot{cur, 0, 0};
+        RKX_HIP(hipMemcpyAsync(&ref.ring->slot[r], &pin.slot, sizeof(step_slot),
+                               hipMemcpyHostToDevice, stream));
       } else {
-        premult(hc.meth, s, cur.h, hc.coef);
-        RKX_HIP(hipMemcpyAsync(cf_dev, &hc.coef, sizeof(hc.coef), hipMemcpyHostToDevice, stream));
-        hs.v = cur;
-        RKX_HIP(hipMemcpyAsync(st_dev, &hs, sizeof(state), hipMemcpyHostToDevice, stream));
+        premult(hc.meth, s, cur.h, pin.coef);
+        RKX_HIP(hipMemcpyAsync(cf_dev, &pin.coef, sizeof(dev_coef), hipMemcpyHostToDevice, stream));
+        pin.st.v = cur;
+        RKX_HIP(hipMemcpyAsync(st_dev, &pin.st, sizeof(state), hipMemcpyHostToDevice, stream));
       }
-      RKX_HIP(hipStreamSynchronize(stream));
     }
   } else {
     auto enqueue_many = [&](int r) { return plan.launch_many(r, stream); };
+    host_view &view = mem.host->view;
     if (int rc = plan.many > 0
-                     ? run_steps(enqueue_many, plan.many, *mem.view, te, o.step_limit, mem.steps,
-                                 stream)
-                     : run_steps(enqueue_step, 0, *mem.view, te, o.step_limit, mem.steps, stream))
+                     ? run_steps(enqueue_many, plan.many, view, te, o.step_limit, mem.steps, stream)
+                     : run_steps(enqueue_step, 0, view, te, o.step_limit, mem.steps, stream))
       return rc;
-    fin.t = mem.view->t;
-    fin.h = mem.view->h;
-    fin.acc = mem.view->acc;
-    fin.rej = mem.view->rej;
-    fin.cur = mem.view->cur;
+    fin.t = view.t;
+    fin.h = view.h;
+    fin.acc = view.acc;
+    fin.rej = view.rej;
+    fin.cur = view.cur;
   }
   const auto t_end = std::chrono::steady_clock::now();
   RKX_HIP(hipMemcpyAsync(y_dev, ybuf[fin.cur], vec, hipMemcpyDeviceToDevice, stream));

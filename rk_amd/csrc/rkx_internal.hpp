@@ -96,19 +96,20 @@ struct alignas(64) step_slot {
   int pending;                       // the attempt from v awaits its control
   int traced;                        // state::trace is set
 };
+struct alignas(128) err_line {
+  unsigned long long bits;           // atomic maximum: bits of a double >= 0
+};
 struct step_ring {
   step_slot slot[kRing];
-  struct alignas(128) {
-    unsigned long long bits;         // atomic maximum: bits of a double >= 0
-  } err[kRing][kErrLines];
+  err_line err[kRing][kErrLines];
 };
 // The error norm of a step: the maximum of its accumulators (doubles >= 0, so
 // their bits compare as the values do).
-__host__ __device__ inline double ring_err(const step_ring &g, int r)
+__host__ __device__ inline double ring_err(const err_line (&err)[kErrLines])
 {
   unsigned long long b = 0ull;
   for (int k = 0; k < kErrLines; ++k)
-    b = g.err[r][k].bits > b ? g.err[r][k].bits : b;
+    b = err[k].bits > b ? err[k].bits : b;
   return __builtin_bit_cast(double, b);
 }
 

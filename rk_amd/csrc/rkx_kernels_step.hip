@@ -19,7 +19,7 @@ __global__ __launch_bounds__(kFlushBlock) void k_step_flush(state *st, int n, in
   step_ring &g = *st[i].ring;
   step_slot s = g.slot[r];
   if (s.pending) {
-    const double err = ring_err(g, r);
+    const double err = ring_err(g.err[r]);
     trace_attempt(st + i, s.v, err);
     double px = 0.0, py = 0.0;
     const bool need = ctrl_decide(s.v, err, px, py);

@@ -149,9 +149,10 @@ int rkx_solve_noalloc(const rkx_ode *p, const rkx_method *m, double t0, double t
     for (int r = 0; !cur.done;) {
       RKX_HIP(step(r));
       r = (r + 1) & (kRing - 1);
-      RKX_HIP(hipMemcpyAsync(&hh.ring, ref.ring, sizeof(hh.ring), hipMemcpyDeviceToHost, stream));
+      RKX_HIP(hipMemcpyAsync(&hh.ring.err[r], &ref.ring->err[r], sizeof(hh.ring.err[r]),
+                             hipMemcpyDeviceToHost, stream));
       RKX_HIP(hipStreamSynchronize(stream));
-      host_finish(cur, ring_err(hh.ring, r));
+      host_finish(cur, ring_err(hh.ring.err[r]));
       const step_slot next{cur, 0, 0};
       RKX_HIP(hipMemcpyAsync(&ref.ring->slot[r], &next, sizeof(next), hipMemcpyHostToDevice,
                              stream));

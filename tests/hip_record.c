@@ -14,7 +14,7 @@
 #include <stdlib.h>
 #include <string.h>
 
-enum { kMaxOps = 1 << 16, kMaxBlocks = 4096, kMaxGraphs = 64 };
+enum { kMaxOps = 1 << 16, kMaxBlocks = 4096, kMaxPinned = 256, kMaxGraphs = 64 };
 
 typedef struct {
   hipStream_t stream;
@@ -29,7 +29,7 @@ typedef struct {
   size_t bytes;
 } block_t;
 
-typedef struct {          /* the library's host_view */
+typedef struct {          /* the library's host_view, in front of its pinned blocks */
   double t, h;
   int acc, rej, cur, done;
 } view_t;
@@ -38,6 +38,8 @@ static op_t ops[kMaxOps];
 static int nops;
 static block_t blocks[kMaxBlocks];
 static int nblocks;
+static block_t pinned[kMaxPinned];
+static int npinned;
 static size_t live, limit;
 static int graph_launches[kMaxGraphs], ngraphs, capturing = -1;
 static view_t *view;
@@ -48,6 +50,8 @@ static struct {
   int graph_destroyed_early;      /* executable graphs destroyed with launches queued */
   int unordered_writes;           /* writes to memory that another stream has still to write */
   int graph_replays;
+  int waits;                      /* for a stream */
+  int pageable_copies;            /* between device memory and memory that is not pinned */
   unsigned pinned_flags;          /* of the pinned block made last */
 } rec;
 
@@ -85,6 +89,8 @@ static hipError_t queue(hipStream_t s, int launch, int graph, void *dst, size_t 
 int rec_graph_destroyed_early(void) { return rec.graph_destroyed_early; }
 int rec_unordered_writes(void) { return rec.unordered_writes; }
 int rec_graph_replays(void) { return rec.graph_replays; }
+int rec_waits(void) { return rec.waits; }
+int rec_pageable_copies(void) { return rec.pageable_copies; }
 unsigned rec_pinned_flags(void) { return rec.pinned_flags; }
 unsigned rec_last_grid(void) { return last_grid; }   /* workgroups of the last launch */
 size_t rec_live_bytes(void) { return live; }
@@ -153,22 +159,39 @@ hipError_t hipHostMalloc(void **p, size_t bytes, unsigned flags)
 {
   *p = calloc(1, bytes);
   rec.pinned_flags = flags;
-  if (bytes == sizeof(view_t))
-    view = (view_t *) *p;
+  view = (view_t *) *p;
+  if (npinned < kMaxPinned)
+    pinned[npinned++] = (block_t){(char *) *p, bytes};
   return hipSuccess;
 }
 hipError_t hipHostFree(void *p)
 {
   if ((char *) view == (char *) p)
     view = NULL;
+  for (int i = 0; i < npinned; ++i)
+    if (pinned[i].p == p)
+      pinned[i--] = pinned[--npinned];
   free(p);
   return hipSuccess;
 }
 
+static int within(const block_t *b, int n, const void *p)
+{
+  for (int i = 0; i < n; ++i)
+    if (b[i].p <= (const char *) p && (const char *) p < b[i].p + b[i].bytes)
+      return 1;
+  return 0;
+}
+static int pageable(const void *p)
+{
+  return !within(blocks, nblocks, p) && !within(pinned, npinned, p);
+}
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t st)
 {
   (void) k;
   memmove(d, s, n);
+  if (pageable(d) || pageable(s))
+    ++rec.pageable_copies;
   for (int i = 0; n == last_copy_bytes && i < nblocks; ++i)
     if (blocks[i].p <= (char *) d && (char *) d < blocks[i].p + blocks[i].bytes)
       last_copy_block = blocks[i].bytes;
@@ -194,7 +217,12 @@ hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned f)
   *s = (hipStream_t) calloc(1, 64);
   return hipSuccess;
 }
-hipError_t hipStreamSynchronize(hipStream_t s) { drain(s, 0); return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s)
+{
+  ++rec.waits;
+  drain(s, 0);
+  return hipSuccess;
+}
 hipError_t hipDeviceSynchronize(void) { drain(NULL, 1); return hipSuccess; }
 hipError_t hipStreamQuery(hipStream_t s)
 {

@@ -101,3 +101,21 @@ for count in (1, 256, 257, 65536, 65537, 262144):
     out["grid"].append(rec.rec_last_grid())
 """ % (meth, tol))
     assert out["grid"] == [1, 1, 2, 256] + ([257, 1024] if even else [256, 256])
+
+
+@pytest.mark.parametrize("problem,impl", [("rk_amd.Bruss2D(64)", "PipeDls"),
+                                          ("rk_amd.Bruss2D(64)", "D"), ("rk_amd.LV(100)", "D")])
+def test_host_control_waits_once_an_attempt(child, problem, impl):
+    """The host's step control waits for each attempt's error and for nothing
+    else, and passes its values through pinned memory."""
+    out = child("""
+p = %s
+for limit in (20, 50):
+    w, c = rec.rec_waits(), rec.rec_pageable_copies()
+    y, st, _ = rk_amd.solve_host(p, "DOPRI54", 0.0, 1e9, p.ode_start(), 0.0, h0=1e-3,
+                                 step_limit=limit, impl=%r, ctrl="host")
+    assert st.steps == limit
+    out[limit] = (rec.rec_waits() - w, rec.rec_pageable_copies() - c)
+""" % (problem, impl))
+    assert out["50"][0] - out["20"][0] == 30
+    assert out["50"][1] == out["20"][1]
