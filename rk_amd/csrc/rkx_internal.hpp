@@ -206,8 +206,8 @@ int default_stream(hipStream_t *out);
 // the step control on the host: ctrl_decide/ctrl_finish with the C library's pow
 void host_finish(step_vars &v, double err);
 
-// Device blocks kept between solves (rkx_pool.cpp): take a block of at least
-// `bytes` (its size in *got), give it back once no stream uses it.
+// Device blocks kept between solves (rkx_pool.cpp): take a block of
+// `bytes` (to the page: *got), give it back once no stream uses it.
 int pool_take(void **out, size_t bytes, size_t *got);
 void pool_give(void *p, size_t bytes);
 

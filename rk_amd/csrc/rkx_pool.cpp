@@ -3,13 +3,15 @@
 // Mapping and unmapping device memory costs more than short solves do (two
 // vectors of 64 MiB: 0.43 ms of hipMalloc and hipFree a call, two of 256 MiB
 // 0.72 ms), so blocks that a solve or a batch instance is finished with wait
-// here for the next one.  At most kPoolBytes are kept, the least recently
+// here for the next one of their size (to the page: a block is never larger
+// than what its user counts).  At most kPoolBytes are kept, the least recently
 // returned ones are freed beyond that, and all of a device's are freed before
 // an allocation on it is allowed to fail.  A block is returned only when no
 // stream uses it any more (its owner has waited for its stream), so the next
 // owner may use it on any stream and from any thread.
 #include "rkx_internal.hpp"
 
+#include <algorithm>
 #include <list>
 #include <mutex>
 
@@ -46,16 +48,14 @@ int pool_take(void **out, size_t bytes, size_t *got)
   pool_t &P = pool();
   {
     std::lock_guard<std::mutex> lk(P.mu);
-    auto best = P.kept.end();
-    for (auto it = P.kept.begin(); it != P.kept.end(); ++it)
-      if (it->dev == dev && it->bytes >= bytes && it->bytes <= bytes + bytes / 4 &&
-          (best == P.kept.end() || it->bytes < best->bytes))
-        best = it;
-    if (best != P.kept.end()) {
-      *out = best->p;
-      *got = best->bytes;
-      P.bytes -= best->bytes;
-      P.kept.erase(best);
+    const auto it = std::find_if(P.kept.begin(), P.kept.end(), [&](const block &b) {
+      return b.dev == dev && b.bytes == bytes;
+    });
+    if (it != P.kept.end()) {
+      *out = it->p;
+      *got = bytes;
+      P.bytes -= bytes;
+      P.kept.erase(it);
       return RKX_OK;
     }
   }

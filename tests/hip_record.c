@@ -6,7 +6,7 @@
  * hipStreamQuery runs the oldest entry.  Streams do not wait for each other
  * (the library's are non-blocking).  Device memory is host memory; copies move
  * their bytes at once, so only their order is modelled.  A kernel launch does
- * nothing but count as one attempted step in the pinned block made last, as
+ * nothing but count as one attempted step in the solves' pinned block, as
  * the step control reports to a solve's host_view: launch k makes attempt k
  * and runs the control of attempt k - 1. */
 #define __HIP_PLATFORM_AMD__ 1
@@ -159,7 +159,8 @@ hipError_t hipHostMalloc(void **p, size_t bytes, unsigned flags)
 {
   *p = calloc(1, bytes);
   rec.pinned_flags = flags;
-  view = (view_t *) *p;
+  if (flags)                        /* a batch's snapshots ask for none */
+    view = (view_t *) *p;
   if (npinned < kMaxPinned)
     pinned[npinned++] = (block_t){(char *) *p, bytes};
   return hipSuccess;

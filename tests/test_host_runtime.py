@@ -119,3 +119,23 @@ for limit in (20, 50):
 """ % (problem, impl))
     assert out["50"][0] - out["20"][0] == 30
     assert out["50"][1] == out["20"][1]
+
+
+def test_kept_blocks_hold_what_is_asked(child):
+    """A vector gets no larger block than its own size (to the page): the byte
+    counts of a batch and its budget are those of the vectors."""
+    out = child("""
+big, small = rk_amd.Bruss2D(100), rk_amd.Bruss2D(92)
+rec.rec_next_solve(5)
+rk_amd.solve_host(big, "DOPRI54", 0.0, 1.0, big.ode_start(), 1e-6, h0=1e-3)
+rec.rec_watch_copy(8 * small.n)
+with rk_amd.Batch(hbm_budget=rk_amd.Batch.footprint(small, "DOPRI54")) as b:
+    b.add(small, "DOPRI54", 0.0, 1.0, small.ode_start(), 1e-6, h0=1e-3)
+    out["block"], out["asked"] = rec.rec_copy_block(), 8 * small.n
+live = rec.rec_live_bytes()
+rec.rec_next_solve(5)
+rk_amd.solve_host(big, "DOPRI54", 0.0, 1.0, big.ode_start(), 1e-6, h0=1e-3)
+out["again"] = rec.rec_live_bytes() - live
+""")
+    assert out["asked"] <= out["block"] < out["asked"] + 4096
+    assert out["again"] == 0
