@@ -281,6 +281,10 @@ int rkx_solve_noalloc(const rkx_ode *p, const rkx_method *m, double t0, double t
 /* ---- runtime -------------------------------------------------------------- */
 const char *rkx_last_error(void);
 int rkx_device_sync(void);
+/* Frees the device and pinned memory kept between calls: rkx_solve and the
+   batches keep up to 1 GiB of the device blocks they are finished with for the
+   next call that needs one of the same size. */
+int rkx_release_workspaces(void);
 /* Device bytes rkx_solve would hold for this problem/method/impl. */
 size_t rkx_solve_footprint(const rkx_ode *p, const rkx_method *m, int impl);
 

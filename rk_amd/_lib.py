@@ -95,6 +95,7 @@ SIGNATURES = [
     ("rkx_pow_host", C.c_int, [_dp, _dp, _dp, C.c_size_t]),
     ("rkx_last_error", C.c_char_p, []),
     ("rkx_device_sync", C.c_int, []),
+    ("rkx_release_workspaces", C.c_int, []),
     ("rkx_solve_footprint", C.c_size_t, [C.POINTER(Ode), C.POINTER(Method), C.c_int]),
 ]
 

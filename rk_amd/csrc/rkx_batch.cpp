@@ -241,10 +241,9 @@ int rebuild_tables(rkx_batch *b)
         (void) hipFree(g.dev);
       g.dev = nullptr;
       g.dev_cap = std::max<size_t>(g.tiles.size(), 2 * g.dev_cap);
-      if (hipMalloc(reinterpret_cast<void **>(&g.dev), g.dev_cap * sizeof(int2)) != hipSuccess) {
-        (void) hipGetLastError();
+      if (int rc = device_alloc(reinterpret_cast<void **>(&g.dev), g.dev_cap * sizeof(int2))) {
         g.dev_cap = 0;
-        return fail(RKX_ENOMEM, "rkx_batch: tile table allocation failed");
+        return rc;
       }
     }
     if (!g.tiles.empty())
@@ -397,12 +396,8 @@ int rkx_batch_create(rkx_batch **out, const rkx_batch_opts *o)
   if (!b->stream)
     rc = default_stream(&b->stream);
   auto dalloc = [&](void **p, size_t bytes) {
-    if (rc)
-      return;
-    if (hipMalloc(p, bytes) != hipSuccess) {
-      (void) hipGetLastError();
-      rc = fail(RKX_ENOMEM, "rkx_batch_create: device allocation failed");
-    }
+    if (!rc)
+      rc = device_alloc(p, bytes);
   };
   dalloc(reinterpret_cast<void **>(&b->st_dev), sizeof(state) * kBatchCap);
   dalloc(reinterpret_cast<void **>(&b->rg_dev), sizeof(step_ring) * kBatchCap);

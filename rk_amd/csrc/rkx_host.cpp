@@ -214,6 +214,16 @@ struct solve_mem {
                             hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent));
     return RKX_OK;
   }
+  static void release_pinned()
+  {
+    std::vector<pinned *> drop;
+    {
+      std::lock_guard<std::mutex> lk(pinned_mu());
+      drop.swap(pinned_kept());
+    }
+    for (pinned *w : drop)
+      (void) hipHostFree(w);
+  }
   static void give_pinned(pinned *w, bool ok)
   {
     std::lock_guard<std::mutex> lk(pinned_mu());
@@ -468,6 +478,13 @@ extern "C" {
 
 const char *rkx_last_error(void) { return g_last_error.c_str(); }
 
+int rkx_release_workspaces(void)
+{
+  pool_release();
+  solve_mem::release_pinned();
+  return RKX_OK;
+}
+
 int rkx_device_sync(void)
 {
   RKX_HIP(hipDeviceSynchronize());
@@ -646,11 +663,10 @@ int rkx_eval_rng_host(const rkx_ode *p, int i, int j, double t, const double *y,
       (void) hipFree(fd);
     yd = fd = nullptr;
     cap = 0;
-    if (hipMalloc(reinterpret_cast<void **>(&yd), win * sizeof(double)) != hipSuccess ||
-        hipMalloc(reinterpret_cast<void **>(&fd), win * sizeof(double)) != hipSuccess) {
-      (void) hipGetLastError();
-      return fail(RKX_ENOMEM, "rkx_eval_rng_host: device staging allocation failed");
-    }
+    if (int rc = device_alloc(reinterpret_cast<void **>(&yd), win * sizeof(double)))
+      return rc;
+    if (int rc = device_alloc(reinterpret_cast<void **>(&fd), win * sizeof(double)))
+      return rc;
     cap = win;
   }
   hipStream_t s = nullptr;

@@ -210,6 +210,9 @@ void host_finish(step_vars &v, double err);
 // `bytes` (to the page: *got), give it back once no stream uses it.
 int pool_take(void **out, size_t bytes, size_t *got);
 void pool_give(void *p, size_t bytes);
+void pool_release();
+// hipMalloc, again without the device's kept blocks if it fails
+int device_alloc(void **out, size_t bytes);
 
 // What a fused kernel is given of an instance's device-side step state.
 struct step_refs {

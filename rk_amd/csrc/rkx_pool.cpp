@@ -5,8 +5,9 @@
 // 0.72 ms), so blocks that a solve or a batch instance is finished with wait
 // here for the next one of their size (to the page: a block is never larger
 // than what its user counts).  At most kPoolBytes are kept, the least recently
-// returned ones are freed beyond that, and all of a device's are freed before
-// an allocation on it is allowed to fail.  A block is returned only when no
+// returned ones are freed beyond that, all of a device's are freed before one
+// of the library's allocations on it is allowed to fail, and all of them by
+// rkx_release_workspaces.  A block is returned only when no
 // stream uses it any more (its owner has waited for its stream), so the next
 // owner may use it on any stream and from any thread.
 #include "rkx_internal.hpp"
@@ -38,7 +39,44 @@ pool_t &pool()
   return *p;
 }
 
+// Frees the kept blocks of one device (dev < 0: of all).
+void free_kept(int dev)
+{
+  pool_t &P = pool();
+  std::list<block> drop;
+  {
+    std::lock_guard<std::mutex> lk(P.mu);
+    for (auto it = P.kept.begin(); it != P.kept.end();) {
+      const auto nx = std::next(it);
+      if (dev < 0 || it->dev == dev) {
+        P.bytes -= it->bytes;
+        drop.splice(drop.end(), P.kept, it);
+      }
+      it = nx;
+    }
+  }
+  for (const block &b : drop)
+    (void) hipFree(b.p);
+}
+
 }  // namespace
+
+void pool_release() { free_kept(-1); }
+
+int device_alloc(void **out, size_t bytes)
+{
+  if (hipMalloc(out, bytes) == hipSuccess)
+    return RKX_OK;
+  (void) hipGetLastError();
+  int dev = 0;
+  RKX_HIP(hipGetDevice(&dev));
+  free_kept(dev);
+  if (hipMalloc(out, bytes) == hipSuccess)
+    return RKX_OK;
+  (void) hipGetLastError();
+  *out = nullptr;
+  return fail(RKX_ENOMEM, "hipMalloc of " + std::to_string(bytes) + " bytes failed");
+}
 
 int pool_take(void **out, size_t bytes, size_t *got)
 {
@@ -59,29 +97,8 @@ int pool_take(void **out, size_t bytes, size_t *got)
       return RKX_OK;
     }
   }
-  void *p = nullptr;
-  if (hipMalloc(&p, bytes) != hipSuccess) {
-    (void) hipGetLastError();
-    std::list<block> drop;
-    {
-      std::lock_guard<std::mutex> lk(P.mu);
-      for (auto it = P.kept.begin(); it != P.kept.end();) {
-        auto nx = std::next(it);
-        if (it->dev == dev) {
-          P.bytes -= it->bytes;
-          drop.splice(drop.end(), P.kept, it);
-        }
-        it = nx;
-      }
-    }
-    for (const block &b : drop)
-      (void) hipFree(b.p);
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-      (void) hipGetLastError();
-      return fail(RKX_ENOMEM, "hipMalloc of " + std::to_string(bytes) + " bytes failed");
-    }
-  }
-  *out = p;
+  if (int rc = device_alloc(out, bytes))
+    return rc;
   *got = bytes;
   return RKX_OK;
 }

@@ -92,3 +92,9 @@ def solver(t0, te, y0, y, tol, problem, meth="DOPRI54", **kw):
     out, st, _ = solve_host(problem, meth, t0, te, y0, tol, **kw)
     y[...] = out
     return st
+
+
+def release_workspaces():
+    """Free the device and pinned memory the library keeps between calls (up to
+    1 GiB of workspaces), for other users of the device."""
+    check(lib().rkx_release_workspaces())

@@ -139,3 +139,39 @@ out["again"] = rec.rec_live_bytes() - live
 """)
     assert out["asked"] <= out["block"] < out["asked"] + 4096
     assert out["again"] == 0
+
+
+def test_kept_memory_is_given_back(child):
+    """What solves and batches keep goes back on request, and before any of the
+    library's own allocations fails for want of it."""
+    out = child("""
+p = rk_amd.Bruss2D(700)
+y0 = p.ode_start()
+empty = rec.rec_live_bytes()
+def solve():
+    rec.rec_next_solve(5)
+    rk_amd.solve_host(p, "DOPRI54", 0.0, 1.0, y0, 1e-6, h0=1e-3)
+solve()
+out["kept"] = rec.rec_live_bytes() - empty
+rec.rec_limit(rec.rec_live_bytes() + 1000)
+rk_amd.Batch().close()
+out["after a batch at the limit"] = rec.rec_live_bytes() - empty
+solve()
+rec.rec_limit(rec.rec_live_bytes() + 1000)
+import ctypes as C
+dp = C.POINTER(C.c_double)
+q = rk_amd.Bruss2D(280)
+big, g = q.ode_start(), np.empty(q.n)
+rc = rk_amd.lib().rkx_eval_rng_host(C.byref(q.desc), 0, q.n - 1, 0.0, big.ctypes.data_as(dp),
+                                    g.ctypes.data_as(dp))
+out["eval at the limit"] = rc
+rec.rec_limit(0)
+solve()
+staged = 2 * 8 * q.n
+rk_amd.release_workspaces()
+out["released"] = rec.rec_live_bytes() - empty - staged
+""")
+    assert out["kept"] >= 4 * 8 * 2 * 700 * 700
+    assert out["after a batch at the limit"] == 0
+    assert out["eval at the limit"] == 0
+    assert out["released"] == 0
