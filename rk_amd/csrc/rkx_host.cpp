@@ -384,29 +384,34 @@ namespace {
 // the host follows the solve through its view and launches no more than it
 // expects: the steps left at the current step size (most are limited by
 // stability and change little) or to the step limit, and the one launch whose
-// control ends the loop.  Long solves replay a graph of kChunk steps (1.7 us
+// control ends the loop.  Long solves replay a graph of 32 kernels or more (1.7 us
 // of launch a step, 2.6 us launched one by one), captured while the first
 // steps run; it takes 85 us, so short solves do without.  The caller keeps the
 // graph (gh) until the stream is done: replays are still queued when the view
 // shows the end.
 //
+// per_step: kernels of a step.  The graph then has fewer steps and pays after
+// fewer (chain of 100 cells, 13 stages, 27 kernels a step: 60 attempts 5907 us
+// launched one by one, 5049 from graphs).
+//
 // many > 0: a launch makes up to that many attempts (and none pending: the
 // host sees the state after the last of them).  Two launches are kept in
 // flight then, the second covering the host's reaction to the first.
 template <class STEP>
-int run_steps(STEP &&enqueue, int many, const host_view &view, double te, int step_limit,
-              graph_holder &gh, hipStream_t stream)
+int run_steps(STEP &&enqueue, int per_step, int many, const host_view &view, double te,
+              int step_limit, graph_holder &gh, hipStream_t stream)
 {
-  constexpr int kChunk = 32;          // a multiple of kRing
-  constexpr int kLow = 12;            // launches in flight below which more are made
-  constexpr int kGroup = 8;           // made at a time without the graph
-  constexpr int kGraphFrom = 160;     // expected steps worth a graph
+  constexpr int kLow = 12;            // steps in flight below which more are launched
+  constexpr int kGraphFrom = 160;     // expected kernels worth a graph
+  // steps of the graph, and launched at a time without it
+  const int chunk = std::max(32 / per_step / kRing, 1) * kRing;
+  const int group = std::max(8 / per_step, kRing / 2);
   const volatile host_view &w = view;
   long long launched = 0;
   auto capture = [&]() -> int {
     RKX_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
     hipError_t cap = hipSuccess;
-    for (int k = 0; k < kChunk && cap == hipSuccess; ++k)
+    for (int k = 0; k < chunk && cap == hipSuccess; ++k)
       cap = enqueue(k & (kRing - 1));
     const hipError_t end = hipStreamEndCapture(stream, &gh.g);
     if (cap != hipSuccess)
@@ -435,15 +440,15 @@ int run_steps(STEP &&enqueue, int many, const host_view &view, double te, int st
         continue;
       }
     } else if (want >= 1.0 && launched - made < kLow) {
-      const bool chunks = want >= kChunk && launched % kRing == 0;
+      const bool chunks = want >= chunk && launched % kRing == 0;
       const bool graph = chunks && gh.ge;
-      const bool make = chunks && !gh.ge && launched > 0 && left >= kGraphFrom;
+      const bool make = chunks && !gh.ge && launched > 0 && left * per_step >= kGraphFrom;
       if (graph) {
         RKX_HIP(hipGraphLaunch(gh.ge, stream));
-        launched += kChunk;
+        launched += chunk;
       } else {
         // twice as many before a graph is captured, to bridge that time
-        const double most = make ? 2 * kGroup : kGroup;
+        const double most = make ? 2 * group : group;
         const int n = static_cast<int>(std::fmin(want, most));
         for (int k = 0; k < n; ++k, ++launched)
           RKX_HIP(enqueue(static_cast<int>(launched & (kRing - 1))));
@@ -950,9 +955,11 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
   } else {
     auto enqueue_many = [&](int r) { return plan.launch_many(r, stream); };
     host_view &view = mem.host->view;
-    if (int rc = plan.many > 0
-                     ? run_steps(enqueue_many, plan.many, view, te, o.step_limit, mem.steps, stream)
-                     : run_steps(enqueue_step, 0, view, te, o.step_limit, mem.steps, stream))
+    const int kernels = ringed ? 1 : impl == RKX_IMPL_D ? s : impl == RKX_IMPL_F ? s + 1 : 2 * s;
+    if (int rc = plan.many > 0 ? run_steps(enqueue_many, 1, plan.many, view, te, o.step_limit,
+                                           mem.steps, stream)
+                               : run_steps(enqueue_step, kernels, 0, view, te, o.step_limit,
+                                           mem.steps, stream))
       return rc;
     fin.t = view.t;
     fin.h = view.h;

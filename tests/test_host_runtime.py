@@ -175,3 +175,19 @@ out["released"] = rec.rec_live_bytes() - empty - staged
     assert out["after a batch at the limit"] == 0
     assert out["eval at the limit"] == 0
     assert out["released"] == 0
+
+
+@pytest.mark.parametrize("problem,meth,steps,graph", [
+    ("rk_amd.LVChain(100)", "DOPRI87", 60, True), ("rk_amd.LVChain(100)", "DOPRI87", 5, False),
+    ("rk_amd.LVChain(100)", "DOPRI54", 60, False), ("rk_amd.LVChain(100)", "DOPRI54", 170, True)])
+def test_graph_pays_by_kernels(child, problem, meth, steps, graph):
+    """Whether a solve's steps come from a graph depends on the kernels it
+    expects to launch: a step of the full-storage forms is many."""
+    out = child("""
+p = %s
+rec.rec_next_solve(%d)
+y, st, _ = rk_amd.solve_host(p, %r, 0.0, 1e3, p.ode_start(), 1e-6, h0=1e-3, step_limit=%d)
+out["steps"], out["replays"] = st.steps, rec.rec_graph_replays()
+out["early"] = rec.rec_graph_destroyed_early()
+""" % (problem, steps, meth, steps))
+    assert out["early"] == 0 and (out["replays"] > 0) == graph
