@@ -278,7 +278,7 @@ int enqueue_batched_step(rkx_batch *b, int r)
                              b->stream));
     else if (I.storage == RKX_STORAGE_FULL)
       RKX_HIP(launch_d_step(I.dp, b->cf_dev + i, I.m.s, b->st_dev + i, I.y[0], I.y[1], I.w,
-                            I.dy, I.err, b->stream));
+                            I.dy, I.err, false, b->stream));
   }
   return RKX_OK;
 }

@@ -209,6 +209,17 @@ __device__ inline void show(host_view *w, const step_vars &v)
     __hip_atomic_store(&w->done, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// Full-storage forms: the first kernel of a step that reports (and of every
+// step past the end) shows what the control at the end of the step before
+// left.  A kernel ends when its stores to the host's memory have arrived: in
+// the control itself, on every step, they made 1000 LV pairs' steps 9 %
+// longer (HEUN2 in D's form).
+__device__ __forceinline__ void show_last(const state *st, bool report)
+{
+  if ((report || st->v.done) && st->view && blockIdx.x == 0 && threadIdx.x == 0)
+    show(st->view, st->v);
+}
+
 // The trace of an attempt made from v (one thread).
 __device__ inline void trace_attempt(state *st, const step_vars &v, double err)
 {
@@ -241,8 +252,6 @@ __device__ inline bool dev_control(state *st)
   double px = 0.0, py = 0.0;
   const bool need = ctrl_decide(st->v, st->err, px, py);
   ctrl_finish(st->v, need, need ? libm_pow(px, py, dev_pow_tables) : 0.0);
-  if (st->view)
-    show(st->view, st->v);
   return true;
 }
 

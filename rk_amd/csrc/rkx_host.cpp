@@ -390,6 +390,9 @@ namespace {
 // graph (gh) until the stream is done: replays are still queued when the view
 // shows the end.
 //
+// enqueue(r, report): the last of the steps launched together reports the state
+// it starts from, and in a graph every fourth does.
+//
 // per_step: kernels of a step.  The graph then has fewer steps and pays after
 // fewer (chain of 100 cells, 13 stages, 27 kernels a step: 60 attempts 5907 us
 // launched one by one, 5049 from graphs).
@@ -412,7 +415,7 @@ int run_steps(STEP &&enqueue, int per_step, int many, const host_view &view, dou
     RKX_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
     hipError_t cap = hipSuccess;
     for (int k = 0; k < chunk && cap == hipSuccess; ++k)
-      cap = enqueue(k & (kRing - 1));
+      cap = enqueue(k & (kRing - 1), (k & 3) == 3);
     const hipError_t end = hipStreamEndCapture(stream, &gh.g);
     if (cap != hipSuccess)
       return fail(RKX_EDEVICE, std::string("kernel launch during capture failed: ") +
@@ -434,7 +437,7 @@ int run_steps(STEP &&enqueue, int per_step, int many, const host_view &view, dou
     const double want = std::fmin(left + 1.0, 1e9) - static_cast<double>(launched - made);
     if (many > 0) {
       if (want >= 1.0 && launched - made <= many) {
-        RKX_HIP(enqueue(static_cast<int>(launched / many) & (kRing - 1)));
+        RKX_HIP(enqueue(static_cast<int>(launched / many) & (kRing - 1), true));
         launched += many;
         spin = 0;
         continue;
@@ -451,7 +454,7 @@ int run_steps(STEP &&enqueue, int per_step, int many, const host_view &view, dou
         const double most = make ? 2 * group : group;
         const int n = static_cast<int>(std::fmin(want, most));
         for (int k = 0; k < n; ++k, ++launched)
-          RKX_HIP(enqueue(static_cast<int>(launched & (kRing - 1))));
+          RKX_HIP(enqueue(static_cast<int>(launched & (kRing - 1)), k == n - 1));
         if (make)
           if (int rc = capture())
             return rc;
@@ -892,13 +895,16 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
                               gather ? v : w, dy, err, ref};
   }
 
-  // one attempted step; r: the ring slot a fused kernel reads
-  auto enqueue_step = [&](int r) -> hipError_t {
+  // one attempted step; r: the ring slot a fused kernel reads; report: the
+  // full-storage forms show the state the step starts from
+  auto enqueue_step = [&](int r, bool report) -> hipError_t {
     if (ringed)
       return plan.launch(r, stream);
     if (impl == RKX_IMPL_D)
-      return launch_d_step(dp, cf_dev, s, st_dev, ybuf[0], ybuf[1], w, dy, err, stream);
-    return launch_gather_step(impl, dp, cf_dev, s, nz, st_dev, ybuf[0], ybuf[1], v, w, w1, stream);
+      return launch_d_step(dp, cf_dev, s, st_dev, ybuf[0], ybuf[1], w, dy, err, report,
+                           stream);
+    return launch_gather_step(impl, dp, cf_dev, s, nz, st_dev, ybuf[0], ybuf[1], v, w, w1, report,
+                              stream);
   };
 
   RKX_HIP(hipStreamSynchronize(stream));           // the copies above read hc
@@ -918,7 +924,7 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
     dump_file dump;
     std::vector<double> ydump;
     for (int r = 0; !cur.done;) {
-      RKX_HIP(enqueue_step(r));
+      RKX_HIP(enqueue_step(r, false));
       r = (r + 1) & (kRing - 1);
       if (ringed)
         RKX_HIP(hipMemcpyAsync(&pin.err, &ref.ring->err[r], sizeof(pin.err), hipMemcpyDeviceToHost,
@@ -953,7 +959,7 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
       }
     }
   } else {
-    auto enqueue_many = [&](int r) { return plan.launch_many(r, stream); };
+    auto enqueue_many = [&](int r, bool) { return plan.launch_many(r, stream); };
     host_view &view = mem.host->view;
     const int kernels = ringed ? 1 : impl == RKX_IMPL_D ? s : impl == RKX_IMPL_F ? s + 1 : 2 * s;
     if (int rc = plan.many > 0 ? run_steps(enqueue_many, 1, plan.many, view, te, o.step_limit,

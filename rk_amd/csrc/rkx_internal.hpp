@@ -229,7 +229,7 @@ hipError_t launch_eval_rng(const dev_ode &p, int i, int j, const double *y, doub
                            hipStream_t s);
 hipError_t launch_d_step(const dev_ode &p, const dev_coef *cf, int s, state *st,
                          double *y0, double *y1, double *w, double *dy, double *err,
-                         hipStream_t stream);
+                         bool report, hipStream_t stream);
 // Stage-fused step of independent LV pairs (rkx_kernels_lvpairs.hip): every
 // table with 2, 3, 4, 7, 8 or 13 stages
 bool pairs_supported(const dev_ode &p, const rkx_method &m);
@@ -254,7 +254,7 @@ gather_masks make_gather_masks(const rkx_method &m);
 // w1 for F) one each
 hipError_t launch_gather_step(int form, const dev_ode &p, const dev_coef *cf, int s,
                               const gather_masks &nz, state *st, double *y0, double *y1,
-                              double *v, double *w0, double *w1, hipStream_t stream);
+                              double *v, double *w0, double *w1, bool report, hipStream_t stream);
 
 struct sweep_cfg {
   int waves;     // wavefronts per workgroup (strip width 64*waves lanes)

@@ -36,8 +36,9 @@ __global__ __launch_bounds__(kBlock) void k_d_first(dev_ode p, const dev_coef *_
                                                     int s, state *st, double *y0, double *y1,
                                                     double *__restrict__ w,
                                                     double *__restrict__ dy,
-                                                    double *__restrict__ err)
+                                                    double *__restrict__ err, bool report)
 {
+  show_last(st, report);
   if (st->v.done)
     return;
   const int cell = blockIdx.x * kBlock + threadIdx.x;
@@ -167,11 +168,12 @@ hipError_t launch_eval_rng(const dev_ode &p, int i, int j, const double *y, doub
 }
 
 hipError_t launch_d_step(const dev_ode &p, const dev_coef *m, int s, state *st, double *y0,
-                         double *y1, double *w, double *dy, double *err, hipStream_t stream)
+                         double *y1, double *w, double *dy, double *err, bool report,
+                         hipStream_t stream)
 {
   const int grid = (p.cells + kBlock - 1) / kBlock;
   hipLaunchKernelGGL(k_d_first, dim3(grid), dim3(kBlock), 0, stream, p, m, s, st, y0, y1, w,
-                     dy, err);
+                     dy, err, report);
   for (int i = 1; i < s - 1; ++i)
     hipLaunchKernelGGL(k_d_interm, dim3(grid), dim3(kBlock), 0, stream, p, m, s, i, st, w, dy,
                        err);

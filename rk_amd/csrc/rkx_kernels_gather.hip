@@ -41,8 +41,10 @@ __device__ __forceinline__ const double *gcur(const state *st, const double *y0,
 __global__ __launch_bounds__(kGBlock) void k_g_rhs(dev_ode p, int l, state *st,
                                                    const double *y0, const double *y1,
                                                    const double *__restrict__ w,
-                                                   double *__restrict__ v)
+                                                   double *__restrict__ v, bool report)
 {
+  if (l == 0)
+    show_last(st, report);
   if (st->v.done)
     return;
   const int cell = blockIdx.x * kGBlock + threadIdx.x;
@@ -92,8 +94,10 @@ __global__ __launch_bounds__(kGBlock) void k_g_rhs_gather(dev_ode p,
                                                           const double *y1,
                                                           const double *__restrict__ wl,
                                                           double *__restrict__ v,
-                                                          double *__restrict__ wn)
+                                                          double *__restrict__ wn, bool report)
 {
+  if (l == 0)
+    show_last(st, report);
   if (st->v.done)
     return;
   const int cell = blockIdx.x * kGBlock + threadIdx.x;
@@ -173,7 +177,8 @@ __global__ __launch_bounds__(kGOutThreads) void k_g_output(dev_ode p,
 
 hipError_t launch_gather_step(int form, const dev_ode &p, const dev_coef *m, int s,
                               const gather_masks &nz, state *st, double *y0, double *y1,
-                              double *v, double *w0, double *w1, hipStream_t stream)
+                              double *v, double *w0, double *w1, bool report,
+                              hipStream_t stream)
 {
   const int grid = (p.cells + kGBlock - 1) / kGBlock;
   const dim3 g(grid), b(kGBlock);
@@ -182,15 +187,16 @@ hipError_t launch_gather_step(int form, const dev_ode &p, const dev_coef *m, int
   if (form == RKX_IMPL_F) {
     double *wc = w0, *wn = w1;
     for (int l = 0; l < s - 1; ++l) {
-      hipLaunchKernelGGL(k_g_rhs_gather, g, b, 0, stream, p, m, l, st, y0, y1, wc, v, wn);
+      hipLaunchKernelGGL(k_g_rhs_gather, g, b, 0, stream, p, m, l, st, y0, y1, wc, v, wn,
+                         report);
       std::swap(wc, wn);
     }
-    hipLaunchKernelGGL(k_g_rhs, g, b, 0, stream, p, s - 1, st, y0, y1, wc, v);
+    hipLaunchKernelGGL(k_g_rhs, g, b, 0, stream, p, s - 1, st, y0, y1, wc, v, false);
     hipLaunchKernelGGL((k_g_output<false>), go, bo, 0, stream, p,
                        m, s, nz.b, nz.e, st, y0, y1, v);
   } else {
     const bool skip = (form == RKX_IMPL_A);
-    hipLaunchKernelGGL(k_g_rhs, g, b, 0, stream, p, 0, st, y0, y1, w0, v);
+    hipLaunchKernelGGL(k_g_rhs, g, b, 0, stream, p, 0, st, y0, y1, w0, v, report);
     for (int l = 1; l < s; ++l) {
       if (skip)
         hipLaunchKernelGGL((k_g_gather<true>), g, b, 0, stream, p, m, l, nz.rowA[l], st, y0, y1,
@@ -198,7 +204,7 @@ hipError_t launch_gather_step(int form, const dev_ode &p, const dev_coef *m, int
       else
         hipLaunchKernelGGL((k_g_gather<false>), g, b, 0, stream, p, m, l, nz.rowA[l], st, y0, y1,
                            v, w0);
-      hipLaunchKernelGGL(k_g_rhs, g, b, 0, stream, p, l, st, y0, y1, w0, v);
+      hipLaunchKernelGGL(k_g_rhs, g, b, 0, stream, p, l, st, y0, y1, w0, v, false);
     }
     if (skip)
       hipLaunchKernelGGL((k_g_output<true>), go, bo, 0, stream, p,
