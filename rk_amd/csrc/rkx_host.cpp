@@ -3,9 +3,10 @@
 // The step loop of the reference's solver() (src/impl/seq/D.c:58-78) runs on
 // the device: every step's kernels read t, h and the current-buffer index from
 // a device-resident state, and the step control (accept/reject and the next
-// h) runs on the device as well.  The host only enqueues chunks of
-// steps, captured once as a hipGraph, and polls the state between chunks;
-// kernels of a chunk that run past the end of the integration return at once.
+// h) runs on the device as well.  The host follows t, h and the counts in
+// pinned memory and keeps a few steps launched ahead, long solves from a graph
+// captured while the first steps run (run_steps); launches past the end of the
+// integration return at once.
 #include "rkx_internal.hpp"
 
 #include <algorithm>
@@ -799,9 +800,10 @@ int rkx_solve(const rkx_ode *p, const rkx_method *m, double t0, double te,
   const int s = m->s;
   int impl = o.impl;
   // fused forms: the row sweep, the tile form or the one-workgroup form for
-  // BRUSS2D, the segment kernel for the LV chain, the per-pair kernel for LV pairs; anything else (tables without a
-  // compiled pattern or stage count) runs the full-storage loop order with
-  // the least traffic.  D, A, E and F run as asked on every problem.
+  // BRUSS2D, the segment kernel for the LV chain, the per-pair kernel for LV
+  // pairs; anything else (tables without a compiled pattern or stage count)
+  // runs the full-storage loop order with the least traffic.  D, A, E and F
+  // run as asked on every problem.
   bool fused = impl == RKX_IMPL_PIPED || impl == RKX_IMPL_PIPEDLS;
   if (fused && !chain_supported(dp, *m) && !pairs_supported(dp, *m) &&
       !sweep_supported(dp, *m)) {

@@ -237,9 +237,9 @@ bool pairs_supported(const dev_ode &p, const rkx_method &m);
 hipError_t launch_lv_step(const dev_ode &p, int s, const step_refs &R, dev_coef *cf, double *y0,
                           double *y1, int r, hipStream_t stream);
 // Runs the pending step control of n states (those without a ring, and those
-// that have ended, are left alone), publishes it, and moves each ring on to slot 0 (rkx_kernels_step.hip):
-// after launches that ended on ring slot r, before the host reads the states
-// for good or starts again at slot 0.
+// that have ended, are left alone), publishes it, and moves each ring on to
+// slot 0 (rkx_kernels_step.hip): after launches that ended on ring slot r,
+// before the host reads the states for good or starts again at slot 0.
 hipError_t launch_step_flush(state *st, int n, int r, hipStream_t stream);
 
 // Gather forms A, E, F (src/impl/seq/A.c, E.c, F.c): non-zero patterns of the

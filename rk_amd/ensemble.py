@@ -1,8 +1,8 @@
 """Ensembles of independent Lotka-Volterra pairs (rkx_lv_ensemble).
 
 Each system has its own constants (x' = c0 x - d0 x y, y' = d1 x y - c1 y),
-start value, step size and accept/reject; one GPU thread integrates one
-system over the whole interval.
+start value, step size and accept/reject; a GPU lane integrates one system at a
+time over the whole interval, and takes another when it has finished.
 """
 import ctypes as C
 import math
