@@ -91,7 +91,8 @@ constexpr int peeled_iters(int s) { return 2 * (s - 1); }
 // alone round a band up by up to s rows.  us per step, whole trips / exits:
 // VERNER65 N = 800 31.1 / 24.5, N = 1300 50.0 / 43.0, N = 2000 85.4 / 80.2,
 // N = 4001 294 / 286; DOPRI87 N = 300 39.1 / 25.1, N = 600 59.6 / 45.8, N = 1400
-// 142.4 / 136.5.  More exits cost the 13-stage kernel registers (every 3
+// 142.4 / 136.5 (one exit, after 4 iterations: N = 300 23.9 and N = 600 44.4, but
+// N = 450 39.9 where the exits give 32.3).  More exits cost the 13-stage kernel registers (every 3
 // iterations: N = 2000 282 against 266); VERNER65's need fewer with exits than
 // without (246 VGPRs for 256 and spills).
 constexpr int trip_step(int s) { return s > 9 ? 5 : 2; }
