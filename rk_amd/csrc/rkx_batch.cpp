@@ -69,6 +69,7 @@ struct rkx_batch {
   dev_method *dm_dev = nullptr;
   sweep_inst *si_dev = nullptr;
   chain_inst *ci_dev = nullptr;
+  std::vector<std::pair<void *, size_t>> blocks;   // what the arrays above lie in
   state *st_pinned = nullptr;          // 2 x kBatchCap: snapshots of two chunks in flight
   hipEvent_t ev[2] = {nullptr, nullptr};
   hipGraph_t graph = nullptr;           // kPollSteps batched steps, captured once per table set
@@ -396,8 +397,11 @@ int rkx_batch_create(rkx_batch **out, const rkx_batch_opts *o)
   if (!b->stream)
     rc = default_stream(&b->stream);
   auto dalloc = [&](void **p, size_t bytes) {
+    size_t got = 0;
     if (!rc)
-      rc = device_alloc(p, bytes);
+      rc = pool_take(p, bytes, &got);
+    if (!rc)
+      b->blocks.push_back({*p, got});
   };
   dalloc(reinterpret_cast<void **>(&b->st_dev), sizeof(state) * kBatchCap);
   dalloc(reinterpret_cast<void **>(&b->rg_dev), sizeof(step_ring) * kBatchCap);
@@ -451,11 +455,8 @@ int rkx_batch_destroy(rkx_batch *b)
   for (auto &kv : b->groups)
     if (kv.second.dev)
       (void) hipFree(kv.second.dev);
-  for (void *p : {static_cast<void *>(b->st_dev), static_cast<void *>(b->rg_dev),
-                  static_cast<void *>(b->cf_dev), static_cast<void *>(b->dm_dev), static_cast<void *>(b->si_dev),
-                  static_cast<void *>(b->ci_dev)})
-    if (p)
-      (void) hipFree(p);
+  for (const auto &q : b->blocks)
+    pool_give(q.first, q.second);
   if (b->st_pinned)
     (void) hipHostFree(b->st_pinned);
   drop_graph(b);

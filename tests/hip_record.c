@@ -50,6 +50,7 @@ static struct {
   int graph_destroyed_early;      /* executable graphs destroyed with launches queued */
   int unordered_writes;           /* writes to memory that another stream has still to write */
   int graph_replays;
+  int allocations;                /* of device memory */
   int waits;                      /* for a stream */
   int pageable_copies;            /* between device memory and memory that is not pinned */
   unsigned pinned_flags;          /* of the pinned block made last */
@@ -89,6 +90,7 @@ static hipError_t queue(hipStream_t s, int launch, int graph, void *dst, size_t 
 int rec_graph_destroyed_early(void) { return rec.graph_destroyed_early; }
 int rec_unordered_writes(void) { return rec.unordered_writes; }
 int rec_graph_replays(void) { return rec.graph_replays; }
+int rec_allocations(void) { return rec.allocations; }
 int rec_waits(void) { return rec.waits; }
 int rec_pageable_copies(void) { return rec.pageable_copies; }
 unsigned rec_pinned_flags(void) { return rec.pinned_flags; }
@@ -141,6 +143,7 @@ hipError_t hipMalloc(void **p, size_t bytes)
   *p = calloc(1, bytes);
   blocks[nblocks++] = (block_t){(char *) *p, bytes};
   live += bytes;
+  ++rec.allocations;
   return hipSuccess;
 }
 hipError_t hipFree(void *p)
