@@ -2,14 +2,14 @@
 //
 // Mapping and unmapping device memory costs more than short solves do (two
 // vectors of 64 MiB: 0.43 ms of hipMalloc and hipFree a call, two of 256 MiB
-// 0.72 ms), so blocks that a solve or a batch instance is finished with wait
-// here for the next one of their size (to the page: a block is never larger
-// than what its user counts).  At most kPoolBytes are kept, the least recently
-// returned ones are freed beyond that, all of a device's are freed before one
-// of the library's allocations on it is allowed to fail, and all of them by
-// rkx_release_workspaces.  A block is returned only when no
-// stream uses it any more (its owner has waited for its stream), so the next
-// owner may use it on any stream and from any thread.
+// 0.72 ms), so blocks that a solve, a batch or one of its instances is finished
+// with wait here for the next one of their size (to the page: a block is never
+// larger than what its user counts).  At most kPoolBytes are kept, the least
+// recently returned ones are freed beyond that, all of a device's are freed
+// before one of the library's allocations on it is allowed to fail, and all of
+// them by rkx_release_workspaces.  A block is returned only when no stream uses
+// it any more (its owner has waited for its stream), so the next owner may use
+// it on any stream and from any thread.
 #include "rkx_internal.hpp"
 
 #include <algorithm>
